@@ -12,7 +12,8 @@
 #pragma once
 
 #include "device_common.h"
-#include "kernels_rows.h"  // stage_quant
+#include "kernels_rows.h"     // stage_quant
+#include "kernels_stacked.h"  // stage_quant_quads
 
 #define MOE_GROUP_MAX_E 1024
 #define MOE_GROUP_MAX_PAIRS 65535  // grouped rows are kept in 16 bits in k_group
@@ -28,12 +29,12 @@ static inline int group_item_cap(int T, int k, int E, int BT) {
 }
 
 // Workspace words for the grouped chain: counts[E] offsets[E+1] perm[P]
-// inv[P], then two item lists (4-word header, 4 words per item), each sized
-// for BT = 1 (group_list_words).
+// inv[P], then the item list (4-word header, 4 words per item), sized for
+// BT = 1 (group_list_words).
 static inline size_t group_list_words(int T, int k, int E) { return 4 + 4 * (size_t)group_item_cap(T, k, E, 1); }
 static inline size_t group_ws_words(int T, int k, int E) {
   const size_t P = (size_t)T * k;
-  return (size_t)E + (E + 1) + 2 * P + 2 * group_list_words(T, k, E);
+  return (size_t)E + (E + 1) + 2 * P + group_list_words(T, k, E);
 }
 
 // Lanes of the wave holding the same expert id as this lane (e >= 0, ids
@@ -48,6 +49,18 @@ __device__ __forceinline__ uint64_t same_id_lanes(int e, bool valid) {
   return m;
 }
 
+// Q8_0 of the x blocks [b0, b0 + most) below n in one of the two staged formats.
+__device__ __forceinline__ void group_quant(const float *__restrict__ x, int n, int b0, int most, uint32_t *xq, float *xd,
+                                            int quads, int tid, int nthr) {
+  const int nb = n - b0 < most ? n - b0 : most;
+  if (nb <= 0) return;
+  const float *xb = x + (size_t)b0 * MOE_QK;
+  if (quads)
+    stage_quant_quads(xb, nb, xq + (size_t)(b0 / 4) * MOE_SQ_DW, tid, nthr);
+  else
+    stage_quant(xb, nb, xq + (size_t)b0 * MOE_XSW, xd + b0, tid, nthr);
+}
+
 // Workgroup 0: the grouping.  Wave w owns the pairs [w*PW, (w+1)*PW) and
 // walks them 64 at a time in pair order; lanes with the same expert are
 // found by ballots over the id bits (rank = same-expert lanes below).
@@ -60,27 +73,24 @@ __device__ __forceinline__ uint64_t same_id_lanes(int e, bool valid) {
 //   wc[w][e] turned into wave w's first row of expert e;
 //   pass 2: row of a pair = wc[w][e] + rank, so rows ascend in pair order
 //   within each expert (ggml mul_mat_id's order).
-// items2 != NULL: a second item list of at most BT2 rows per item, the same
-// way (the gate/up and down kernels of a call may take different item sizes).
 // Workgroups 1..: Q8_0 of x (T rows of H, flat n_xblocks blocks) into the
-// staged format of the grouped kernels (xq, xd), MOE_GROUP_QBLOCKS blocks
-// each; none when xq is NULL.
+// staged format of the grouped kernels (the quad records of kernels_stacked.h
+// in xq when `quads`, else the digit format of kernels_rows.h in xq and xd),
+// MOE_GROUP_QBLOCKS blocks each; none when xq is NULL.
 __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids, int P, int E, int T, int shared,
                                                 int BT, int32_t *__restrict__ counts,
                                                 int32_t *__restrict__ offsets,
                                                 int32_t *__restrict__ perm, int32_t *__restrict__ inv,
                                                 int32_t *__restrict__ items, const float *__restrict__ x,
                                                 int n_xblocks, uint32_t *__restrict__ xq, float *__restrict__ xd,
-                                                int BT2, int32_t *__restrict__ items2) {
+                                                int quads) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (blockIdx.x > 0) {
-    const int b0 = (blockIdx.x - 1) * MOE_GROUP_QBLOCKS;
-    const int nb = n_xblocks - b0 < MOE_GROUP_QBLOCKS ? n_xblocks - b0 : MOE_GROUP_QBLOCKS;
-    if (nb > 0) stage_quant(x + (size_t)b0 * MOE_QK, nb, xq + (size_t)b0 * MOE_XSW, xd + b0, tid, 1024);
+    group_quant(x, n_xblocks, (blockIdx.x - 1) * MOE_GROUP_QBLOCKS, MOE_GROUP_QBLOCKS, xq, xd, quads, tid, 1024);
     return;
   }
   __shared__ uint16_t wc[16][MOE_GROUP_MAX_E];  // per-wave counts, then per-wave first rows (< 2^16)
-  __shared__ int32_t wsum[16], wsumi[16], wsumi2[16], tot[2];
+  __shared__ int32_t wsum[16], wsumi[16], tot;
   const int PW = ((P + 15) / 16 + 63) & ~63;    // pairs per wave, whole steps of 64
   const int p_lo = wave * PW, p_hi = p_lo + PW < P ? p_lo + PW : P;
   // up to MOE_GROUP_IT steps of 64 pairs per wave (P <= 16 * 64 * MOE_GROUP_IT):
@@ -126,30 +136,26 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids,
   if (tid < E)
     for (int w = 0; w < 16; w++) c += wc[w][tid];
   const int ni = items ? (c + BT - 1) / BT : 0;
-  const int ni2 = items2 ? (c + BT2 - 1) / BT2 : 0;
-  int v = c, vi = ni, vi2 = ni2;
+  int v = c, vi = ni;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
-    const int u = __shfl_up(v, off), ui = __shfl_up(vi, off), ui2 = __shfl_up(vi2, off);
+    const int u = __shfl_up(v, off), ui = __shfl_up(vi, off);
     if (lane >= off) {
       v += u;
       vi += ui;
-      vi2 += ui2;
     }
   }
   if (lane == 63) {
     wsum[wave] = v;
     wsumi[wave] = vi;
-    wsumi2[wave] = vi2;
   }
   __syncthreads();
-  int base = 0, basei = 0, basei2 = 0;
+  int base = 0, basei = 0;
   for (int w = 0; w < wave; w++) {
     base += wsum[w];
     basei += wsumi[w];
-    basei2 += wsumi2[w];
   }
-  const int excl = base + v - c, excli = basei + vi - ni, excli2 = basei2 + vi2 - ni2;
+  const int excl = base + v - c, excli = basei + vi - ni;
   if (tid < E) {
     counts[tid] = c;
     offsets[tid] = excl;
@@ -164,35 +170,20 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids,
       const int r = j * BT;
       rec[j] = make_int4(tid, excl + r, c - r < BT ? c - r : BT, ni > 1 ? MOE_ITEM_SPLIT : 0);
     }
-    int4 *rec2 = items2 ? reinterpret_cast<int4 *>(items2) + 1 + excli2 : nullptr;
-    for (int j = 0; j < ni2; j++) {
-      const int r = j * BT2;
-      rec2[j] = make_int4(tid, excl + r, c - r < BT2 ? c - r : BT2, ni2 > 1 ? MOE_ITEM_SPLIT : 0);
-    }
   }
   if (tid == 1023) {  // thread 1023's inclusive sums are the totals
     offsets[E] = base + v;
-    tot[0] = basei + vi;
-    tot[1] = basei2 + vi2;
+    tot = basei + vi;
   }
   __syncthreads();
   if (items) {
     const int ns = shared ? (T + BT - 1) / BT : 0;
     for (int j = tid; j < ns; j += 1024) {
       const int r = j * BT;
-      reinterpret_cast<int4 *>(items)[1 + tot[0] + j] =
+      reinterpret_cast<int4 *>(items)[1 + tot + j] =
           make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
     }
-    if (tid == 0) items[0] = tot[0] + ns;
-  }
-  if (items2) {
-    const int ns = shared ? (T + BT2 - 1) / BT2 : 0;
-    for (int j = tid; j < ns; j += 1024) {
-      const int r = j * BT2;
-      reinterpret_cast<int4 *>(items2)[1 + tot[1] + j] =
-          make_int4(E, P + r, T - r < BT2 ? T - r : BT2, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
-    }
-    if (tid == 0) items2[0] = tot[1] + ns;
+    if (tid == 0) items[0] = tot + ns;
   }
   // pass 2: row of a pair = wc[w][e] + rank (the lanes of one id read wc
   // before the last of them advances it)
@@ -277,7 +268,7 @@ template <int NPL>
 __device__ __forceinline__ void group_one_wave(const int32_t *__restrict__ ids, int P, int E, int T, int shared,
                                                int BT, int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
                                                int32_t *__restrict__ perm, int32_t *__restrict__ inv,
-                                               int32_t *__restrict__ items, int BT2, int32_t *__restrict__ items2) {
+                                               int32_t *__restrict__ items) {
   const int lane = threadIdx.x;
   int e[NPL];
   bool ok[NPL];
@@ -336,44 +327,40 @@ __device__ __forceinline__ void group_one_wave(const int32_t *__restrict__ ids, 
     for (int c = 0; c < NPL; c++) n += __popcll(__ballot(ok[c]));
     if (lane == 0) offsets[E] = n;
   }
-  for (int li = 0; li < 2; li++) {
-    int32_t *list = li ? items2 : items;
-    if (!list) continue;
-    const int bt = li ? BT2 : BT;
-    int n[NPL], base[NPL], tot = 0;
+  if (!items) return;
+  int n[NPL], base[NPL], tot = 0;
 #pragma unroll
-    for (int i = 0; i < NPL; i++) {
-      n[i] = ok[i] && before[i] == 0 ? (cnt[i] + bt - 1) / bt : 0;  // first pair of its expert
-      base[i] = 0;
-    }
-    bool big = false;  // an expert of more than one item on this lane
-#pragma unroll
-    for (int i = 0; i < NPL; i++) big |= n[i] > 1;
-    // counts of 0 or 1 everywhere (the common case): one bit; else every bit a count can have
-    const int nbits = __ballot(big) ? gf_bits((P + bt - 1) / bt) : 1;
-    for (int b = 0; b < nbits; b++) {
-#pragma unroll
-      for (int c = 0; c < NPL; c++) {
-        const uint64_t m = __ballot((n[c] >> b) & 1);
-        tot += __popcll(m) << b;
-#pragma unroll
-        for (int i = 0; i < NPL; i++) base[i] += __popcll(ltm[i][c] & m) << b;
-      }
-    }
-    int4 *rec = reinterpret_cast<int4 *>(list) + 1;
-#pragma unroll
-    for (int i = 0; i < NPL; i++)
-      for (int j = 0; j < n[i]; j++) {
-        const int r = j * bt;
-        rec[base[i] + j] = make_int4(e[i], less[i] + r, cnt[i] - r < bt ? cnt[i] - r : bt, n[i] > 1 ? MOE_ITEM_SPLIT : 0);
-      }
-    const int ns = shared ? (T + bt - 1) / bt : 0;  // the shared expert's items follow the routed ones
-    for (int j = lane; j < ns; j += 64) {
-      const int r = j * bt;
-      rec[tot + j] = make_int4(E, P + r, T - r < bt ? T - r : bt, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
-    }
-    if (lane == 0) list[0] = tot + ns;
+  for (int i = 0; i < NPL; i++) {
+    n[i] = ok[i] && before[i] == 0 ? (cnt[i] + BT - 1) / BT : 0;  // first pair of its expert
+    base[i] = 0;
   }
+  bool big = false;  // an expert of more than one item on this lane
+#pragma unroll
+  for (int i = 0; i < NPL; i++) big |= n[i] > 1;
+  // counts of 0 or 1 everywhere (the common case): one bit; else every bit a count can have
+  const int nbits = __ballot(big) ? gf_bits((P + BT - 1) / BT) : 1;
+  for (int b = 0; b < nbits; b++) {
+#pragma unroll
+    for (int c = 0; c < NPL; c++) {
+      const uint64_t m = __ballot((n[c] >> b) & 1);
+      tot += __popcll(m) << b;
+#pragma unroll
+      for (int i = 0; i < NPL; i++) base[i] += __popcll(ltm[i][c] & m) << b;
+    }
+  }
+  int4 *rec = reinterpret_cast<int4 *>(items) + 1;
+#pragma unroll
+  for (int i = 0; i < NPL; i++)
+    for (int j = 0; j < n[i]; j++) {
+      const int r = j * BT;
+      rec[base[i] + j] = make_int4(e[i], less[i] + r, cnt[i] - r < BT ? cnt[i] - r : BT, n[i] > 1 ? MOE_ITEM_SPLIT : 0);
+    }
+  const int ns = shared ? (T + BT - 1) / BT : 0;  // the shared expert's items follow the routed ones
+  for (int j = lane; j < ns; j += 64) {
+    const int r = j * BT;
+    rec[tot + j] = make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
+  }
+  if (lane == 0) items[0] = tot + ns;
 }
 
 __global__ __launch_bounds__(256) void k_group_few(const int32_t *__restrict__ ids, int P, int E, int T, int shared,
@@ -381,19 +368,16 @@ __global__ __launch_bounds__(256) void k_group_few(const int32_t *__restrict__ i
                                                    int32_t *__restrict__ offsets, int32_t *__restrict__ perm,
                                                    int32_t *__restrict__ inv, int32_t *__restrict__ items,
                                                    const float *__restrict__ x, int n_xblocks,
-                                                   uint32_t *__restrict__ xq, float *__restrict__ xd, int BT2,
-                                                   int32_t *__restrict__ items2) {
+                                                   uint32_t *__restrict__ xq, float *__restrict__ xd, int quads) {
   if (blockIdx.x > 0) {
-    const int b0 = (blockIdx.x - 1) * MOE_GF_QBLOCKS;
-    const int nb = n_xblocks - b0 < MOE_GF_QBLOCKS ? n_xblocks - b0 : MOE_GF_QBLOCKS;
-    if (nb > 0) stage_quant(x + (size_t)b0 * MOE_QK, nb, xq + (size_t)b0 * MOE_XSW, xd + b0, threadIdx.x, 256);
+    group_quant(x, n_xblocks, (blockIdx.x - 1) * MOE_GF_QBLOCKS, MOE_GF_QBLOCKS, xq, xd, quads, threadIdx.x, 256);
     return;
   }
   if (threadIdx.x >= 64) return;
   if (P <= 64)
-    group_one_wave<1>(ids, P, E, T, shared, BT, counts, offsets, perm, inv, items, BT2, items2);
+    group_one_wave<1>(ids, P, E, T, shared, BT, counts, offsets, perm, inv, items);
   else
-    group_one_wave<2>(ids, P, E, T, shared, BT, counts, offsets, perm, inv, items, BT2, items2);
+    group_one_wave<2>(ids, P, E, T, shared, BT, counts, offsets, perm, inv, items);
 }
 
 // ---------------------------------------------------------------------------

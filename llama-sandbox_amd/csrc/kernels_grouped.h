@@ -858,30 +858,6 @@ __device__ __forceinline__ void stage_octet_lds(const uint32_t *__restrict__ hs,
   }
 }
 
-// The same layout with a 16-byte zero slot after each step's 64 lanes
-// (stride 65), read by the operand half without data (bs32z).
-__host__ __device__ constexpr size_t octet_lds_bytes_z(int KB) {
-  return (size_t)(KB / 2) * 65 * 16 + (size_t)(KB / 2) * 16 * 4;
-}
-
-__device__ __forceinline__ void stage_octet_lds_z(const uint32_t *__restrict__ hs, const float *__restrict__ hd,
-                                                  int row0, int nt, int KB, u32x4_t *bl, float *dl, int tid,
-                                                  int nthr) {
-  const u32x4_t *src = reinterpret_cast<const u32x4_t *>(hs + (size_t)row0 * KB * MOE_XSW);
-  const int n16 = 8 * KB * 4;  // 16-byte chunks of 8 rows
-#pragma unroll 4
-  for (int c = tid; c < n16; c += nthr) {
-    const int t = c / (4 * KB), w = c - t * 4 * KB, b = w >> 2, sub = w & 3;
-    const int L = 32 * (sub & 1) + 4 * t + 2 * (sub >> 1) + (b & 1);
-    bl[(b >> 1) * 65 + L] = t < nt ? src[c] : u32x4_t{0u, 0u, 0u, 0u};
-  }
-  for (int c = tid; c < KB / 2; c += nthr) bl[c * 65 + 64] = u32x4_t{0u, 0u, 0u, 0u};
-  for (int c = tid; c < 8 * KB; c += nthr) {
-    const int t = c / KB, b = c - t * KB;
-    dl[((b >> 1) * 8 + t) * 2 + (b & 1)] = t < nt ? hd[(size_t)(row0 + t) * KB + b] : 0.0f;
-  }
-}
-
 // Ring of the LDS-B octet loop: weights of 4 quads (3 ahead), B of 2 quads
 // (1 ahead, from LDS) for NO octets, exponent dwords of NG groups.
 template <int NW, int NO, int NG>
@@ -982,576 +958,5 @@ void k_down_ol(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
 #pragma unroll
     for (int i = 0; i < 4; i++)
       *reinterpret_cast<float4 *>(dst + 8 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-  }
-}
-
-// B of one step as both 16-byte halves of each octet's MFMA operand, read
-// from LDS where each step's 64 lanes are followed by a 16-byte zero slot
-// (stride 65): the half that carries no data reads the zero slot, so the
-// block-diagonal operand needs no selects.
-template <int NO>
-struct bs32z {
-  u32x4_t lo[NO], hi[NO];
-  float d[NO];
-};
-
-// Per-lane offsets (16-byte units within a step) of the two operand halves:
-// a lane of an odd column (block 2s+1) carries its data in the upper half.
-struct zoff {
-  int lo, hi;
-};
-
-__device__ __forceinline__ zoff make_zoff(int lane) {
-  const bool upper = lane_upper32(lane);
-  return zoff{upper ? 64 : lane, upper ? lane : 64};
-}
-
-template <int NO, int OB, int OD>
-__device__ __forceinline__ void load_bs32z_lds(bs32z<NO> &b, const u32x4_t *bl, const float *dl, const zoff &z,
-                                               int dlo, int step) {
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    b.lo[o] = bl[o * OB + step * 65 + z.lo];
-    b.hi[o] = bl[o * OB + step * 65 + z.hi];
-    b.d[o] = dl[o * OD + step * 16 + dlo];
-  }
-}
-
-template <int NO, int OB>
-__device__ __forceinline__ void load_bs32z_lds_v(bs32z<NO> &b, const u32x4_t *bl, const zoff &z, int step) {
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    b.lo[o] = bl[o * OB + step * 65 + z.lo];
-    b.hi[o] = bl[o * OB + step * 65 + z.hi];
-  }
-}
-
-template <int NO, int OD>
-__device__ __forceinline__ void load_bs32z_lds_d(bs32z<NO> &b, const float *dl, int dlo, int step) {
-#pragma unroll
-  for (int o = 0; o < NO; o++) b.d[o] = dl[o * OD + step * 16 + dlo];
-}
-
-// Step J of a quad (op_sel SEL = quad % 4): acc[o] += d[o] * (A . B[o]) for
-// one weight stream; the per-octet sequence is that of quad_mma32 (same bits).
-template <int SEL, int J, int NO>
-__device__ __forceinline__ void step_mma32z(const wq32<1> &w, const uint32_t (&sc)[1][2], const bs32z<NO> &b, int sb,
-                                            f32x16_t (&acc)[NO][1]) {
-  const u32x4_t a4 = w.w[0][J];
-  const i32x8_t a = {(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w, 0, 0, 0, 0};
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const u32x4_t l = b.lo[o], h = b.hi[o];
-    const i32x8_t bv = {(int)l.x, (int)l.y, (int)l.z, (int)l.w, (int)h.x, (int)h.y, (int)h.z, (int)h.w};
-    f32x16_t z;
-#pragma unroll
-    for (int e = 0; e < 16; e++) z[e] = 0.0f;
-    const f32x16_t r = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, bv, z, 4, 0, SEL, (int)sc[0][J], 0, sb);
-    acc[o][0] = acc[o][0] + b.d[o] * r;
-  }
-#pragma unroll
-  for (int o = 0; o < NO; o++) asm volatile("" : "+v"(acc[o][0]));
-}
-
-// step_mma32z in two parts: the NO MFMAs of the step (results and scales
-// kept), then the scaling into acc (same operations per octet, same bits),
-// so the next step's B can be read from LDS between the two.
-template <int NO>
-struct stepres {
-  f32x16_t r[NO];
-};
-
-template <int SEL, int J, int NO>
-__device__ __forceinline__ void step_mma32z_issue(const u32x4_t &a4, const uint32_t (&sc)[1][2], const bs32z<NO> &b,
-                                                  int sb, stepres<NO> &res) {
-  const i32x8_t a = {(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w, 0, 0, 0, 0};
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const u32x4_t l = b.lo[o], h = b.hi[o];
-    const i32x8_t bv = {(int)l.x, (int)l.y, (int)l.z, (int)l.w, (int)h.x, (int)h.y, (int)h.z, (int)h.w};
-    f32x16_t z;
-#pragma unroll
-    for (int e = 0; e < 16; e++) z[e] = 0.0f;
-    res.r[o] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, bv, z, 4, 0, SEL, (int)sc[0][J], 0, sb);
-  }
-}
-
-template <int NO>
-__device__ __forceinline__ void step_scale(const stepres<NO> &res, const float (&d)[NO], f32x16_t (&acc)[NO][1]) {
-#pragma unroll
-  for (int o = 0; o < NO; o++) acc[o][0] = acc[o][0] + d[o] * res.r[o];
-#pragma unroll
-  for (int o = 0; o < NO; o++) asm volatile("" : "+v"(acc[o][0]));
-}
-
-// One step's weights (step S = 2 * quad + j of the stream), cache policy CPOL.
-template <int CPOL = 0>
-__device__ __forceinline__ void load_w32step(u32x4_t &w, const wstream (&ws)[1], const aoff32 &ao, int S) {
-  const int q = S >> 1, j = S & 1;
-  w = __builtin_amdgcn_raw_buffer_load_b128(ws[0].rec, ao.v + j * 512, (q >> 2) * MOE_REC_BYTES + (q & 3) * 1024,
-                                            CPOL);
-}
-
-#define MOE_DRS 4  // weight ring of the down step loop, in steps
-
-// Ring of the step-B loop: weights of MOE_DRS steps (3 ahead) of one
-// stream, exponent dwords of NG groups, B of the next step (a zero-slot
-// operand, read from LDS between the step's MFMAs and its scaling, so the
-// LDS latency overlaps them; a deeper B ring does not fit 128 registers).
-template <int NO, int NG>
-struct sring {
-  u32x4_t w[MOE_DRS];  // weights of steps S .. S + MOE_DRS - 1 (slot S % MOE_DRS)
-  uint32_t sc[NG][1][2];
-  bs32z<NO> b[1];
-};
-
-// Quads QL .. NQW-1 with B from LDS one step ahead.
-template <int QL, int NQW, int NO, int NG, int OB, int OD>
-__device__ __forceinline__ void slfixed_from(sring<NO, NG> &r, const wstream (&ws)[1], const aoff32 &ao,
-                                             const u32x4_t *bl, const float *dl, const zoff &z, int dlo, int sb,
-                                             f32x16_t (&acc)[NO][1]) {
-  if constexpr (QL < NQW) {
-    if constexpr ((QL & 3) == 0 && (QL >> 2) + 1 < NG) load_sc32<1>(r.sc[(QL >> 2) + 1], ws, ao, (QL >> 2) + 1);
-    constexpr int S0 = 2 * QL, RS = MOE_DRS;
-    if constexpr (S0 + RS - 1 < 2 * NQW) load_w32step(r.w[(S0 + RS - 1) % RS], ws, ao, S0 + RS - 1);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      stepres<NO> res;
-      step_mma32z_issue<QL & 3, 0, NO>(r.w[S0 % RS], r.sc[QL >> 2], r.b[0], sb, res);
-      __builtin_amdgcn_sched_barrier(0);
-      load_bs32z_lds_v<NO, OB>(r.b[0], bl, z, 2 * QL + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      step_scale<NO>(res, r.b[0].d, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      load_bs32z_lds_d<NO, OD>(r.b[0], dl, dlo, 2 * QL + 1);
-    }
-    if constexpr (S0 + RS < 2 * NQW) load_w32step(r.w[(S0 + RS) % RS], ws, ao, S0 + RS);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      stepres<NO> res;
-      step_mma32z_issue<QL & 3, 1, NO>(r.w[(S0 + 1) % RS], r.sc[QL >> 2], r.b[0], sb, res);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (QL + 1 < NQW) load_bs32z_lds_v<NO, OB>(r.b[0], bl, z, 2 * QL + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      step_scale<NO>(res, r.b[0].d, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (QL + 1 < NQW) load_bs32z_lds_d<NO, OD>(r.b[0], dl, dlo, 2 * QL + 2);
-    }
-    slfixed_from<QL + 1, NQW, NO, NG, OB, OD>(r, ws, ao, bl, dl, z, dlo, sb, acc);
-  }
-}
-
-#define MOE_DOL2_WAVES 8
-
-// The item's NO octets of h staged as stage_octet_lds_z lays them out, by
-// direct global-to-LDS loads (buffer_load ... lds): unit u of a step holds
-// row (u>>2)&7 of the octet, block 2*step + (u&1) and 16-byte piece
-// (u>>5) | ((u>>1)&1)<<1; scale f holds row (f>>1)&7 of block
-// 2*(f>>4) + (f&1).  Of the 32*NO (octet, step) loads wave w issues
-// w*4*NO .. w*4*NO + 4*NO - 1 (all of one octet), and of the 8*NO loads of
-// 64 scales w*NO .. w*NO + NO - 1.  Rows past the item read nothing (their
-// columns are never stored).  For 8 waves and KB == 64.
-template <int NO, int KB>
-__device__ __forceinline__ void stage_octets_dma(const gsrc &src, int row0, int nt, uint32_t *lds, int lane,
-                                                 int wave) {
-  static_assert(KB == 64, "32 steps per octet: 4 per wave and octet");
-  typedef __attribute__((address_space(3))) void *lds_t;
-  constexpr int OW = (int)(octet_lds_bytes_z(KB) / 4);  // dwords per staged octet
-  const int o = (wave * NO) >> 3;
-  const int td = (lane >> 2) & 7, ts = (lane >> 1) & 7;
-  const int sub = (lane >> 5) | (((lane >> 1) & 1) << 1);
-  const uint32_t xo = 8 * o + td < nt ? (uint32_t)(((row0 + 8 * o + td) * KB + (lane & 1)) * (MOE_XSW * 4) + sub * 16)
-                                      : MOE_OOB;
-  const uint32_t so = 8 * o + ts < nt ? (uint32_t)(((row0 + 8 * o + ts) * KB + 2 * (lane >> 4) + (lane & 1)) * 4)
-                                      : MOE_OOB;
-  uint32_t *ol = lds + o * OW;
-#pragma unroll
-  for (int j = 0; j < 4 * NO; j++) {
-    const int st = (wave * 4 * NO + j) & 31;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.x, (lds_t)(ol + st * 65 * 4), 16, xo, 2 * st * (MOE_XSW * 4), 0, 0);
-  }
-#pragma unroll
-  for (int j = 0; j < NO; j++) {
-    const int hh = (wave * NO + j) & 7;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.d, (lds_t)(ol + (KB / 2) * 65 * 4 + hh * 64), 4, so, 8 * hh * 4, 0,
-                                             0);
-  }
-}
-
-// The down work of one wave against NO octets staged at lds (octet o at
-// dword o * octet_lds_bytes(KB) / 4): y of token 8*o + t of the item.
-template <int NQ, int NO>
-__device__ __forceinline__ void dn_ol_octets(const wstream (&ws)[1], const aoff32 &ao, uint32_t *lds,
-                                             const uint32_t *__restrict__ hs, const float *__restrict__ hd,
-                                             int n_rows, const int4 &it, const int32_t *__restrict__ perm,
-                                             const float *__restrict__ wts, int H, int t32, int lane,
-                                             float *__restrict__ y) {
-  constexpr int NQ4 = (NQ + 3) / 4, NG = NQ4, KB = NQ * 4;
-  constexpr int OW = (int)(octet_lds_bytes_z(KB) / 4);  // dwords per staged octet
-  const int row0 = it.y, nt = it.z;
-  const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
-  sring<NO, NG> r;
-  if constexpr (KB == 64) {
-    // the h loads straight into LDS first, then the first weights, then the
-    // zero slots; the h loads are waited for (vmcnt) right before the barrier
-    stage_octets_dma<NO, KB>(make_gsrc(hs, hd, n_rows, KB), row0, nt, lds, threadIdx.x & 63,
-                             __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    load_sc32<1>(r.sc[0], ws, ao, 0);
-#pragma unroll
-    for (int i = 0; i + 1 < MOE_DRS; i++)
-      if (i < 2 * NQ) load_w32step(r.w[i], ws, ao, i);
-#pragma unroll
-    for (int o = 0; o < NO; o++)
-      for (int c = threadIdx.x; c < KB / 2; c += 64 * MOE_DOL2_WAVES)
-        reinterpret_cast<u32x4_t *>(lds + o * OW)[c * 65 + 64] = u32x4_t{0u, 0u, 0u, 0u};
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 + (MOE_DRS - 1 < 2 * NQ ? MOE_DRS - 1 : 2 * NQ)));
-    lds_barrier();
-  } else {
-    // first weights in flight during the staging
-    load_sc32<1>(r.sc[0], ws, ao, 0);
-#pragma unroll
-    for (int i = 0; i + 1 < MOE_DRS; i++)
-      if (i < 2 * NQ) load_w32step(r.w[i], ws, ao, i);
-#pragma unroll
-    for (int o = 0; o < NO; o++) {
-      uint32_t *ol = lds + o * OW;
-      stage_octet_lds_z(hs, hd, row0 + 8 * o, nt - 8 * o, KB, reinterpret_cast<u32x4_t *>(ol),
-                        reinterpret_cast<float *>(ol + (KB / 2) * 65 * 4), threadIdx.x, 64 * MOE_DOL2_WAVES);
-    }
-    __syncthreads();
-  }
-  const u32x4_t *bl = reinterpret_cast<const u32x4_t *>(lds);
-  const float *dl = reinterpret_cast<const float *>(lds + (KB / 2) * 65 * 4);
-  const int n = lane & 31, gb = lane >> 5, t = n >> 2;
-  const int dlo = t * 2 + (n & 1);
-  f32x16_t acc[NO][1];
-#pragma unroll
-  for (int o = 0; o < NO; o++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[o][0][e] = 0.0f;
-  const zoff z = make_zoff(lane);
-  load_bs32z_lds<NO, OW / 4, OW>(r.b[0], bl, dl, z, dlo, 0);
-  slfixed_from<0, NQ, NO, NG, OW / 4, OW>(r, ws, ao, bl, dl, z, dlo, lane_bscale32(lane), acc);
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const int tt = 8 * o + t;
-    const bool live = tt < nt;
-    const int rr = row0 + (live ? tt : 0);
-    const float wt = (live && !shared) ? wts[perm[rr]] : 1.0f;
-    float v[16];
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      v[e] = col4_sum(acc[o][0][e]);
-      if (!shared) v[e] = __fmul_rn(v[e], wt);
-    }
-    if ((n & 3) == 0 && live) {
-      float *dst = y + (size_t)rr * H + (size_t)t32 * 32 + 4 * gb;
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        *reinterpret_cast<float4 *>(dst + 8 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    }
-  }
-}
-
-// k_down_ol on items of up to 16 rows: a workgroup of 8 waves stages the
-// item's two octets of h in LDS (octet 1 only when the item holds more than
-// 8 rows) and each wave multiplies its 32-row tile of H against both from
-// the same weight registers, so one pass over the item's down weights
-// serves 16 tokens.  Both halves of each block-diagonal B operand come from
-// LDS (the half without data from the step's zero slot: no selects), one
-// step ahead, which keeps the wave within 128 VGPRs (4 waves per SIMD with
-// two workgroups per CU).  Per token the MFMA and scaling sequence is
-// k_down_ol's (same bits).  grid (H/256, item capacity), 512 threads, LDS
-// 2 * octet_lds_bytes_z(F/32).
-template <int NQ>
-__global__ __launch_bounds__(64 * MOE_DOL2_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
-void k_down_ol2(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, const float *__restrict__ hd,
-                int n_rows, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
-                const float *__restrict__ wts, int F, int H, float *__restrict__ y) {
-  extern __shared__ __align__(16) uint32_t lds[];
-  if ((int)blockIdx.y >= items[0]) return;
-  const int4 it = item_of(items, blockIdx.y);
-  constexpr int NQ4 = (NQ + 3) / 4;
-  const int tiles = H / MOE_TILE;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int t32 = blockIdx.x * MOE_DOL2_WAVES + wave;  // 32-row tile of H
-  const int nt = it.z;
-  const wstream ws[1] = {make_wstream32(w_d, (size_t)it.x * tiles + 2 * t32, NQ4)};
-  const aoff32 ao = make_aoff32(lane, NQ4);
-  if (nt > 8) dn_ol_octets<NQ, 2>(ws, ao, lds, hs, hd, n_rows, it, perm, wts, H, t32, lane, y);  // uniform branch
-  else dn_ol_octets<NQ, 1>(ws, ao, lds, hs, hd, n_rows, it, perm, wts, H, t32, lane, y);
-}
-
-// ===========================================================================
-// Grouped gate/up with the item's B staged in LDS, chunk by chunk of K.
-//
-// One workgroup of 2*NU waves per (NU units of F, item of <= 16 rows): wave
-// w streams the gate (w < NU) or up tile of unit NU*blockIdx.x + w%NU over
-// all of K against the item's one or two octets.  The workgroup copies
-// B (the octets' x rows) into LDS in chunks of MOE_GCH quads, already in
-// MFMA lane order (the layout of stage_octet_lds, per chunk, each step's 64
-// lanes followed by a 16-byte zero slot), double buffered: chunk c+1 goes
-// out at chunk c's first quad as direct global-to-LDS loads and is waited
-// for only at the chunk's end barrier.  Every B byte thus crosses the
-// vector-memory unit once per workgroup and never occupies a VGPR; a wave
-// reads both halves of each MFMA operand from LDS (the half without data
-// from the zero slot, so no selects) and holds one weight stream with a
-// ring of MOE_GU_RS steps: 128 VGPRs, 4 waves per SIMD, which beat deeper
-// rings at 3 waves.  Each step issues its MFMAs (one result register set
-// per octet), then the next step's B reads, then the scaling FMAs, so the
-// LDS round trip overlaps the MFMAs and the FMAs instead of following them.
-// After the K loop gate and up meet in LDS for clamp + SwiGLU + Q8_0(h) as
-// in k_gate_up_o.
-#define MOE_GCH 4                                  // quads per staged chunk
-#define MOE_GCH_STEPS (2 * MOE_GCH)                // MFMA steps per chunk
-#define MOE_GCH_OCT_U4 (MOE_GCH_STEPS * 65)        // 16-byte units per octet per chunk (digits, zero slots)
-#define MOE_GCH_OCT_D (MOE_GCH_STEPS * 16)         // scales per octet per chunk
-#define MOE_GCH_BUF_DW (2 * MOE_GCH_OCT_U4 * 4 + 2 * MOE_GCH_OCT_D)  // dwords per chunk buffer (two octets)
-
-
-// The staging of a chunk by direct global-to-LDS loads (buffer_load ... lds):
-// a wave's loads write 64 consecutive 16-byte units (one octet's step, lane
-// u = unit u) or 64 consecutive scales, so the data never passes through
-// VGPRs.  Unit u of a step holds token (u>>2)&7, block 2*step + (u&1) of the
-// chunk and 16-byte piece (u>>5) | ((u>>1)&1)<<1 of that block; scale f of
-// an octet's 128 holds token (f>>1)&7 of block 2*(f>>4) + (f&1).  Of the
-// 8*NO (octet, step) loads of a chunk wave w issues w*NO .. w*NO+NO-1 (all
-// of one octet), and waves 0 .. 2*NO-1 one half of an octet's scales each.
-// The loads of chunk c+1 go out at chunk c's first quad; the wave waits for
-// them (vmcnt) only right before the chunk's end barrier.
-struct gdma {
-  uint32_t xo;  // this lane's digit bytes at chunk 0 (MOE_OOB: absent token)
-  uint32_t so;  // this lane's scale at chunk 0 (MOE_OOB: absent, or no scale load for this wave)
-};
-
-template <int NO>
-__device__ __forceinline__ gdma make_gdma(int lane, int wave, int xr_dig, int xr_sc, int KB) {
-  gdma g;
-  const int sub = (lane >> 5) | (((lane >> 1) & 1) << 1);
-  g.xo = xr_dig >= 0 ? (uint32_t)((xr_dig * KB + (lane & 1)) * (MOE_XSW * 4) + sub * 16) : MOE_OOB;
-  g.so = (wave < 2 * NO && xr_sc >= 0) ? (uint32_t)((xr_sc * KB + 2 * (lane >> 4) + (lane & 1)) * 4) : MOE_OOB;
-  return g;
-}
-
-template <int NO, int NX, int C>
-__device__ __forceinline__ void gdma_issue(const gdma &g, const gsrc &src, uint32_t *buf, int wave) {
-  typedef __attribute__((address_space(3))) void *lds_t;
-#pragma unroll
-  for (int j = 0; j < NO; j++) {
-    const int i = wave * NO + j, o = i >> 3, st = i & 7;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.x, (lds_t)(buf + (o * MOE_GCH_OCT_U4 + st * 65) * 4), 16, g.xo,
-                                             (16 * C + 2 * st) * (MOE_XSW * 4), 0, 0);
-  }
-  if (wave < 2 * NO) {
-    const int o = wave >> 1, hh = wave & 1;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.d, (lds_t)(buf + NX * MOE_GCH_OCT_U4 * 4 + o * MOE_GCH_OCT_D + hh * 64),
-                                             4, g.so, (16 * C + 8 * hh) * 4, 0, 0);
-  }
-}
-
-// The digits (lo, hi) and the scales of one step's B, read apart.
-template <int NO>
-__device__ __forceinline__ void load_bs32_chunk_v(bs32z<NO> &b, const uint32_t *buf, const zoff &z, int ls) {
-  const u32x4_t *bl = reinterpret_cast<const u32x4_t *>(buf);
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    b.lo[o] = bl[o * MOE_GCH_OCT_U4 + ls * 65 + z.lo];
-    b.hi[o] = bl[o * MOE_GCH_OCT_U4 + ls * 65 + z.hi];
-  }
-}
-
-template <int NO>
-__device__ __forceinline__ void load_bs32_chunk_d(bs32z<NO> &b, const uint32_t *buf, int dlo, int ls) {
-  const float *dl = reinterpret_cast<const float *>(buf) + 2 * MOE_GCH_OCT_U4 * 4;
-#pragma unroll
-  for (int o = 0; o < NO; o++) b.d[o] = dl[o * MOE_GCH_OCT_D + ls * 16 + dlo];
-}
-
-template <int NO>
-__device__ __forceinline__ void load_bs32_chunk(bs32z<NO> &b, const uint32_t *buf, const zoff &z, int dlo, int ls) {
-  load_bs32z_lds<NO, MOE_GCH_OCT_U4, MOE_GCH_OCT_D>(b, reinterpret_cast<const u32x4_t *>(buf),
-                                                    reinterpret_cast<const float *>(buf) + 2 * MOE_GCH_OCT_U4 * 4, z,
-                                                    dlo, ls);
-}
-
-#define MOE_GU_RS 4  // weight ring of the gate/up step loop, in steps (3 ahead)
-
-template <int NO, int NG>
-struct gring {
-  u32x4_t w[MOE_GU_RS];  // weights of steps S .. S + MOE_GU_RS - 1 (slot S % MOE_GU_RS)
-  uint32_t sc[NG][1][2];
-  bs32z<NO> b[1];
-};
-
-// VMEM loads a wave issues after its chunk-C staging loads, up to the end of
-// the chunk (the exponent dwords of the next group, two weight steps a quad).
-template <int C, int NQ, int NG>
-__host__ __device__ constexpr int gdma_after() {
-  int n = 0;
-  if (C + 1 < NG) n += 2;
-  for (int qc = 0; qc < MOE_GCH; qc++) {
-    const int S0 = 2 * (MOE_GCH * C + qc);
-    if (S0 + MOE_GU_RS - 1 < 2 * NQ) n++;
-    if (S0 + MOE_GU_RS < 2 * NQ) n++;
-  }
-  return n;
-}
-
-// Quads QL .. NQ-1 of the chunked K loop.
-template <int QL, int NQ, int NO, int NG>
-__device__ __forceinline__ void gl_from(gring<NO, NG> &r, const wstream (&ws)[1], const aoff32 &ao,
-                                        const gsrc &src, const gdma &g, uint32_t *lds, int wave, const zoff &z,
-                                        int dlo, int sb, f32x16_t (&acc)[NO][1]) {
-  if constexpr (QL < NQ) {
-    constexpr int C = QL / MOE_GCH, QC = QL % MOE_GCH, NC = NQ / MOE_GCH, RS = MOE_GU_RS;
-    const uint32_t *buf = lds + (C & 1) * MOE_GCH_BUF_DW;
-    if constexpr (C + 1 < NC && QC == 0) {  // the next chunk's staging, straight into the other buffer
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      gdma_issue<NO, 2, C + 1>(g, src, lds + ((C + 1) & 1) * MOE_GCH_BUF_DW, wave);
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if constexpr ((QL & 3) == 0 && (QL >> 2) + 1 < NG) load_sc32<1>(r.sc[(QL >> 2) + 1], ws, ao, (QL >> 2) + 1);
-    constexpr int S0 = 2 * QL;
-    if constexpr (S0 + RS - 1 < 2 * NQ) load_w32step(r.w[(S0 + RS - 1) % RS], ws, ao, S0 + RS - 1);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      stepres<NO> res;
-      step_mma32z_issue<QL & 3, 0, NO>(r.w[S0 % RS], r.sc[QL >> 2], r.b[0], sb, res);
-      __builtin_amdgcn_sched_barrier(0);
-      load_bs32_chunk_v<NO>(r.b[0], buf, z, 2 * QC + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      step_scale<NO>(res, r.b[0].d, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      load_bs32_chunk_d<NO>(r.b[0], buf, dlo, 2 * QC + 1);
-    }
-    if constexpr (S0 + RS < 2 * NQ) load_w32step(r.w[(S0 + RS) % RS], ws, ao, S0 + RS);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      stepres<NO> res;
-      step_mma32z_issue<QL & 3, 1, NO>(r.w[(S0 + 1) % RS], r.sc[QL >> 2], r.b[0], sb, res);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (QC + 1 < MOE_GCH) load_bs32_chunk_v<NO>(r.b[0], buf, z, 2 * QC + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      step_scale<NO>(res, r.b[0].d, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (QC + 1 < MOE_GCH) load_bs32_chunk_d<NO>(r.b[0], buf, dlo, 2 * QC + 2);
-    }
-    if constexpr (QC + 1 == MOE_GCH && C + 1 < NC) {
-      // the next chunk has landed in LDS (this wave's loads, then everyone's)
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(gdma_after<C, NQ, NG>()));
-      uint32_t *nb = lds + ((C + 1) & 1) * MOE_GCH_BUF_DW;
-      lds_barrier();
-      load_bs32_chunk<NO>(r.b[0], nb, z, dlo, 0);
-    }
-    gl_from<QL + 1, NQ, NO, NG>(r, ws, ao, src, g, lds, wave, z, dlo, sb, acc);
-  }
-}
-
-// The K loop of one wave (of 8: NU = 4) against NO octets; xrow(i) = the
-// staged x row of the item's token i (< 0: absent).  Leaves this wave's sums
-// (the 4 columns of a token added) in red[w%NU][w/NU][token][row].
-template <int NQ, int NO, int NU, class XR>
-__device__ __forceinline__ void gu_ol_octets(const wstream (&ws)[1], const aoff32 &ao, const gsrc &src,
-                                             const XR &xrow, int KB, uint32_t *lds, int tid, int wave, int lane) {
-  static_assert(NU == 4, "the staging loads are laid out for 8 waves");
-  constexpr int NQ4 = (NQ + 3) / 4, NG = NQ4, RS = MOE_GU_RS;
-  const int xr_dig = xrow(8 * ((wave * NO) >> 3) + ((lane >> 2) & 7));
-  const int xr_sc = wave < 2 * NO ? xrow(8 * (wave >> 1) + ((lane >> 1) & 7)) : -1;
-  const gdma g = make_gdma<NO>(lane, wave, xr_dig, xr_sc, KB);
-  gring<NO, NG> r;
-  // chunk 0 straight into LDS, then the first weights
-  gdma_issue<NO, 2, 0>(g, src, lds, wave);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  load_sc32<1>(r.sc[0], ws, ao, 0);
-#pragma unroll
-  for (int i = 0; i + 1 < RS; i++)
-    if (i < 2 * NQ) load_w32step(r.w[i], ws, ao, i);
-  if (tid < 2 * 2 * MOE_GCH_STEPS) {  // the zero slots of both chunk buffers, never written by the staging
-    const int bf = tid / (2 * MOE_GCH_STEPS), o = (tid / MOE_GCH_STEPS) & 1, st = tid % MOE_GCH_STEPS;
-    reinterpret_cast<u32x4_t *>(lds + bf * MOE_GCH_BUF_DW)[o * MOE_GCH_OCT_U4 + st * 65 + 64] =
-        u32x4_t{0u, 0u, 0u, 0u};
-  }
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  // the chunk-0 loads have landed (2 exponent dwords and RS-1 weight steps went out after them)
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 + (RS - 1 < 2 * NQ ? RS - 1 : 2 * NQ)));
-  lds_barrier();
-  const int n = lane & 31, gb = lane >> 5, t = n >> 2;
-  const int dlo = t * 2 + (n & 1);
-  f32x16_t acc[NO][1];
-#pragma unroll
-  for (int o = 0; o < NO; o++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[o][0][e] = 0.0f;
-  const zoff z = make_zoff(lane);
-  load_bs32_chunk<NO>(r.b[0], lds, z, dlo, 0);
-  gl_from<0, NQ, NO, NG>(r, ws, ao, src, g, lds, wave, z, dlo, lane_bscale32(lane), acc);
-  lds_barrier();  // every wave is done with the chunk buffers, which now hold the sums
-  float *red = reinterpret_cast<float *>(lds);  // [unit][gate/up][token][row]
-#pragma unroll
-  for (int o = 0; o < NO; o++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const float v = col4_sum(acc[o][0][e]);
-      if ((n & 3) == 0)
-        red[(((wave % NU) * 2 + wave / NU) * 16 + 8 * o + (n >> 2)) * MOE_UNIT + 8 * (e >> 2) + 4 * gb + (e & 3)] = v;
-    }
-}
-
-// grid (F/(32 NU), item capacity), 128*NU threads (NU units of F: wave w
-// streams the gate (w < NU) or up tile of unit NU*blockIdx.x + w%NU), LDS
-// 2 * MOE_GCH_BUF_DW dwords.  With NU = 4 the item's staged x serves twice
-// the weight rows of NU = 2, so the x rows are a fifth of the bytes a
-// workgroup moves instead of a third.  Requires H == 128 * NQ,
-// NQ % MOE_GCH == 0, (F/32) % NU == 0.
-template <int NQ, int NU>
-__global__ __launch_bounds__(128 * NU) __attribute__((amdgpu_waves_per_eu(4)))
-void k_gate_up_ol(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_u, const uint32_t *__restrict__ xq,
-                  const float *__restrict__ xd, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
-                  int k, int T, int F, int H, float clamp, uint32_t *__restrict__ hs, float *__restrict__ hd,
-                  float *__restrict__ htap) {
-  __shared__ __align__(16) uint32_t lds[2 * MOE_GCH_BUF_DW];
-  if ((int)blockIdx.y >= items[0]) return;
-  const int4 it = item_of(items, blockIdx.y);
-  constexpr int NQ4 = (NQ + 3) / 4, KB = NQ * 4;
-  const int U = F / MOE_UNIT, tiles = F / MOE_TILE;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int P = T * k, row0 = it.y, nt = it.z;
-  const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
-  const int u = NU * blockIdx.x + wave % NU;
-  const wstream ws[1] = {make_wstream32(wave >= NU ? w_u : w_g, (size_t)it.x * tiles + 2 * u, NQ4)};
-  const aoff32 ao = make_aoff32(lane, NQ4);
-  const gsrc src = make_gsrc(xq, xd, T, KB);
-  auto xrow = [&](int i) { return i < nt ? (shared ? row0 + i - P : perm[row0 + i] / k) : -1; };
-  if (nt > 8) gu_ol_octets<NQ, 2, NU>(ws, ao, src, xrow, KB, lds, tid, wave, lane);  // uniform branch
-  else gu_ol_octets<NQ, 1, NU>(ws, ao, src, xrow, KB, lds, tid, wave, lane);
-  __syncthreads();
-  const float *red = reinterpret_cast<const float *>(lds);
-  // (unit, token) c = 4*NU*round + 2*wave + half-wave: unit c / 16, token c % 16
-#pragma unroll
-  for (int round = 0; round < 4; round++) {
-    const int c = 4 * NU * round + 2 * wave + (lane >> 5);
-    const int ul2 = c >> 4, t = c & 15, j = lane & 31;
-    if (((4 * NU * round) & 15) >= nt && NU == 2) continue;  // no token of this round (uniform over the workgroup)
-    const bool live = t < nt;
-    const float gsum = red[((ul2 * 2 + 0) * 16 + t) * MOE_UNIT + j];
-    const float usum = red[((ul2 * 2 + 1) * 16 + t) * MOE_UNIT + j];
-    const float h = live ? swiglu(gsum, usum, clamp) : 0.0f;
-    const int hrow = row0 + (live ? t : 0), uu = NU * blockIdx.x + ul2;
-    h_unit_store(h, live, hs + ((size_t)hrow * U + uu) * MOE_XSW, hd + (size_t)hrow * U + uu, lane);
-    if (htap && live) htap[(size_t)hrow * F + (size_t)uu * MOE_UNIT + j] = h;
   }
 }

@@ -1,119 +1,248 @@
 // kernels_stacked.h -- grouped gate/up and down on items of up to 32 rows,
-// the two Q8_0 digit planes stacked along K of one MFMA.
+// the two Q8_0 digit planes stacked along K of one MFMA, in fp6.
 //
-// v_mfma_scale_f32_32x32x64_f8f6f4 reduces 64 K per output value.  Here A
-// is the item's tokens (A row t = token t) and B the weight tile (B column
-// r = weight row r), and the 64 K are one MXFP4 block twice: K 0-31 carry
-// the block's hi digits (A scale 2^4), K 32-63 its lo digits (A scale 2^0),
-// and both B lane halves (lane r + 32*gb, gb = 0, 1) hold the same weight
-// block of row r with its exponent.  D[t][r] is then 2^(e_w - 127) times
-// the exact integer block dot of token t and row r (16*hi + lo = q): one
-// MFMA is 32 tokens x 32 rows x one block with no zero half, and each
-// result value is scaled by its token's d once.  Against an item of up to
-// 32 rows one pass over the expert's weights serves every row of the item,
-// so an expert with 17-32 rows is streamed once, not twice.
+// v_mfma_scale_f32_32x32x64_f8f6f4 reduces 64 K per output value.  Here A is
+// the weight tile (A row r = weight row r, fp4 with its E8M0 exponent) and B
+// the item's tokens (B column n = token n), and the 64 K are one MXFP4 block
+// twice: K 0-31 carry the block's hi digits (B scale 2^4), K 32-63 its lo
+// digits (2^0), and both A lane halves hold the same weight block.  D[r][n]
+// is then 2^(e_w - 127) times the exact integer block dot of row r and token
+// n (16*hi + lo = q), scaled by the token's d and added in f32, block by
+// block.
 //
-// Tokens are A's rows so that a lane's 16 result values are 16 tokens of one
-// weight row (D lane r + 32*gb holds column r, tokens 8*i + 4*gb + j at
-// element 4*i + j): the d scaling of the tokens an item lacks is skipped
-// whole, 4 FMAs per 8 tokens (an item of 9-16 rows pays 8 FMAs per MFMA, not
-// 16), at the price of each lane reading its tokens' d as float4s.
+// The digits (hi in [-8, 7], lo in [0, 15]) are e2m3 codes (fp6: digit / 8,
+// the code of a magnitude is the magnitude itself, the sign bit 32), not e4m3:
+// with fp6 an MFMA takes 45-54 cycles instead of 77 (random operands, the
+// clock that the chip holds under them), and a token's block 48 bytes instead
+// of 64.
 //
-// Operand lanes (the layouts the octet kernels use): B lane r + 32*gb holds
-// weight row r and K [32*gb, 32*gb + 32); the record layout gives lane (r, gb)
-// block 2j + gb of a quad in one load (step j), and v_permlane32_swap turns
-// that pair into [block 2j | block 2j] and [block 2j+1 | block 2j+1].  A lane
-// t + 32*ga holds token t: bytes 0-15 = K [16*ga, +16) (hi digits 16*ga ..
-// 16*ga + 15), bytes 16-31 = K [32 + 16*ga, +16) (lo digits, same offsets).
-// The A scale of lane t + 32*ga is that of K block ga (hi: 2^4, lo: 2^0).
+// Staged activations ("quad records"): per row and quad of 4 blocks 208 bytes
+//   [0, 96)    hi digits of blocks 0..3, 24 bytes each (6 bits per K offset)
+//   [96, 192)  lo digits, likewise
+//   [192, 208) d of the 4 blocks, f32
+// rows of records one after another.  A chunk of 4 quads of a row is one run
+// of 832 bytes, and the direct global-to-LDS loads of a chunk (1 KiB each)
+// read such runs in order, about 10 cache lines per load; with one 16-byte
+// piece per (token, block) and load, 64 lines, the load path bounds the kernel
+// (a build that staged 96 bytes per block that way: gate/up of 2048 tokens on
+// the V3 layer 2003 us, 1353 us with the same bytes contiguous).
 //
-// A is staged in LDS by chunks of MOE_SK_CH quads (8 blocks), double
-// buffered, with direct global-to-LDS loads: per block, two 1 KiB runs (the
-// 64 lanes' bytes 0-15, then bytes 16-31, each lane 16 consecutive bytes,
-// so the operand reads are conflict-free), then the chunk's scales
-// [block][32 tokens].  An absent token reads zeros (out-of-range offset).
-// The x rows are read from the grouped chain's staged x; the h rows that
-// k_gate_up_sk writes for k_down_sk are block-major, so the 32 rows of an
-// item are adjacent for each block.
+// What bounds them (V3 layer): at 512 tokens, uniform, the weight stream
+// (gate/up 740 us, 712 us with the staging and the scaling left out; the bare
+// stream of the same bytes 560 us); at 2048 tokens the vector issue, 26
+// instructions per MFMA in 88% of the cycles at the 1.5 GHz that the chip
+// holds.  Measured on one box against the e4m3 digits staged in pieces:
+// prefill 512 uniform 1200 -> 1153 us, Zipf 808 -> 732 us, 2048 tokens 2761 ->
+// 2368 us, the V4-Pro layer 927 -> 833 us; 300 tokens on a 5120 x 1536 layer,
+// where the 8-row octet kernels ran, 563 -> 413 us.
+//
+// Operand lanes.  A lane r + 32*g holds weight row r, K [32g, 32g + 32): the
+// record layout gives lane (r, g) block 2j + g of a quad in one load, and
+// v_permlane32_swap turns that pair into [block 2j | block 2j] and [block
+// 2j+1 | block 2j+1].  B lane n + 32*g holds token n's hi (g = 0) or lo (g = 1)
+// digits, 24 bytes.  D lane n + 32*g holds token n, rows 8i + 4g + j at element
+// 4i + j: a lane has one d, and the epilogues need no exchange (a lane holds
+// gate and up of the same values).
 #pragma once
 
 #include "kernels_grouped.h"
 
-#define MOE_SK_CH 2                            // quads per staged chunk (4: 16 blocks, 100 VGPRs, measured 2% slower)
-#define MOE_SK_STEPS (4 * MOE_SK_CH)           // blocks (MFMA steps) per chunk
-#define MOE_SK_STEP_U4 128                     // 16-byte units per block: [2 halves][64 lanes]
-#define MOE_SK_SC_DW (MOE_SK_STEPS * MOE_SK_STEP_U4 * 4)  // dword offset of the scales in a chunk buffer
-#define MOE_SK_BUF_DW (MOE_SK_SC_DW + MOE_SK_STEPS * 32)  // dwords per chunk buffer (17 KiB)
-#define MOE_SK_LDS_BYTES (2 * MOE_SK_BUF_DW * 4)          // two chunk buffers (34 KiB)
-#define MOE_SK_DN_LDS_BYTES (MOE_SK_LDS_BYTES + MOE_SK_WAVES * 32 * 4)  // k_down_sk: + 32 router weights per wave
-#define MOE_SK_WAVES 8                          // waves per workgroup (one 32-row weight tile each)
-#define MOE_SK_RP 4  // weight ring, in block pairs (3 ahead: 3 KiB in flight per wave; 2 and 5 ahead measured the same)
+#define MOE_SQ_DW 52    // dwords of a quad record
+#define MOE_SQ_U4 13    // its 16-byte units (odd: the operand reads of 8 tokens hit 8 bank groups)
+#define MOE_SK_CH 4     // quads per staged chunk
+#define MOE_SK_ROWS 32  // rows of an item
+#define MOE_SK_BUF_DW (MOE_SK_CH * MOE_SK_ROWS * MOE_SQ_DW)  // 26 KiB
+#define MOE_SK_DMA (MOE_SK_BUF_DW / 256)                     // 1 KiB loads per chunk (26)
+#define MOE_SK_NBUF 2
+#define MOE_SK_LDS_BYTES (MOE_SK_NBUF * MOE_SK_BUF_DW * 4)
+#define MOE_SK_WAVES 4
+#define MOE_SK_WDMA ((MOE_SK_DMA + MOE_SK_WAVES - 1) / MOE_SK_WAVES)  // loads per wave and chunk (7; waves 2, 3: 6)
+#define MOE_SK_OOB 0xffffff00u  // a lane offset past any staged buffer: the load returns 0
 
-// This lane's staging offsets at block 0 of the staged rows (MOE_OOB: absent
-// token): digits of token lane&31, K half lane>>5; scale of token lane&31,
-// block lane>>5.  The staged rows are row-major ([row][block], x) or
-// block-major ([block][row], the h rows these kernels write): bs / bs4 =
-// bytes from one block to the next of a row, digits / scales.
-struct sdma {
-  uint32_t xo, so, bs, bs4;
+// ---------------------------------------------------------------------------
+// Q8_0 into quad records
+
+// Eight digits (K order) of one plane as 48 bits, from digits packed one per byte.
+__device__ __forceinline__ uint32_t pack6x4(uint32_t b) {  // 4 bytes of 6 bits -> 24 bits
+  const uint32_t x = (b & 0x003f003fu) | ((b >> 2) & 0x0fc00fc0u);
+  return (x & 0xfffu) | ((x >> 4) & 0xfff000u);
+}
+
+// The fp6 codes of q's digits: lo in byte 0, hi in byte 1.
+__device__ __forceinline__ uint32_t digit_codes(int q) {
+  const int hi = q >> 4;
+  return (uint32_t)(q & 15) | (uint32_t)(hi < 0 ? 32 - hi : hi) << 8;
+}
+
+// Codes of 8 values in K order -> 48 bits of lo digits and of hi digits.
+struct half48 {
+  uint32_t lo, hi;  // low 32 and high 16 bits
 };
 
-__device__ __forceinline__ sdma make_sdma(int lane, int xr, int KB, bool block_major, int n_rows) {
+__device__ __forceinline__ void pack_digits8(const uint32_t (&c)[8], half48 &l, half48 &h) {
+  uint32_t yl[2], yh[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t *a = c + 4 * i;
+    // v_perm selects bytes 0-3 from the second operand, 4-7 from the first
+    const uint32_t t0 = __builtin_amdgcn_perm(a[1], a[0], 0x05010400u);  // lo0 lo1 hi0 hi1
+    const uint32_t t1 = __builtin_amdgcn_perm(a[3], a[2], 0x05010400u);
+    yl[i] = pack6x4(__builtin_amdgcn_perm(t1, t0, 0x05040100u));
+    yh[i] = pack6x4(__builtin_amdgcn_perm(t1, t0, 0x07060302u));
+  }
+  l.lo = yl[0] | (yl[1] << 24);
+  l.hi = yl[1] >> 8;
+  h.lo = yh[0] | (yh[1] << 24);
+  h.hi = yh[1] >> 8;
+}
+
+// 48 + 48 bits: half a block's digits of one plane.
+__device__ __forceinline__ void join48(const half48 &a, const half48 &b, uint32_t *dst) {
+  dst[0] = a.lo;
+  dst[1] = a.hi | (b.lo << 16);
+  dst[2] = (b.lo >> 16) | (b.hi << 16);
+}
+
+// Q8_0 of nb blocks (whole rows of a multiple of 4 blocks, from a quad's first
+// block on) into quad records; two lanes per block, lane half h the K offsets
+// 16h .. 16h + 15 (offset 2i: element 8h + i, 2i + 1: element 16 + 8h + i).
+__device__ __forceinline__ void stage_quant_quads(const float *__restrict__ x, int nb, uint32_t *xs, int tid, int nthr) {
+  const int h = tid & 1;
+  for (int b = tid >> 1; b < nb; b += nthr >> 1) {
+    const float4 *xb = reinterpret_cast<const float4 *>(x + (size_t)b * MOE_QK + 8 * h);
+    const float4 a0 = xb[0], a1 = xb[1], c0 = xb[4], c1 = xb[5];
+    const float v[16] = {a0.x, c0.x, a0.y, c0.y, a0.z, c0.z, a0.w, c0.w,
+                         a1.x, c1.x, a1.y, c1.y, a1.z, c1.z, a1.w, c1.w};
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(v[i]));
+    amax = fmaxf(amax, dpp_f<0xB1>(amax));  // partner lane (lane ^ 1) holds the other half
+    half48 l[2], u[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      uint32_t code[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) code[i] = digit_codes((int)q8_code(v[8 * c + i], amax));
+      pack_digits8(code, l[c], u[c]);
+    }
+    uint32_t *rec = xs + (size_t)(b >> 2) * MOE_SQ_DW;
+    join48(u[0], u[1], rec + (b & 3) * 6 + 3 * h);
+    join48(l[0], l[1], rec + 24 + (b & 3) * 6 + 3 * h);
+    if (!h) rec[48 + (b & 3)] = __builtin_bit_cast(uint32_t, (float)q8_scale_f16(amax));
+  }
+}
+
+// The 32 h values of a token's unit, 16 in each of the lanes n and n + 32
+// (h[4i + j] = row 8i + 4g + j), as Q8_0 into block b of quad record rec.
+__device__ __forceinline__ void h_quad_store(const float (&h)[16], bool live, uint32_t *rec, int b, int lane) {
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(h[i]));
+  amax = fmaxf(amax, __shfl_xor(amax, 32));
+  // rows 8c + 4g + (0..3) and the same + 16: K offsets 16c + 8g + (0..7)
+  half48 l[2], u[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    uint32_t code[8];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      code[2 * j] = digit_codes((int)q8_code(h[4 * c + j], amax));
+      code[2 * j + 1] = digit_codes((int)q8_code(h[8 + 4 * c + j], amax));
+    }
+    pack_digits8(code, l[c], u[c]);
+  }
+  // lane n collects the hi digits of both lanes, lane n + 32 the lo digits,
+  // of K offsets 0-15 (c = 0) and 16-31 (c = 1)
+  uint32_t o[6];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const auto a = __builtin_amdgcn_permlane32_swap(u[c].lo, l[c].lo, false, false);
+    const auto e = __builtin_amdgcn_permlane32_swap(u[c].hi, l[c].hi, false, false);
+    join48(half48{a[0], e[0]}, half48{a[1], e[1]}, o + 3 * c);
+  }
+  const int g = lane >> 5;
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < 6; i++) rec[24 * g + 6 * b + i] = o[i];
+    if (!g) rec[48 + b] = __builtin_bit_cast(uint32_t, (float)q8_scale_f16(amax));
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Staging of a chunk: 1 KiB load i = wave, wave + 4, ... fills the units [64i,
+// 64i + 64) of [quad][token][unit].
+struct sdma {
+  const uint32_t *src;
+  uint32_t bytes;
+  uint32_t vo[MOE_SK_WDMA];  // this lane's offsets at chunk 0
+  int wave, chunks;
+};
+
+// row: the staged row of token lane % 32 (< 0: absent), of `rows` rows of NQ quads.
+__device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ, int row, int lane, int wave) {
   sdma s;
-  const uint32_t rs = block_major ? MOE_XSW * 4 : (uint32_t)KB * MOE_XSW * 4, rs4 = block_major ? 4 : (uint32_t)KB * 4;
-  s.bs = block_major ? (uint32_t)n_rows * MOE_XSW * 4 : MOE_XSW * 4;
-  s.bs4 = block_major ? (uint32_t)n_rows * 4 : 4;
-  s.xo = xr >= 0 ? (uint32_t)xr * rs + (uint32_t)(lane >> 5) * 16 : MOE_OOB;
-  s.so = xr >= 0 ? (uint32_t)xr * rs4 + (uint32_t)(lane >> 5) * s.bs4 : MOE_OOB;
+  s.src = src;
+  s.bytes = (uint32_t)rows * (uint32_t)NQ * (MOE_SQ_DW * 4);
+  s.wave = wave;
+  s.chunks = moe_nq4(NQ);
+#pragma unroll
+  for (int i = 0; i < MOE_SK_WDMA; i++) {
+    const int u = 64 * (wave + MOE_SK_WAVES * i) + lane;
+    const int q = u / (MOE_SK_ROWS * MOE_SQ_U4), v = u % (MOE_SK_ROWS * MOE_SQ_U4);
+    const int r = __shfl(row, v / MOE_SQ_U4);
+    s.vo[i] = r >= 0 ? ((uint32_t)r * (uint32_t)NQ + q) * (MOE_SQ_DW * 4) + (v % MOE_SQ_U4) * 16 : MOE_SK_OOB;
+  }
   return s;
 }
 
-// Chunk C of the staged rows into buf: wave w loads the blocks w*SW ..
-// w*SW + SW - 1 of the chunk (both halves; SW = blocks per wave) and the
-// scales of two blocks (waves below MOE_SK_STEPS/2): 2*SW + 1 loads or 2*SW.
-#define MOE_SK_SW (MOE_SK_STEPS / MOE_SK_WAVES)
-__device__ __forceinline__ void sdma_issue(const sdma &g, const gsrc &src, uint32_t *buf, int wave, int C) {
+// Chunk C into buf.  The quads past a row's end (NQ % 4 != 0) read on into the
+// next row, or past the buffer: the K loop does not use them.  A chunk past the
+// end issues its loads out of range, since the waits count them; its scalar
+// offset stays 0, as the bounds check compares the lane offset with the
+// buffer's size less the scalar offset.
+__device__ __forceinline__ void sdma_issue(const sdma &s, uint32_t *buf, int C) {
   typedef __attribute__((address_space(3))) void *lds_t;
+  const bool in = C < s.chunks;
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)s.src, 0, (int)s.bytes, MOE_RSRC_FLAGS);
+  const uint32_t so = in ? (uint32_t)C * (MOE_SK_CH * MOE_SQ_DW * 4) : 0u;
 #pragma unroll
-  for (int i = 0; i < MOE_SK_SW; i++) {
-    const int st = MOE_SK_SW * wave + i;
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(src.x, (lds_t)(buf + (st * 2 + h) * 64 * 4), 16, g.xo,
-                                               (MOE_SK_STEPS * C + st) * g.bs + h * 32, 0, 0);
+  for (int i = 0; i < MOE_SK_WDMA; i++) {
+    if (MOE_SK_WAVES * i + s.wave >= MOE_SK_DMA) break;  // uniform over the wave
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(buf + (s.wave + MOE_SK_WAVES * i) * 256), 16,
+                                             in ? s.vo[i] : MOE_SK_OOB, so, 0, 0);
   }
-  if (wave < MOE_SK_STEPS / 2)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.d, (lds_t)(buf + MOE_SK_SC_DW + 2 * wave * 32), 4, g.so,
-                                             (MOE_SK_STEPS * C + 2 * wave) * g.bs4, 0, 0);
 }
 
-// One block's A operand (the tokens' digits) of this lane, from a chunk buffer.
+// ---------------------------------------------------------------------------
+// A block pair (K step) of this lane's B operands: the digits (hi or lo by lane half) of its two blocks.
 struct skb {
-  u32x4_t lo, hi;
+  u32x4_t v[3];
 };
 
-__device__ __forceinline__ void load_skb_v(skb &b, const uint32_t *buf, int lane, int st) {
-  const u32x4_t *bl = reinterpret_cast<const u32x4_t *>(buf);
-  b.lo = bl[(st * 2 + 0) * 64 + lane];
-  b.hi = bl[(st * 2 + 1) * 64 + lane];
+__device__ __forceinline__ const u32x4_t *sk_units(const uint32_t *buf, int lane) {
+  return reinterpret_cast<const u32x4_t *>(buf) + (lane & 31) * MOE_SQ_U4;
 }
 
-// The d of this lane's result tokens 8*i + 4*gb + (0..3), i < NK, of block
-// st of a chunk buffer (NK = the groups of 8 tokens that the item holds).
-template <int NK>
-__device__ __forceinline__ void load_skd(f32x4_t (&dq)[NK], const uint32_t *buf, int lane, int st) {
-  const f32x4_t *s = reinterpret_cast<const f32x4_t *>(buf + MOE_SK_SC_DW + st * 32 + 4 * (lane >> 5));
+// Pair j of quad q of a chunk.
+__device__ __forceinline__ void load_skb(skb &b, const uint32_t *buf, int lane, int q, int j) {
+  const u32x4_t *p = sk_units(buf, lane) + 6 * (lane >> 5) + q * (MOE_SK_ROWS * MOE_SQ_U4) + 3 * j;
 #pragma unroll
-  for (int i = 0; i < NK; i++) dq[i] = s[2 * i];
+  for (int i = 0; i < 3; i++) b.v[i] = p[i];
 }
 
-// acc[4i + j] += dq[i][j] * r[4i + j] for the token groups i < NK.
-template <int NK>
-__device__ __forceinline__ void sk_scale(f32x16_t &acc, const f32x16_t &r, const f32x4_t (&dq)[NK]) {
+// d of the quad's 4 blocks for this lane's token.
+__device__ __forceinline__ f32x4_t load_skd(const uint32_t *buf, int lane, int q) {
+  return __builtin_bit_cast(f32x4_t, sk_units(buf, lane)[q * (MOE_SK_ROWS * MOE_SQ_U4) + 12]);
+}
+
+// Block J of the pair as the MFMA's fp6 operand (6 dwords).
+template <int J>
+__device__ __forceinline__ i32x8_t skb_block(const skb &b) {
+  i32x8_t r;
 #pragma unroll
-  for (int i = 0; i < NK; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[4 * i + j] = __builtin_fmaf(dq[i][j], r[4 * i + j], acc[4 * i + j]);
+  for (int i = 0; i < 6; i++) r[i] = (int)b.v[(6 * J + i) / 4][(6 * J + i) % 4];
+  r[6] = r[7] = 0;
+  return r;
 }
 
 // [x | x] and [y | y] from a register holding x in lanes 0-31, y in 32-63.
@@ -132,290 +261,278 @@ __device__ __forceinline__ void dup_halves1(uint32_t w, uint32_t &a0, uint32_t &
   a1 = p[1];
 }
 
-struct skring {
-  u32x4_t w[MOE_SK_RP];  // block pair P in slot P % MOE_SK_RP (pair P = blocks 2P, 2P+1 of the stream)
-  uint32_t sc[1][2], scn[1][2];  // exponent dwords of this 4-quad group and the next: lane (r, gb) holds
-                                 // block position 2j + gb
-  skb b;                         // the next step's A
+// Two weight streams of 32 rows (gate and up, or two tiles of down).
+struct skw {
+  const uint8_t *w[2];
+  uint32_t bytes, vo, so;  // of a 32-row tile; lane offsets of the data and of the exponents
+  int pairs, NG;
 };
 
-// Weight pair 8*G + SL of the stream (SL may reach into the next group).
+__device__ __forceinline__ skw make_skw(const uint8_t *w0, const uint8_t *w1, int NQ, int lane) {
+  skw p;
+  p.w[0] = w0;
+  p.w[1] = w1;
+  p.NG = moe_nq4(NQ);
+  p.pairs = 2 * NQ;
+  p.bytes = 2u * p.NG * MOE_REC_BYTES;
+  const aoff32 ao = make_aoff32(lane, p.NG);
+  p.vo = ao.v;
+  p.so = ao.s;
+  return p;
+}
+
+// Block pair S (past the end: no records and scalar offset 0, nothing read).
 template <int CPOL>
-__device__ __forceinline__ void load_w32g(u32x4_t &w, const wstream (&ws)[1], const aoff32 &ao, int G, int SL) {
-  const int q = SL >> 1, j = SL & 1;
-  w = __builtin_amdgcn_raw_buffer_load_b128(ws[0].rec, ao.v + j * 512, (G + (q >> 2)) * MOE_REC_BYTES + (q & 3) * 1024,
-                                            CPOL);
+__device__ __forceinline__ void load_skw(u32x4_t (&w)[2], const skw &p, int S) {
+  const bool in = S < p.pairs;
+  const int q = S >> 1, so = in ? (q >> 2) * (int)MOE_REC_BYTES + (q & 3) * 1024 : 0;
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc((void *)p.w[s], 0, in ? (int)p.bytes : 0, MOE_RSRC_FLAGS);
+    w[s] = __builtin_amdgcn_raw_buffer_load_b128(r, p.vo + (S & 1) * 512, so, CPOL);
+  }
 }
 
-// VMEM loads a wave issues after its chunk-C staging loads up to the end of
-// chunk C: the next group's 2 exponent dwords, and the weight pairs issued
-// during the chunk's 4 pairs (3 ahead).
-template <int C, int NQ>
-__host__ __device__ constexpr int sdma_after() {
-  int n = 0;
-  for (int q = MOE_SK_CH * C; q < MOE_SK_CH * (C + 1); q++) {
-    if ((q & 3) == 0 && q / 4 + 1 < NQ / 4) n += 2;  // the next group's exponent dwords
+// Exponent dwords of group G: lane (r, g) holds block position 2j + g, byte q = quad q.
+__device__ __forceinline__ void load_sksc(uint32_t (&sc)[2][2], const skw &p, int G) {
+  const bool in = G < p.NG;
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc((void *)p.w[s], 0, in ? (int)p.bytes : 0, MOE_RSRC_FLAGS);
+#pragma unroll
     for (int j = 0; j < 2; j++)
-      if (2 * q + j + MOE_SK_RP - 1 < 2 * NQ) n++;  // weight pairs
+      sc[s][j] = __builtin_amdgcn_raw_buffer_load_b32(r, p.so + j * 128, in ? G * (int)MOE_REC_BYTES : 0, 0);
   }
-  return n;
 }
 
-// One MFMA step (block st of the chunk buffer cbuf), software-pipelined by
-// one step: the MFMA goes out into its own result registers, then the next
-// step's digits are read from LDS (nbuf, block nst), then the previous
-// step's result is scaled by its tokens' d into acc while this MFMA runs,
-// then this step's d is read for the next step's scaling.  The scaled sums
-// reach acc in block order; sk_loop adds the last step's after the loop.
-// w4, sw: the weight block (both lane halves) and its exponent dword (byte
-// SEL); sa: the digits' scale (2^4 hi, 2^0 lo).
-template <int SEL, int NK>
-__device__ __forceinline__ void sk_step(const u32x4_t &w4, uint32_t sw, skb &b, const uint32_t *cbuf, int st,
-                                        const uint32_t *nbuf, int nst, bool next, int lane, int sa, f32x16_t &acc,
-                                        f32x16_t &rp, f32x4_t (&dq)[NK]) {
-  const i32x8_t wv = {(int)w4.x, (int)w4.y, (int)w4.z, (int)w4.w, 0, 0, 0, 0};
-  const i32x8_t xv = {(int)b.lo.x, (int)b.lo.y, (int)b.lo.z, (int)b.lo.w,
-                      (int)b.hi.x, (int)b.hi.y, (int)b.hi.z, (int)b.hi.w};
-  f32x16_t z;
+#define MOE_SK_RP 4  // weight ring, in block pairs: 3 ahead, 6 KiB in flight per wave (7 ahead measured the same)
+
+struct skring {
+  u32x4_t w[MOE_SK_RP][2];
+  uint32_t e[2][4];    // this group's exponents by block position, the same in both lane halves
+  uint32_t scn[2][2];  // the next group's, as loaded
+  skb b[2];            // B of this pair and the next
+  f32x4_t d[2];        // d of this quad and the next
+  f32x16_t r[2];       // the block sums last multiplied
+  float du;            // d of stream 1's pending block
+};
+
+// One block against both streams.  Stream 0's MFMA runs while stream 1's last
+// result is scaled, and the other way round; stream 1's result stays pending.
+template <int SEL, int J, int JD>
+__device__ __forceinline__ void sk_block(skring &g, const u32x4_t &w0, const u32x4_t &w1, const skb &b, float d, int sb,
+                                         f32x16_t (&acc)[2]) {
+  const i32x8_t x = skb_block<J>(b);
+  const i32x8_t a0 = {(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w, 0, 0, 0, 0};
+  const i32x8_t a1 = {(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w, 0, 0, 0, 0};
+  const f32x16_t z = {};
+  g.r[0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, x, z, 4, 2, SEL, (int)g.e[0][JD], 0, sb);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int e = 0; e < 16; e++) z[e] = 0.0f;
-  const f32x16_t r = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(xv, wv, z, 0, 4, 0, sa, SEL, (int)sw);
+  for (int i = 0; i < 16; i++) acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
+  asm volatile("" : "+v"(acc[1]));
   __builtin_amdgcn_sched_barrier(0);
-  if (next) load_skb_v(b, nbuf, lane, nst);
+  g.r[1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, x, z, 4, 2, SEL, (int)g.e[1][JD], 0, sb);
   __builtin_amdgcn_sched_barrier(0);
-  sk_scale<NK>(acc, rp, dq);
-  asm volatile("" : "+v"(acc));
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[0][i] = __builtin_fmaf(d, g.r[0][i], acc[0][i]);
+  asm volatile("" : "+v"(acc[0]));
+  g.du = d;
   __builtin_amdgcn_sched_barrier(0);
-  rp = r;
-  load_skd<NK>(dq, cbuf, lane, st);
 }
 
-// Quad QL (0..3) of the 4-quad group G of the K loop; the group's chunks
-// 2G and 2G + 1 are in buffers 0 and 1.  Every group but the last (LAST: G
-// == NQ/4 - 1, known at compile time) runs the same code from a rolled loop:
-// it stages the chunk after each of its chunks, loads the next group's
-// exponents, keeps the weight ring 3 pairs ahead, and each chunk end waits
-// for exactly the next chunk's staging (a constant count of younger loads).
-// Weights are loaded with cache policy CPOL.
-template <int QL, int NQ, int CPOL, int NK, bool LAST>
-__device__ __forceinline__ void sk_quad(skring &r, const wstream (&ws)[1], const aoff32 &ao, const gsrc &src,
-                                        const sdma &g, uint32_t *lds, int wave, int lane, int sa, int G,
-                                        f32x16_t &acc, f32x16_t &rp, f32x4_t (&dq)[NK]) {
-  constexpr int NG = NQ / 4, RP = MOE_SK_RP, c = QL >> 1, qc = QL & 1;  // chunk of the group, quad of the chunk
-  static_assert(MOE_SK_CH == 2 && RP == 4, "a group is two chunks of two quads, the ring 4 pairs");
-  constexpr bool next_chunk = !LAST || c == 0;  // chunk 2G + c + 1 exists
-  const uint32_t *buf = lds + c * MOE_SK_BUF_DW;
-  if constexpr (qc == 0 && next_chunk) {  // the next chunk's staging, straight into the other buffer
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    sdma_issue(g, src, lds + (c ^ 1) * MOE_SK_BUF_DW, wave, 2 * G + c + 1);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  if constexpr (QL == 0 && !LAST) load_sc32<1>(r.scn, ws, ao, G + 1);
-  uint32_t e[4];  // this quad's group exponents, every lane block position 0..3
-  dup_halves1(r.sc[0][0], e[0], e[1]);
-  dup_halves1(r.sc[0][1], e[2], e[3]);
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int SL = 2 * QL + j + RP - 1;  // the pair 3 ahead, from the group's first pair
-    if (!LAST || SL < 8) load_w32g<CPOL>(r.w[SL % RP], ws, ao, G, SL);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    u32x4_t w0, w1;
-    dup_halves(r.w[(2 * QL + j) % RP], w0, w1);
-    const int st = 4 * qc + 2 * j;  // block of the chunk
-    sk_step<QL, NK>(w0, e[2 * j], r.b, buf, st, buf, st + 1, true, lane, sa, acc, rp, dq);
-    const bool last_of_chunk = qc == 1 && j == 1;
-    sk_step<QL, NK>(w1, e[2 * j + 1], r.b, buf, st + 1, buf, st + 2, !last_of_chunk, lane, sa, acc, rp, dq);
-  }
-  if constexpr (qc == 1 && next_chunk) {
-    // the next chunk has landed in LDS (this wave's loads, then everyone's)
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(sdma_after<(LAST ? 2 * (NG - 1) : 0) + c, NQ>()));
+// Pair SG of group G (its chunk in buffer cur).  The barrier of a chunk sits
+// before its last pair: every wave has then read its operands of that pair, so
+// the buffer is free for the chunk MOE_SK_NBUF ahead, and the next chunk,
+// loaded MOE_SK_NBUF - 1 chunks ago, is visible to all.
+template <int CPOL, int SG>
+__device__ __forceinline__ void sk_pair(skring &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane, int sb,
+                                        int G, f32x16_t (&acc)[2]) {
+  static_assert(MOE_SK_CH == 4 && 8 % MOE_SK_RP == 0 && MOE_SK_NBUF == 2, "a chunk is one group; two buffers");
+  load_skw<CPOL>(g.w[(SG + MOE_SK_RP - 1) % MOE_SK_RP], w, G * 8 + SG + MOE_SK_RP - 1);
+  if constexpr (SG == 0) load_sksc(g.scn, w, G + 1);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (SG == 7) {
+    // younger than the next chunk's staging: a chunk's weights (8 pairs of two loads) and exponents
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(8 * 2 + 4));
     lds_barrier();
-    load_skb_v(r.b, lds + (c ^ 1) * MOE_SK_BUF_DW, lane, 0);
+    sdma_issue(st, lds + cur * MOE_SK_BUF_DW, G + MOE_SK_NBUF);
+    cur ^= 1;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-template <int NQ, int CPOL, int NK, bool LAST>
-__device__ __forceinline__ void sk_group(skring &r, const wstream (&ws)[1], const aoff32 &ao, const gsrc &src,
-                                         const sdma &g, uint32_t *lds, int wave, int lane, int sa, int G,
-                                         f32x16_t &acc, f32x16_t &rp, f32x4_t (&dq)[NK]) {
-  sk_quad<0, NQ, CPOL, NK, LAST>(r, ws, ao, src, g, lds, wave, lane, sa, G, acc, rp, dq);
-  sk_quad<1, NQ, CPOL, NK, LAST>(r, ws, ao, src, g, lds, wave, lane, sa, G, acc, rp, dq);
-  sk_quad<2, NQ, CPOL, NK, LAST>(r, ws, ao, src, g, lds, wave, lane, sa, G, acc, rp, dq);
-  sk_quad<3, NQ, CPOL, NK, LAST>(r, ws, ao, src, g, lds, wave, lane, sa, G, acc, rp, dq);
-  if constexpr (!LAST) {
-    r.sc[0][0] = r.scn[0][0];
-    r.sc[0][1] = r.scn[0][1];
-  }
-}
-
-// The K loop of one wave: its 32-row weight tile over NQ quads against the
-// 32 staged tokens (xr: the staged row of token lane&31, < 0 absent).  acc:
-// lane r + 32*gb, element 4i + j = weight row r, token 8i + 4gb + j (left 0
-// for the groups i >= NK, which hold no token of the item).  CPOL: the
-// weights' cache policy (non-temporal where no other item reads them).
-template <int NQ, int CPOL, int NK>
-__device__ __forceinline__ void sk_loop(const wstream (&ws)[1], const aoff32 &ao, const gsrc &src, int xr, int KB,
-                                        bool block_major, int n_rows, uint32_t *lds, int wave, int lane,
-                                        f32x16_t &acc) {
-  static_assert(NQ % 4 == 0 && NQ >= 8, "whole groups, at least two");
-  const sdma g = make_sdma(lane, xr, KB, block_major, n_rows);
-  skring r;
-  sdma_issue(g, src, lds, wave, 0);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  load_sc32<1>(r.sc, ws, ao, 0);
+  const uint32_t *buf = lds + cur * MOE_SK_BUF_DW;
+  load_skb(g.b[(SG + 1) & 1], buf, lane, ((SG + 1) & 7) >> 1, (SG + 1) & 1);
+  if constexpr (SG & 1) g.d[((SG >> 1) + 1) & 1] = load_skd(buf, lane, ((SG + 1) & 7) >> 1);
+  u32x4_t a[2][2];
 #pragma unroll
-  for (int i = 0; i + 1 < MOE_SK_RP; i++) load_w32g<CPOL>(r.w[i], ws, ao, 0, i);
+  for (int s = 0; s < 2; s++) dup_halves(g.w[SG % MOE_SK_RP][s], a[s][0], a[s][1]);
+  __builtin_amdgcn_sched_barrier(0);
+  const f32x4_t d = g.d[(SG >> 1) & 1];
+  constexpr int j = SG & 1;
+  sk_block<(SG >> 1), 0, 2 * j>(g, a[0][0], a[1][0], g.b[j], d[2 * j], sb, acc);
+  sk_block<(SG >> 1), 1, 2 * j + 1>(g, a[0][1], a[1][1], g.b[j], d[2 * j + 1], sb, acc);
+}
+
+template <int CPOL, int SG>
+__device__ __forceinline__ void sk_group(skring &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane, int sb,
+                                         int G, int quads, f32x16_t (&acc)[2]) {
+  if constexpr (SG < 8) {
+    if (quads <= (SG >> 1)) return;  // the last group of a K that is no multiple of 512
+    sk_pair<CPOL, SG>(g, w, st, lds, cur, lane, sb, G, acc);
+    sk_group<CPOL, SG + 1>(g, w, st, lds, cur, lane, sb, G, quads, acc);
+  }
+}
+
+// The K loop of one wave: its two weight streams over NQ quads against the
+// staged tokens.  acc[s]: lane n + 32*g, element 4i + j = row 8i + 4g + j of
+// stream s, token n, summed block by block; GROUPED: the sums of 4-quad groups
+// added up instead.  CPOL: the weights' cache policy.
+template <int CPOL, bool GROUPED>
+__device__ __forceinline__ void sk_loop(const skw &w, const sdma &st, int NQ, uint32_t *lds, int lane, f32x16_t (&acc)[2]) {
+  skring g;
+  uint32_t sc[2][2];
+  f32x16_t tot[2];
+#pragma unroll
+  for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  // chunk 0 has landed (2 exponent dwords and the first weight pairs went out after it)
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 + MOE_SK_RP - 1));
+  load_sksc(sc, w, 0);
+#pragma unroll
+  for (int i = 0; i + 1 < MOE_SK_RP; i++) load_skw<CPOL>(g.w[i], w, i);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  // chunk 0 has landed (the second chunk, the exponents and the first weights went out after it)
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1 + 4 + 2 * (MOE_SK_RP - 1)));
   lds_barrier();
-  f32x16_t rp;
-  f32x4_t dq[NK];
+  int cur = 0;
+  load_skb(g.b[0], lds, lane, 0, 0);
+  g.d[0] = load_skd(lds, lane, 0);
 #pragma unroll
-  for (int e = 0; e < 16; e++) {
-    acc[e] = 0.0f;
-    rp[e] = 0.0f;  // the first step scales a zero result: acc stays +0
+  for (int s = 0; s < 2; s++) {
+    acc[s] = f32x16_t{};
+    tot[s] = f32x16_t{};
   }
+  g.r[1] = f32x16_t{};  // the first block scales a zero result: acc stays +0
+  g.du = 0.0f;
+  const int sb = (lane >> 5) ? 130 : 134;  // lo digits x 2^3 (fp6 codes are eighths), hi digits x 2^7
+  auto group = [&](int G, int quads) {
 #pragma unroll
-  for (int i = 0; i < NK; i++) dq[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  load_skb_v(r.b, lds, lane, 0);
-  const int sa = (lane >> 5) ? 127 : 131;
+    for (int s = 0; s < 2; s++) {
+      dup_halves1(sc[s][0], g.e[s][0], g.e[s][1]);
+      dup_halves1(sc[s][1], g.e[s][2], g.e[s][3]);
+    }
+    sk_group<CPOL, 0>(g, w, st, lds, cur, lane, sb, G, quads, acc);
+    if constexpr (GROUPED) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
+        tot[0][i] += acc[0][i];
+        tot[1][i] += acc[1][i];
+        acc[0][i] = acc[1][i] = g.r[1][i] = 0.0f;
+      }
+    }
+  };
+  int G = 0;
+  // whole groups in a loop of their own: with the last group's exits in it,
+  // the waits at its head would cover the loads in flight
 #pragma unroll 1
-  for (int G = 0; G + 1 < NQ / 4; G++) sk_group<NQ, CPOL, NK, false>(r, ws, ao, src, g, lds, wave, lane, sa, G, acc, rp, dq);
-  sk_group<NQ, CPOL, NK, true>(r, ws, ao, src, g, lds, wave, lane, sa, NQ / 4 - 1, acc, rp, dq);
-  sk_scale<NK>(acc, rp, dq);  // the last step's scaled sums
-}
-
-// sk_loop for the item's nk = ceil(rows / 8) groups of 8 tokens and weight
-// cache policy (split: the default policy, else non-temporal).
-template <int NQ>
-__device__ __forceinline__ void sk_loop_any(const wstream (&ws)[1], const aoff32 &ao, const gsrc &src, int xr,
-                                            int KB, bool block_major, int n_rows, uint32_t *lds, int wave, int lane,
-                                            int nk, bool split, f32x16_t &acc) {
-#define MOE_SK_LOOP(CP, K) sk_loop<NQ, CP, K>(ws, ao, src, xr, KB, block_major, n_rows, lds, wave, lane, acc)
-  if (split) {
-    switch (nk) {
-      case 1: MOE_SK_LOOP(0, 1); break;
-      case 2: MOE_SK_LOOP(0, 2); break;
-      case 3: MOE_SK_LOOP(0, 3); break;
-      default: MOE_SK_LOOP(0, 4); break;
-    }
-  } else {
-    switch (nk) {
-      case 1: MOE_SK_LOOP(MOE_CPOL_NT, 1); break;
-      case 2: MOE_SK_LOOP(MOE_CPOL_NT, 2); break;
-      case 3: MOE_SK_LOOP(MOE_CPOL_NT, 3); break;
-      default: MOE_SK_LOOP(MOE_CPOL_NT, 4); break;
-    }
+  for (; 4 * G + 4 <= NQ; G++) {
+    group(G, 4);
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) sc[s][j] = g.scn[s][j];
   }
-#undef MOE_SK_LOOP
+  if (4 * G < NQ) group(G, NQ - 4 * G);
+  if constexpr (GROUPED) {
+    acc[0] = tot[0];
+    acc[1] = tot[1];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
+  }
 }
 
-// gate/up -> clamp -> SwiGLU -> Q8_0(h) on items of up to 32 rows.  One
-// workgroup of 8 waves per (4 units of F, item): wave w streams the gate
-// (w < 4) or up tile of unit 4*blockIdx.x + w%4 over all of K against the
-// item's tokens; gate and up meet in LDS.  grid (F/128, item capacity), 512
-// threads, LDS MOE_SK_LDS_BYTES.  Requires H == 128 * NQ, NQ % 4 == 0,
-// (F/32) % 4 == 0.
-template <int NQ>
-__global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
-void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_u, const uint32_t *__restrict__ xq,
-                  const float *__restrict__ xd, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
-                  int k, int T, int F, int H, float clamp, uint32_t *__restrict__ hs, float *__restrict__ hd,
-                  float *__restrict__ htap) {
+// gate/up -> clamp -> SwiGLU -> Q8_0(h) on items of up to 32 rows: one
+// workgroup of 4 waves per (quad of F, item), wave = the gate and the up tile
+// of one 32-row unit over all of K.  h row-major in quad records.  grid (F/128,
+// item capacity), 256 threads, LDS MOE_SK_LDS_BYTES.
+template <bool GROUPED>
+__global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_u, const uint32_t *__restrict__ xs,
+                  const int32_t *__restrict__ items, const int32_t *__restrict__ perm, int k, int T, int F, int H,
+                  float clamp, uint32_t *__restrict__ hs, float *__restrict__ htap) {
   extern __shared__ __align__(16) uint32_t lds[];
   if ((int)blockIdx.y >= items[0]) return;
   const int4 it = item_of(items, blockIdx.y);
-  constexpr int NQ4 = NQ / 4, KB = NQ * 4;
-  const int tiles = F / MOE_TILE;
+  const int NQ = H / 128, NG = moe_nq4(NQ), tiles = F / MOE_TILE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int P = T * k, NR = P + T, row0 = it.y, nt = it.z;
+  const int P = T * k, row0 = it.y, nt = it.z;
   const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
-  const int u = 4 * blockIdx.x + (wave & 3);
-  const wstream ws[1] = {make_wstream32(wave >= 4 ? w_u : w_g, (size_t)it.x * tiles + 2 * u, NQ4)};
-  const aoff32 ao = make_aoff32(lane, NQ4);
-  const gsrc src = make_gsrc(xq, xd, T, KB);
-  const int n = lane & 31, gb = lane >> 5;
-  const int xr = n < nt ? (shared ? row0 + n - P : perm[row0 + n] / k) : -1;
-  const int nk = __builtin_amdgcn_readfirstlane((nt + 7) >> 3);
-  f32x16_t acc;
+  const int u = MOE_SK_WAVES * blockIdx.x + wave, n = lane & 31, gb = lane >> 5;
+  const size_t rec = ((size_t)it.x * tiles + 2 * u) * NG * MOE_REC_BYTES;
+  const bool live = n < nt;
+  const int xr = live ? (shared ? row0 + n - P : perm[row0 + n] / k) : -1;
+  const sdma st = make_sdma(xs, T, NQ, xr, lane, wave);
+  const skw w = make_skw(w_g + rec, w_u + rec, NQ, lane);
+  f32x16_t acc[2];
   // an expert of one item reads its tiles once: non-temporal, as in decode;
   // the items of a larger expert share them through L2
-  sk_loop_any<NQ>(ws, ao, src, xr, KB, false, T, lds, wave, lane, nk, (it.w & MOE_ITEM_SPLIT) != 0, acc);
-  lds_barrier();  // every wave is done with the chunk buffers
-  float *red = reinterpret_cast<float *>(lds);  // [unit][gate/up][token][row]
+  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED>(w, st, NQ, lds, lane, acc);
+  else sk_loop<MOE_CPOL_NT, GROUPED>(w, st, NQ, lds, lane, acc);
+  float h[16];
 #pragma unroll
-  for (int e = 0; e < 16; e++)
-    red[(((wave & 3) * 2 + (wave >> 2)) * 32 + 8 * (e >> 2) + 4 * gb + (e & 3)) * MOE_UNIT + n] = acc[e];
-  __syncthreads();
-  // (unit, token) c = 16*round + 2*wave + half-wave: unit c / 32, token c % 32
+  for (int i = 0; i < 16; i++) h[i] = live ? swiglu(acc[0][i], acc[1][i], clamp) : 0.0f;
+  const int hrow = row0 + (live ? n : 0);
+  h_quad_store(h, live, hs + ((size_t)hrow * (F / 128) + blockIdx.x) * MOE_SQ_DW, wave, lane);
+  if (htap && live) {
 #pragma unroll
-  for (int round = 0; round < 8; round++) {
-    if ((round & 1) && nt <= 16) continue;  // odd rounds hold tokens 16..31 (uniform over the workgroup)
-    const int c = 16 * round + 2 * wave + (lane >> 5);
-    const int ul = c >> 5, t = c & 31, j = lane & 31;
-    const bool live = t < nt;
-    const float gsum = red[((ul * 2 + 0) * 32 + t) * MOE_UNIT + j];
-    const float usum = red[((ul * 2 + 1) * 32 + t) * MOE_UNIT + j];
-    const float h = live ? swiglu(gsum, usum, clamp) : 0.0f;
-    const int hrow = row0 + (live ? t : 0), uu = 4 * blockIdx.x + ul;
-    // h block-major ([unit of F][grouped row]): an item's rows of one unit are adjacent
-    h_unit_store(h, live, hs + ((size_t)uu * NR + hrow) * MOE_XSW, hd + (size_t)uu * NR + hrow, lane);
-    if (htap && live) htap[(size_t)hrow * F + (size_t)uu * MOE_UNIT + j] = h;
+    for (int i = 0; i < 16; i++)
+      htap[(size_t)hrow * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
   }
 }
 
-// down x router weight on items of up to 32 rows: one workgroup of 8 waves
-// per (256 rows of H, item), wave = one 32-row tile of H over all of F
-// against the item's h rows; y[row] = the tile's rows x the pair's router
-// weight (the shared expert's rows unweighted).  grid (H/256, item
-// capacity), 512 threads, LDS MOE_SK_DN_LDS_BYTES.  Requires F == 128 * NQ,
-// NQ % 4 == 0, H % 256 == 0.
-template <int NQ>
-__global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
-void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, const float *__restrict__ hd,
-               int n_rows, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
-               const float *__restrict__ wts, int F, int H, float *__restrict__ y) {
+// down x router weight on items of up to 32 rows: one workgroup of 4 waves
+// per (256 rows of H, item), wave = two 32-row tiles over all of F against the
+// item's h rows; y[row] = the tiles' rows x the pair's router weight (the
+// shared expert's rows unweighted).  grid (ceil(H/256), item capacity), 256
+// threads, LDS MOE_SK_LDS_BYTES.
+template <bool GROUPED>
+__global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, int n_rows,
+               const int32_t *__restrict__ items, const int32_t *__restrict__ perm, const float *__restrict__ wts, int F,
+               int H, float *__restrict__ y) {
   extern __shared__ __align__(16) uint32_t lds[];
   if ((int)blockIdx.y >= items[0]) return;
   const int4 it = item_of(items, blockIdx.y);
-  constexpr int NQ4 = NQ / 4, KB = NQ * 4;
-  const int tiles = H / MOE_TILE;
+  const int NQ = F / 128, NG = moe_nq4(NQ), tiles = H / MOE_TILE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = it.y, nt = it.z;
   const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
-  const int t32 = blockIdx.x * MOE_SK_WAVES + wave;  // 32-row tile of H
-  const wstream ws[1] = {make_wstream32(w_d, (size_t)it.x * tiles + 2 * t32, NQ4)};
-  const aoff32 ao = make_aoff32(lane, NQ4);
-  const gsrc src = make_gsrc(hs, hd, n_rows, KB);
   const int n = lane & 31, gb = lane >> 5;
-  const int nk = __builtin_amdgcn_readfirstlane((nt + 7) >> 3);
-  f32x16_t acc;
-  const int xr = n < nt ? row0 + n : -1;
-  sk_loop_any<NQ>(ws, ao, src, xr, KB, true, n_rows, lds, wave, lane, nk, (it.w & MOE_ITEM_SPLIT) != 0, acc);
-  // the router weight of token n, then of this lane's result tokens through
-  // the wave's own 32 floats past the chunk buffers
-  float *wtl = reinterpret_cast<float *>(lds + 2 * MOE_SK_BUF_DW) + 32 * wave;
-  const float wt = (n < nt && !shared) ? wts[perm[row0 + n]] : 1.0f;
-  if (gb == 0) wtl[n] = wt;
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  const f32x4_t *wq = reinterpret_cast<const f32x4_t *>(wtl + 4 * gb);
-  float *dst = y + (size_t)row0 * H + (size_t)t32 * 32 + n;
+  const bool live = n < nt;
+  const int t64 = MOE_SK_WAVES * blockIdx.x + wave;  // 64 rows of H
+  const bool rows = t64 < H / 64;                    // H % 256 == 128: the last workgroup's upper waves only stage
+  const uint8_t *w0 = w_d + ((size_t)it.x * tiles + 4 * (rows ? t64 : 0)) * NG * MOE_REC_BYTES;
+  const sdma st = make_sdma(hs, n_rows, NQ, live ? row0 + n : -1, lane, wave);
+  const skw w = make_skw(w0, w0 + (size_t)2 * NG * MOE_REC_BYTES, NQ, lane);
+  f32x16_t acc[2];
+  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED>(w, st, NQ, lds, lane, acc);
+  else sk_loop<MOE_CPOL_NT, GROUPED>(w, st, NQ, lds, lane, acc);
+  if (!live || !rows) return;
+  const float wt = shared ? 1.0f : wts[perm[row0 + n]];
+  float *dst = y + (size_t)(row0 + n) * H + (size_t)t64 * 64 + 4 * gb;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (i >= nk) break;
-    const f32x4_t w4 = wq[2 * i];
+  for (int s = 0; s < 2; s++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int t = 8 * i + 4 * gb + j;
-      if (t < nt) dst[(size_t)t * H] = shared ? acc[4 * i + j] : __fmul_rn(acc[4 * i + j], w4[j]);
+    for (int i = 0; i < 4; i++) {
+      f32x4_t v;
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = shared ? acc[s][4 * i + j] : __fmul_rn(acc[s][4 * i + j], wt);
+      *reinterpret_cast<f32x4_t *>(dst + 32 * s + 8 * i) = v;
     }
-  }
 }

@@ -53,10 +53,12 @@ struct dev_layer {
 struct work_bufs {
   // sized for (T, H, F, E, k)
   int T = 0, H = 0, F = 0, E = 0, k = 0;
-  uint32_t *hq = nullptr; float *hd = nullptr;     // staged h: [P+T][F/32][16] dwords, [P+T][F/32]
+  // staged h: [P+T][F/32][16] dwords and [P+T][F/32] scales, or in hq alone the
+  // stacked kernels' quad records, [P+T][F/128][52] dwords
+  uint32_t *hq = nullptr; float *hd = nullptr;
   float *htap = nullptr;                           // [P+T][F]
   float *y = nullptr;                              // [P+T][H]
-  uint32_t *xq = nullptr; float *xd = nullptr;     // staged x of the grouped chain: [T][H/32][16] dwords, [T][H/32]
+  uint32_t *xq = nullptr; float *xd = nullptr;     // staged x of the grouped chain, likewise
   // balanced decode gate/up: per-task row sums [16 slots][F/32][4][16] and
   // per-unit tickets (zeroed here once, left at zero by every launch)
   float *part = nullptr; int *tick = nullptr;
@@ -403,26 +405,6 @@ extern "C" moe_status moe_ctx_create(int device, uint64_t budget_bytes, moe_ctx 
 
   c->budget = (inject & 2) ? 0 : budget_bytes;
   c->inject = inject;
-  // the two-octet down kernels stage more than 64 KiB of LDS per workgroup
-  const std::pair<const void *, int> big_lds[] = {{(const void *)k_down_ol2<6>, 6 * 4}};
-  for (const auto &kb : big_lds)
-    if (hipFuncSetAttribute(kb.first, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(2 * octet_lds_bytes_z(kb.second))) != hipSuccess) {
-      delete c;
-      return MOE_ERR_NO_DEVICE;
-    }
-  // and the stacked-digit kernels (two 17 KiB chunk buffers, 34 KiB, and
-  // down's router weights; set for uniformity)
-  const std::pair<const void *, int> sk_kernels[] = {
-      {(const void *)k_gate_up_sk<56>, MOE_SK_LDS_BYTES},   {(const void *)k_gate_up_sk<48>, MOE_SK_LDS_BYTES},
-      {(const void *)k_gate_up_sk<32>, MOE_SK_LDS_BYTES},   {(const void *)k_gate_up_sk<16>, MOE_SK_LDS_BYTES},
-      {(const void *)k_down_sk<24>, MOE_SK_DN_LDS_BYTES}, {(const void *)k_down_sk<16>, MOE_SK_DN_LDS_BYTES},
-      {(const void *)k_down_sk<12>, MOE_SK_DN_LDS_BYTES}, {(const void *)k_down_sk<8>, MOE_SK_DN_LDS_BYTES}};
-  for (const auto &kf : sk_kernels)
-    if (hipFuncSetAttribute(kf.first, hipFuncAttributeMaxDynamicSharedMemorySize, kf.second) != hipSuccess) {
-      delete c;
-      return MOE_ERR_NO_DEVICE;
-    }
   noalloc_setup(c);
   *out = c;
   return MOE_OK;
@@ -807,11 +789,11 @@ extern "C" moe_status moe_group(moe_ctx *c, const int32_t *ids, int T, int k, in
     if ((long)T * k <= MOE_GF_PAIRS)
       hipLaunchKernelGGL(k_group_few, dim3(1), dim3(256), 0, (hipStream_t)stream, ids, T * k, E, T, 0, 1,
                          counts, offsets, perm, inv, (int32_t *)nullptr, (const float *)nullptr, 0,
-                         (uint32_t *)nullptr, (float *)nullptr, 0, (int32_t *)nullptr);
+                         (uint32_t *)nullptr, (float *)nullptr, 0);
     else
       hipLaunchKernelGGL(k_group, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, T * k, E, T, 0, 1, counts,
                          offsets, perm, inv, (int32_t *)nullptr, (const float *)nullptr, 0, (uint32_t *)nullptr,
-                         (float *)nullptr, 0, (int32_t *)nullptr);
+                         (float *)nullptr, 0);
   }
   HIPC(c, hipGetLastError());
   return MOE_OK;
@@ -890,7 +872,8 @@ static moe_status forward_decode(moe_ctx *c, dev_layer &L, work_bufs &s, const f
 
 // The grouped chain runs token pairs on the 16x16x128 MFMA for T <= 4
 // (items of at most 4 rows: NPMAX = 2 pairs), token octets on the 32x32x64
-// MFMA above that (items of at most 8 rows).
+// MFMA above that (items of at most 8 rows), and the stacked kernels on items
+// of up to 32 rows where the batch averages 2 pairs per expert or more.
 static bool use_octets(int T) { return T > 4; }
 
 static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const float *x, const int32_t *ids,
@@ -903,24 +886,16 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     return fail(c, MOE_ERR_UNSUPPORTED, "grouped: more than %d pairs or %d experts", MOE_GROUP_MAX_PAIRS,
                 MOE_GROUP_MAX_E);
   const bool oct = use_octets(T);
-  const int BT = oct ? 8 : 4;
+  const bool sk = oct && P >= 2 * E;
+  const int BT = sk ? MOE_SK_ROWS : oct ? 8 : 4;
   // a few tokens (the pairs path): down per 16-row tile of H with the slot
   // combine in the same launch (k_down_few)
   const bool few = !oct && T <= MOE_DF_TMAX && k + 1 <= MOE_DF_SMAX && H % MOE_DF_ROWS == 0;
+  // the stacked kernels add their block sums one by one on the shapes that
+  // always did (results keep their bits), else in groups (a smaller error)
+  const bool in_order = (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
+                        (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24);
   int32_t *counts = s.grp, *offsets = counts + E, *perm = offsets + E + 1, *inv = perm + P, *items = inv + P;
-  // where the shape has an instance and the batch averages 2 pairs per
-  // expert or more, gate/up and down run on a second item list with B staged
-  // in LDS: items of up to 32 rows on the stacked-digit kernels
-  // (k_gate_up_sk, H = 128 * {16, 32, 48, 56}; k_down_sk, F = 128 * {8, 12,
-  // 16, 24}), else items of up to 16 rows on the octet kernels (k_gate_up_ol /
-  // k_down_ol2, H = 128 * {16, 32, 56}); below 2 pairs per expert most items
-  // hold one octet and the 8-row list with B from global memory is used
-  int32_t *items16 = items + group_list_words(T, k, E);
-  const bool dense = oct && P >= 2 * E && (F / MOE_UNIT) % 4 == 0;
-  const bool sk = dense && (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
-                  (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24) && H % 256 == 0;
-  const bool o2 = sk || (dense && (H == 128 * 56 || H == 128 * 32 || H == 128 * 16));
-  const int BT2 = sk ? 32 : 16;
   float *htap = c->taps ? s.htap : nullptr;
   const int n_xblocks = T * (H / MOE_QK);
   {
@@ -929,29 +904,22 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     if (P <= MOE_GF_PAIRS)
       hipLaunchKernelGGL(k_group_few, dim3(1 + ceil_div(n_xblocks, MOE_GF_QBLOCKS)), dim3(256), 0, st,
                          ids, P, E, T, shared, BT, (int32_t *)nullptr, (int32_t *)nullptr, perm, inv, items, x,
-                         n_xblocks, s.xq, s.xd, BT2, (o2 || sk) ? items16 : (int32_t *)nullptr);
+                         n_xblocks, s.xq, s.xd, sk ? 1 : 0);
     else
       hipLaunchKernelGGL(k_group, dim3(1 + ceil_div(n_xblocks, MOE_GROUP_QBLOCKS)), dim3(1024), 0, st, ids, P, E, T,
-                         shared, BT, counts, offsets, perm, inv, items, x, n_xblocks, s.xq, s.xd, BT2,
-                         (o2 || sk) ? items16 : (int32_t *)nullptr);
+                         shared, BT, counts, offsets, perm, inv, items, x, n_xblocks, s.xq, s.xd, sk ? 1 : 0);
   }
   const int cap = group_item_cap(T, k, E, BT);
   {
     prof_scope pg(c, K_GU_GROUPED, st, s.timed);
 #define MOE_GU_ARGS L.m[T_GATE].w, L.m[T_UP].w, s.xq, s.xd, items, perm, k, T, F, H, d.clamp, s.hq, s.hd, htap
-#define MOE_GU_ARGS16 L.m[T_GATE].w, L.m[T_UP].w, s.xq, s.xd, items16, perm, k, T, F, H, d.clamp, s.hq, s.hd, htap
-    const dim3 g16(F / (4 * MOE_UNIT), group_item_cap(T, k, E, BT2));  // 4 units of F per workgroup
-    if (sk && H == 128 * 56) hipLaunchKernelGGL(k_gate_up_sk<56>, g16, dim3(512), MOE_SK_LDS_BYTES, st, MOE_GU_ARGS16);
-    else if (sk && H == 128 * 48) hipLaunchKernelGGL(k_gate_up_sk<48>, g16, dim3(512), MOE_SK_LDS_BYTES, st, MOE_GU_ARGS16);
-    else if (sk && H == 128 * 32) hipLaunchKernelGGL(k_gate_up_sk<32>, g16, dim3(512), MOE_SK_LDS_BYTES, st, MOE_GU_ARGS16);
-    else if (sk && H == 128 * 16) hipLaunchKernelGGL(k_gate_up_sk<16>, g16, dim3(512), MOE_SK_LDS_BYTES, st, MOE_GU_ARGS16);
-    else if (o2 && H == 128 * 56) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gate_up_ol<56, 4>), g16, dim3(512), 0, st, MOE_GU_ARGS16);
-    else if (o2 && H == 128 * 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gate_up_ol<32, 4>), g16, dim3(512), 0, st, MOE_GU_ARGS16);
-    else if (o2 && H == 128 * 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gate_up_ol<16, 4>), g16, dim3(512), 0, st, MOE_GU_ARGS16);
+    if (sk)
+      hipLaunchKernelGGL(in_order ? k_gate_up_sk<false> : k_gate_up_sk<true>, dim3(F / 128, cap),
+                         dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st, L.m[T_GATE].w, L.m[T_UP].w, s.xq, items, perm, k,
+                         T, F, H, d.clamp, s.hq, htap);
     else if (oct) hipLaunchKernelGGL(k_gate_up_o, dim3(F / (2 * MOE_UNIT), cap), dim3(256), 0, st, MOE_GU_ARGS);
     else hipLaunchKernelGGL(k_gate_up_g<2>, dim3(F / MOE_UNIT, cap), dim3(256), 0, st, MOE_GU_ARGS);
 #undef MOE_GU_ARGS
-#undef MOE_GU_ARGS16
   }
   s.h_rows = htap ? (size_t)P + (shared ? T : 0) : 0;
   s.last_F = F;
@@ -959,19 +927,11 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     prof_scope pd(c, K_DOWN_GROUPED, st, s.timed);
 #define MOE_DN_ARGS L.m[T_DOWN].w, s.hq, s.hd, P + T, items, perm, wts, F, H, s.y
     const dim3 gdo(H / 128, cap);
-    const size_t lo = octet_lds_bytes(F / MOE_QK), lo2 = 2 * octet_lds_bytes_z(F / MOE_QK);
-    // two octets per wave on the 16-row items where that list exists and two
-    // workgroups' LDS (2 x 2 staged octets) fit a CU (F = 768; the stacked
-    // kernels take F = 1024, 1536, 2048 and 3072)
-    const dim3 gdo2(H / (32 * MOE_DOL2_WAVES), group_item_cap(T, k, E, BT2));
-    const bool dn2 = o2 && !sk && H % (32 * MOE_DOL2_WAVES) == 0;
-    const dim3 b2(64 * MOE_DOL2_WAVES);
-#define MOE_DN_ARGS16 L.m[T_DOWN].w, s.hq, s.hd, P + T, items16, perm, wts, F, H, s.y
-    if (sk && F == 128 * 16) hipLaunchKernelGGL(k_down_sk<16>, gdo2, b2, MOE_SK_DN_LDS_BYTES, st, MOE_DN_ARGS16);
-    else if (sk && F == 128 * 24) hipLaunchKernelGGL(k_down_sk<24>, gdo2, b2, MOE_SK_DN_LDS_BYTES, st, MOE_DN_ARGS16);
-    else if (sk && F == 128 * 12) hipLaunchKernelGGL(k_down_sk<12>, gdo2, b2, MOE_SK_DN_LDS_BYTES, st, MOE_DN_ARGS16);
-    else if (sk && F == 128 * 8) hipLaunchKernelGGL(k_down_sk<8>, gdo2, b2, MOE_SK_DN_LDS_BYTES, st, MOE_DN_ARGS16);
-    else if (dn2 && F == 128 * 6) hipLaunchKernelGGL(k_down_ol2<6>, gdo2, b2, lo2, st, MOE_DN_ARGS16);
+    const size_t lo = octet_lds_bytes(F / MOE_QK);
+    if (sk)
+      hipLaunchKernelGGL(in_order ? k_down_sk<false> : k_down_sk<true>,
+                         dim3(ceil_div(H, 64 * MOE_SK_WAVES), cap), dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st, L.m[T_DOWN].w, s.hq, P + T, items, perm, wts, F, H,
+                         s.y);
     else if (oct && F == 128 * 16) hipLaunchKernelGGL(k_down_ol<16>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
     else if (oct && F == 128 * 6) hipLaunchKernelGGL(k_down_ol<6>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
     else if (oct && F == 128 * 8) hipLaunchKernelGGL(k_down_ol<8>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
@@ -983,7 +943,6 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     else hipLaunchKernelGGL(k_down_g<2>, dim3(ceil_div(H / (2 * MOE_TILE), MOE_DG_WAVES), cap),
                             dim3(64 * MOE_DG_WAVES), 0, st, MOE_DN_ARGS);
 #undef MOE_DN_ARGS
-#undef MOE_DN_ARGS16
   }
   if (few) {  // k_down_few wrote out
     HIPC(c, hipGetLastError());
