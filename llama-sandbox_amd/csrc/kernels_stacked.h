@@ -20,10 +20,11 @@
 //   [0, 96)    hi digits of blocks 0..3, 24 bytes each (6 bits per K offset)
 //   [96, 192)  lo digits, likewise
 //   [192, 208) d of the 4 blocks, f32
-// rows of records one after another.  A chunk of 4 quads of a row is one run
-// of 832 bytes, and the direct global-to-LDS loads of a chunk (1 KiB each)
-// read such runs in order, about 10 cache lines per load; with one 16-byte
-// piece per (token, block) and load, 64 lines, the load path bounds the kernel
+// x row by row (a chunk of 4 quads of a row is one run of 832 bytes), h quad by
+// quad (an item's rows of a quad are one run).  The direct global-to-LDS loads
+// of a chunk (1 KiB each) read such runs in order, about 10 cache lines per
+// load; with one 16-byte piece per (token, block) and load, 64 lines, the load
+// path bounds the kernel
 // (a build that staged 96 bytes per block that way: gate/up of 2048 tokens on
 // the V3 layer 2003 us, 1353 us with the same bytes contiguous).
 //
@@ -134,7 +135,7 @@ __device__ __forceinline__ void stage_quant_quads(const float *__restrict__ x, i
 
 // The 32 h values of a token's unit, 16 in each of the lanes n and n + 32
 // (h[4i + j] = row 8i + 4g + j), as Q8_0 into block b of quad record rec.
-__device__ __forceinline__ void h_quad_store(const float (&h)[16], bool live, uint32_t *rec, int b, int lane) {
+__device__ __forceinline__ void h_quad_store(const float (&h)[16], uint32_t *rec, int b, int lane) {
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(h[i]));
@@ -161,11 +162,9 @@ __device__ __forceinline__ void h_quad_store(const float (&h)[16], bool live, ui
     join48(half48{a[0], e[0]}, half48{a[1], e[1]}, o + 3 * c);
   }
   const int g = lane >> 5;
-  if (live) {
 #pragma unroll
-    for (int i = 0; i < 6; i++) rec[24 * g + 6 * b + i] = o[i];
-    if (!g) rec[48 + b] = __builtin_bit_cast(uint32_t, (float)q8_scale_f16(amax));
-  }
+  for (int i = 0; i < 6; i++) rec[24 * g + 6 * b + i] = o[i];
+  if (!g) rec[48 + b] = __builtin_bit_cast(uint32_t, (float)q8_scale_f16(amax));
 }
 
 // ---------------------------------------------------------------------------
@@ -174,15 +173,20 @@ __device__ __forceinline__ void h_quad_store(const float (&h)[16], bool live, ui
 struct sdma {
   const uint32_t *src;
   uint32_t bytes;
+  uint32_t chunk;            // from one chunk to the next
   uint32_t vo[MOE_SK_WDMA];  // this lane's offsets at chunk 0
   int wave, chunks;
 };
 
-// row: the staged row of token lane % 32 (< 0: absent), of `rows` rows of NQ quads.
-__device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ, int row, int lane, int wave) {
+// row: the staged row of token lane % 32 (< 0: absent), of `rows` rows of NQ
+// quads (quad_major: all rows of a quad, then the next quad).
+__device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ, bool quad_major, int row, int lane,
+                                          int wave) {
   sdma s;
+  const uint32_t rs = quad_major ? 1u : (uint32_t)NQ, qs = quad_major ? (uint32_t)rows : 1u;
   s.src = src;
   s.bytes = (uint32_t)rows * (uint32_t)NQ * (MOE_SQ_DW * 4);
+  s.chunk = MOE_SK_CH * qs * (MOE_SQ_DW * 4);
   s.wave = wave;
   s.chunks = moe_nq4(NQ);
 #pragma unroll
@@ -190,13 +194,13 @@ __device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ,
     const int u = 64 * (wave + MOE_SK_WAVES * i) + lane;
     const int q = u / (MOE_SK_ROWS * MOE_SQ_U4), v = u % (MOE_SK_ROWS * MOE_SQ_U4);
     const int r = __shfl(row, v / MOE_SQ_U4);
-    s.vo[i] = r >= 0 ? ((uint32_t)r * (uint32_t)NQ + q) * (MOE_SQ_DW * 4) + (v % MOE_SQ_U4) * 16 : MOE_SK_OOB;
+    s.vo[i] = r >= 0 ? ((uint32_t)r * rs + (uint32_t)q * qs) * (MOE_SQ_DW * 4) + (v % MOE_SQ_U4) * 16 : MOE_SK_OOB;
   }
   return s;
 }
 
-// Chunk C into buf.  The quads past a row's end (NQ % 4 != 0) read on into the
-// next row, or past the buffer: the K loop does not use them.  A chunk past the
+// Chunk C into buf.  The quads past the end (NQ % 4 != 0) read on into the next
+// row, or past the buffer: the K loop does not use them.  A chunk past the
 // end issues its loads out of range, since the waits count them; its scalar
 // offset stays 0, as the bounds check compares the lane offset with the
 // buffer's size less the scalar offset.
@@ -204,7 +208,7 @@ __device__ __forceinline__ void sdma_issue(const sdma &s, uint32_t *buf, int C) 
   typedef __attribute__((address_space(3))) void *lds_t;
   const bool in = C < s.chunks;
   const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)s.src, 0, (int)s.bytes, MOE_RSRC_FLAGS);
-  const uint32_t so = in ? (uint32_t)C * (MOE_SK_CH * MOE_SQ_DW * 4) : 0u;
+  const uint32_t so = in ? (uint32_t)C * s.chunk : 0u;
 #pragma unroll
   for (int i = 0; i < MOE_SK_WDMA; i++) {
     if (MOE_SK_WAVES * i + s.wave >= MOE_SK_DMA) break;  // uniform over the wave
@@ -391,22 +395,24 @@ __device__ __forceinline__ void sk_group(skring &g, const skw &w, const sdma &st
 // staged tokens.  acc[s]: lane n + 32*g, element 4i + j = row 8i + 4g + j of
 // stream s, token n, summed block by block; GROUPED: the sums of 4-quad groups
 // added up instead.  CPOL: the weights' cache policy.
-template <int CPOL, bool GROUPED>
-__device__ __forceinline__ void sk_loop(const skw &w, const sdma &st, int NQ, uint32_t *lds, int lane, f32x16_t (&acc)[2]) {
+template <int CPOL, bool GROUPED, bool QUAD_MAJOR, class ROW>
+__device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n_src, int NQ, ROW row, uint32_t *lds, int lane,
+                                        int wave, f32x16_t (&acc)[2]) {
   skring g;
   uint32_t sc[2][2];
   f32x16_t tot[2];
-#pragma unroll
-  for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
+  // the first weights go out before the rows are known (for gate/up a load and a division away)
   load_sksc(sc, w, 0);
 #pragma unroll
   for (int i = 0; i + 1 < MOE_SK_RP; i++) load_skw<CPOL>(g.w[i], w, i);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  // chunk 0 has landed (the second chunk, the exponents and the first weights went out after it)
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1 + 4 + 2 * (MOE_SK_RP - 1)));
+  const sdma st = make_sdma(src, n_src, NQ, QUAD_MAJOR, row(), lane, wave);
+#pragma unroll
+  for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1));  // chunk 0 has landed, the second may be on its way
   lds_barrier();
   int cur = 0;
   load_skb(g.b[0], lds, lane, 0, 0);
@@ -457,9 +463,18 @@ __device__ __forceinline__ void sk_loop(const skw &w, const sdma &st, int NQ, ui
   }
 }
 
+// The chunk buffers are free for an epilogue: the chunks issued past the end
+// (zeros) have landed, and every wave has read its last operands.
+__device__ __forceinline__ void sk_lds_free() {
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  lds_barrier();
+}
+
+#define MOE_SK_YST 260  // floats from a token's row to the next in k_down_sk's LDS
+
 // gate/up -> clamp -> SwiGLU -> Q8_0(h) on items of up to 32 rows: one
 // workgroup of 4 waves per (quad of F, item), wave = the gate and the up tile
-// of one 32-row unit over all of K.  h row-major in quad records.  grid (F/128,
+// of one 32-row unit over all of K.  h quad-major in quad records.  grid (F/128,
 // item capacity), 256 threads, LDS MOE_SK_LDS_BYTES.
 template <bool GROUPED>
 __global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
@@ -467,8 +482,8 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
                   const int32_t *__restrict__ items, const int32_t *__restrict__ perm, int k, int T, int F, int H,
                   float clamp, uint32_t *__restrict__ hs, float *__restrict__ htap) {
   extern __shared__ __align__(16) uint32_t lds[];
+  const int4 it = item_of(items, blockIdx.y);  // beside the count (the list holds a record for every grid row)
   if ((int)blockIdx.y >= items[0]) return;
-  const int4 it = item_of(items, blockIdx.y);
   const int NQ = H / 128, NG = moe_nq4(NQ), tiles = F / MOE_TILE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int P = T * k, row0 = it.y, nt = it.z;
@@ -476,23 +491,28 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
   const int u = MOE_SK_WAVES * blockIdx.x + wave, n = lane & 31, gb = lane >> 5;
   const size_t rec = ((size_t)it.x * tiles + 2 * u) * NG * MOE_REC_BYTES;
   const bool live = n < nt;
-  const int xr = live ? (shared ? row0 + n - P : perm[row0 + n] / k) : -1;
-  const sdma st = make_sdma(xs, T, NQ, xr, lane, wave);
+  auto row = [&]() { return live ? (shared ? row0 + n - P : perm[row0 + n] / k) : -1; };
   const skw w = make_skw(w_g + rec, w_u + rec, NQ, lane);
   f32x16_t acc[2];
   // an expert of one item reads its tiles once: non-temporal, as in decode;
   // the items of a larger expert share them through L2
-  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED>(w, st, NQ, lds, lane, acc);
-  else sk_loop<MOE_CPOL_NT, GROUPED>(w, st, NQ, lds, lane, acc);
+  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+  else sk_loop<MOE_CPOL_NT, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
   float h[16];
 #pragma unroll
-  for (int i = 0; i < 16; i++) h[i] = live ? swiglu(acc[0][i], acc[1][i], clamp) : 0.0f;
-  const int hrow = row0 + (live ? n : 0);
-  h_quad_store(h, live, hs + ((size_t)hrow * (F / 128) + blockIdx.x) * MOE_SQ_DW, wave, lane);
+  for (int i = 0; i < 16; i++) h[i] = swiglu(acc[0][i], acc[1][i], clamp);  // an absent token's sums are 0
+  // the 4 waves' blocks meet as whole records in LDS, and the item's records
+  // of this quad leave as one run (stored from the waves in 24-byte pieces they
+  // cost the weight stream 27 of 730 us at 512 tokens)
+  sk_lds_free();
+  h_quad_store(h, lds + n * MOE_SQ_DW, wave, lane);
+  __syncthreads();
+  uint4 *dst = reinterpret_cast<uint4 *>(hs + ((size_t)blockIdx.x * (P + T) + row0) * MOE_SQ_DW);
+  for (int i = threadIdx.x; i < nt * MOE_SQ_U4; i += 64 * MOE_SK_WAVES) dst[i] = reinterpret_cast<const uint4 *>(lds)[i];
   if (htap && live) {
 #pragma unroll
     for (int i = 0; i < 16; i++)
-      htap[(size_t)hrow * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
+      htap[(size_t)(row0 + n) * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
   }
 }
 
@@ -507,8 +527,8 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
                const int32_t *__restrict__ items, const int32_t *__restrict__ perm, const float *__restrict__ wts, int F,
                int H, float *__restrict__ y) {
   extern __shared__ __align__(16) uint32_t lds[];
+  const int4 it = item_of(items, blockIdx.y);  // beside the count (the list holds a record for every grid row)
   if ((int)blockIdx.y >= items[0]) return;
-  const int4 it = item_of(items, blockIdx.y);
   const int NQ = F / 128, NG = moe_nq4(NQ), tiles = H / MOE_TILE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = it.y, nt = it.z;
@@ -518,14 +538,15 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
   const int t64 = MOE_SK_WAVES * blockIdx.x + wave;  // 64 rows of H
   const bool rows = t64 < H / 64;                    // H % 256 == 128: the last workgroup's upper waves only stage
   const uint8_t *w0 = w_d + ((size_t)it.x * tiles + 4 * (rows ? t64 : 0)) * NG * MOE_REC_BYTES;
-  const sdma st = make_sdma(hs, n_rows, NQ, live ? row0 + n : -1, lane, wave);
+  auto row = [&]() { return live ? row0 + n : -1; };
   const skw w = make_skw(w0, w0 + (size_t)2 * NG * MOE_REC_BYTES, NQ, lane);
   f32x16_t acc[2];
-  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED>(w, st, NQ, lds, lane, acc);
-  else sk_loop<MOE_CPOL_NT, GROUPED>(w, st, NQ, lds, lane, acc);
-  if (!live || !rows) return;
-  const float wt = shared ? 1.0f : wts[perm[row0 + n]];
-  float *dst = y + (size_t)(row0 + n) * H + (size_t)t64 * 64 + 4 * gb;
+  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+  else sk_loop<MOE_CPOL_NT, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+  // token rows of 256 columns meet in LDS and leave as runs of 1 KiB
+  sk_lds_free();
+  const float wt = live && !shared ? wts[perm[row0 + n]] : 1.0f;
+  float *red = reinterpret_cast<float *>(lds);  // [token][256 columns, 4 of padding]
 #pragma unroll
   for (int s = 0; s < 2; s++)
 #pragma unroll
@@ -533,6 +554,11 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
       f32x4_t v;
 #pragma unroll
       for (int j = 0; j < 4; j++) v[j] = shared ? acc[s][4 * i + j] : __fmul_rn(acc[s][4 * i + j], wt);
-      *reinterpret_cast<f32x4_t *>(dst + 32 * s + 8 * i) = v;
+      *reinterpret_cast<f32x4_t *>(red + n * MOE_SK_YST + 64 * wave + 32 * s + 8 * i + 4 * gb) = v;
     }
+  __syncthreads();
+  const int col = 256 * blockIdx.x + 4 * lane;
+  if (col >= H) return;
+  for (int t = wave; t < nt; t += MOE_SK_WAVES)
+    *reinterpret_cast<f32x4_t *>(y + (size_t)(row0 + t) * H + col) = *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
 }
