@@ -67,9 +67,10 @@ __device__ __forceinline__ void group_quant(const float *__restrict__ x, int n, 
 //   pass 1: per-wave counts wc[w][e] (one writer per expert per step);
 //   then the histogram (sum over waves), exclusive scans over experts of
 //   the counts and of the item counts ceil(c_e / BT), the item list
-//   (items != NULL: {expert, first row, rows, flags} per item in expert
-//   order, then the shared expert's {E, P + j*BT, rows, flags} when
-//   `shared`; flags: MOE_ITEM_SHARED, MOE_ITEM_SPLIT), and
+//   (items != NULL: the shared expert's {E, P + j*BT, rows, flags} when
+//   `shared` -- its items are the fullest, and started last they would run
+//   alone at the end of the grid --, then {expert, first row, rows, flags} per
+//   item in expert order; flags: MOE_ITEM_SHARED, MOE_ITEM_SPLIT), and
 //   wc[w][e] turned into wave w's first row of expert e;
 //   pass 2: row of a pair = wc[w][e] + rank, so rows ascend in pair order
 //   within each expert (ggml mul_mat_id's order).
@@ -136,6 +137,7 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids,
   if (tid < E)
     for (int w = 0; w < 16; w++) c += wc[w][tid];
   const int ni = items ? (c + BT - 1) / BT : 0;
+  const int n_sh = shared ? (T + BT - 1) / BT : 0;  // the shared expert's items come first
   int v = c, vi = ni;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids,
       wc[w][tid] = (uint16_t)run;
       run += n;
     }
-    int4 *rec = items ? reinterpret_cast<int4 *>(items) + 1 + excli : nullptr;
+    int4 *rec = items ? reinterpret_cast<int4 *>(items) + 1 + n_sh + excli : nullptr;
     for (int j = 0; j < ni; j++) {
       const int r = j * BT;
       rec[j] = make_int4(tid, excl + r, c - r < BT ? c - r : BT, ni > 1 ? MOE_ITEM_SPLIT : 0);
@@ -177,13 +179,12 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t *__restrict__ ids,
   }
   __syncthreads();
   if (items) {
-    const int ns = shared ? (T + BT - 1) / BT : 0;
-    for (int j = tid; j < ns; j += 1024) {
+    for (int j = tid; j < n_sh; j += 1024) {
       const int r = j * BT;
-      reinterpret_cast<int4 *>(items)[1 + tot + j] =
-          make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
+      reinterpret_cast<int4 *>(items)[1 + j] =
+          make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (n_sh > 1 ? MOE_ITEM_SPLIT : 0));
     }
-    if (tid == 0) items[0] = tot + ns;
+    if (tid == 0) items[0] = tot + n_sh;
   }
   // pass 2: row of a pair = wc[w][e] + rank (the lanes of one id read wc
   // before the last of them advances it)
@@ -349,16 +350,16 @@ __device__ __forceinline__ void group_one_wave(const int32_t *__restrict__ ids, 
     }
   }
   int4 *rec = reinterpret_cast<int4 *>(items) + 1;
+  const int ns = shared ? (T + BT - 1) / BT : 0;  // the shared expert's items come first
 #pragma unroll
   for (int i = 0; i < NPL; i++)
     for (int j = 0; j < n[i]; j++) {
       const int r = j * BT;
-      rec[base[i] + j] = make_int4(e[i], less[i] + r, cnt[i] - r < BT ? cnt[i] - r : BT, n[i] > 1 ? MOE_ITEM_SPLIT : 0);
+      rec[ns + base[i] + j] = make_int4(e[i], less[i] + r, cnt[i] - r < BT ? cnt[i] - r : BT, n[i] > 1 ? MOE_ITEM_SPLIT : 0);
     }
-  const int ns = shared ? (T + BT - 1) / BT : 0;  // the shared expert's items follow the routed ones
   for (int j = lane; j < ns; j += 64) {
     const int r = j * BT;
-    rec[tot + j] = make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
+    rec[j] = make_int4(E, P + r, T - r < BT ? T - r : BT, MOE_ITEM_SHARED | (ns > 1 ? MOE_ITEM_SPLIT : 0));
   }
   if (lane == 0) items[0] = tot + ns;
 }

@@ -1,5 +1,5 @@
-// kernels_stacked.h -- grouped gate/up and down on items of up to 32 rows,
-// the two Q8_0 digit planes stacked along K of one MFMA, in fp6.
+// kernels_stacked.h -- grouped gate/up and down on items of up to 32 or 64
+// rows, the two Q8_0 digit planes stacked along K of one MFMA, in fp6.
 //
 // v_mfma_scale_f32_32x32x64_f8f6f4 reduces 64 K per output value.  Here A is
 // the weight tile (A row r = weight row r, fp4 with its E8M0 exponent) and B
@@ -50,8 +50,9 @@
 
 #define MOE_SQ_DW 52    // dwords of a quad record
 #define MOE_SQ_U4 13    // its 16-byte units (odd: the operand reads of 8 tokens hit 8 bank groups)
-#define MOE_SK_CH 4     // quads per staged chunk
-#define MOE_SK_ROWS 32  // rows of an item
+#define MOE_SK_ROWS 32    // tokens of an MFMA
+#define MOE_SK_ROWS2 64   // rows of an item where two token tiles share the weights (sk_loop2)
+#define MOE_SK_CH 4       // quads per staged chunk of 32 rows (of 64 rows: 2)
 #define MOE_SK_BUF_DW (MOE_SK_CH * MOE_SK_ROWS * MOE_SQ_DW)  // 26 KiB
 #define MOE_SK_DMA (MOE_SK_BUF_DW / 256)                     // 1 KiB loads per chunk (26)
 #define MOE_SK_NBUF 2
@@ -179,21 +180,28 @@ struct sdma {
 };
 
 // row: the staged row of token lane % 32 (< 0: absent), of `rows` rows of NQ
-// quads (quad_major: all rows of a quad, then the next quad).
-__device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ, bool quad_major, int row, int lane,
-                                          int wave) {
+// quads (quad_major: all rows of a quad, then the next quad).  NT == 64: row2 is
+// that of token 32 + lane % 32.
+template <int NT>
+__device__ __forceinline__ sdma make_sdma(const uint32_t *src, int rows, int NQ, bool quad_major, int row, int row2,
+                                          int lane, int wave) {
+  constexpr int CH = MOE_SK_CH * MOE_SK_ROWS / NT;  // quads per chunk
   sdma s;
   const uint32_t rs = quad_major ? 1u : (uint32_t)NQ, qs = quad_major ? (uint32_t)rows : 1u;
   s.src = src;
   s.bytes = (uint32_t)rows * (uint32_t)NQ * (MOE_SQ_DW * 4);
-  s.chunk = MOE_SK_CH * qs * (MOE_SQ_DW * 4);
+  s.chunk = CH * qs * (MOE_SQ_DW * 4);
   s.wave = wave;
-  s.chunks = moe_nq4(NQ);
+  s.chunks = (NQ + CH - 1) / CH;
 #pragma unroll
   for (int i = 0; i < MOE_SK_WDMA; i++) {
     const int u = 64 * (wave + MOE_SK_WAVES * i) + lane;
-    const int q = u / (MOE_SK_ROWS * MOE_SQ_U4), v = u % (MOE_SK_ROWS * MOE_SQ_U4);
-    const int r = __shfl(row, v / MOE_SQ_U4);
+    const int q = u / (NT * MOE_SQ_U4), v = u % (NT * MOE_SQ_U4), t = v / MOE_SQ_U4;
+    int r = __shfl(row, t & 31);
+    if (NT == 64) {
+      const int r2 = __shfl(row2, t & 31);
+      r = t < 32 ? r : r2;
+    }
     s.vo[i] = r >= 0 ? ((uint32_t)r * rs + (uint32_t)q * qs) * (MOE_SQ_DW * 4) + (v % MOE_SQ_U4) * 16 : MOE_SK_OOB;
   }
   return s;
@@ -227,16 +235,18 @@ __device__ __forceinline__ const u32x4_t *sk_units(const uint32_t *buf, int lane
   return reinterpret_cast<const u32x4_t *>(buf) + (lane & 31) * MOE_SQ_U4;
 }
 
-// Pair j of quad q of a chunk.
-__device__ __forceinline__ void load_skb(skb &b, const uint32_t *buf, int lane, int q, int j) {
-  const u32x4_t *p = sk_units(buf, lane) + 6 * (lane >> 5) + q * (MOE_SK_ROWS * MOE_SQ_U4) + 3 * j;
+// Pair j of quad q of a chunk (tile: its second 32 tokens of 64).
+template <int NT = 32>
+__device__ __forceinline__ void load_skb(skb &b, const uint32_t *buf, int lane, int q, int j, int tile = 0) {
+  const u32x4_t *p = sk_units(buf, lane) + 6 * (lane >> 5) + (q * NT + 32 * tile) * MOE_SQ_U4 + 3 * j;
 #pragma unroll
   for (int i = 0; i < 3; i++) b.v[i] = p[i];
 }
 
 // d of the quad's 4 blocks for this lane's token.
-__device__ __forceinline__ f32x4_t load_skd(const uint32_t *buf, int lane, int q) {
-  return __builtin_bit_cast(f32x4_t, sk_units(buf, lane)[q * (MOE_SK_ROWS * MOE_SQ_U4) + 12]);
+template <int NT = 32>
+__device__ __forceinline__ f32x4_t load_skd(const uint32_t *buf, int lane, int q, int tile = 0) {
+  return __builtin_bit_cast(f32x4_t, sk_units(buf, lane)[(q * NT + 32 * tile) * MOE_SQ_U4 + 12]);
 }
 
 // Block J of the pair as the MFMA's fp6 operand (6 dwords).
@@ -407,7 +417,7 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
   for (int i = 0; i + 1 < MOE_SK_RP; i++) load_skw<CPOL>(g.w[i], w, i);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  const sdma st = make_sdma(src, n_src, NQ, QUAD_MAJOR, row(), lane, wave);
+  const sdma st = make_sdma<32>(src, n_src, NQ, QUAD_MAJOR, row(0), 0, lane, wave);
 #pragma unroll
   for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
   asm volatile("" ::: "memory");
@@ -453,7 +463,8 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
 #pragma unroll
       for (int j = 0; j < 2; j++) sc[s][j] = g.scn[s][j];
   }
-  if (4 * G < NQ) group(G, NQ - 4 * G);
+  if constexpr (GROUPED)
+    if (4 * G < NQ) group(G, NQ - 4 * G);
   if constexpr (GROUPED) {
     acc[0] = tot[0];
     acc[1] = tot[1];
@@ -461,6 +472,143 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
   }
+}
+
+// ---------------------------------------------------------------------------
+// The same for items of 33-64 rows: two token tiles share each weight pair, so
+// the weights of a large expert are read (mostly from L2) and duplicated
+// across the lane halves half as often: 21 vector instructions per MFMA
+// instead of 26.  A chunk is 2 quads of 64 rows.  V3 layer: 512 tokens Zipf
+// 744 -> 696 us, 2048 tokens 2300 -> 2116 us; V4-Pro layer 806 -> 778 us.
+struct skring2 {
+  u32x4_t w[MOE_SK_RP][2];
+  uint32_t e[2][4];
+  uint32_t scn[2][2];
+  skb b[2];       // B of this pair, per token tile (loaded again as soon as its last MFMA is out)
+  f32x4_t d[2];   // d of this quad, per token tile
+  f32x16_t r[2];  // the last two MFMAs' results
+  float du;       // d of the pending one (token tile 1, stream 1)
+};
+
+template <int SEL, int J, int JD>
+__device__ __forceinline__ void sk_mma2(skring2 &g, f32x16_t &r, const u32x4_t &w, uint32_t e, const skb &b, int sb) {
+  const i32x8_t x = skb_block<J>(b);
+  const i32x8_t a = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
+  const f32x16_t z = {};
+  __builtin_amdgcn_sched_barrier(0);
+  r = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, x, z, 4, 2, SEL, (int)e, 0, sb);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ void sk_fma2(f32x16_t &acc, float d, const f32x16_t &r) {
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[i] = __builtin_fmaf(d, r[i], acc[i]);
+  asm volatile("" : "+v"(acc));
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Pair SG of group G.  acc[tile][stream]; each MFMA runs while the result
+// before it is scaled.  The barrier of a chunk sits at the end of its last pair
+// (SG 3 and 7).
+template <int CPOL, int SG>
+__device__ __forceinline__ void sk_pair2(skring2 &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane, int sb,
+                                         int G, f32x16_t (&acc)[2][2]) {
+  load_skw<CPOL>(g.w[(SG + MOE_SK_RP - 1) % MOE_SK_RP], w, G * 8 + SG + MOE_SK_RP - 1);
+  if constexpr (SG == 0) load_sksc(g.scn, w, G + 1);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4_t a[2][2];  // [stream][block]
+#pragma unroll
+  for (int s = 0; s < 2; s++) dup_halves(g.w[SG % MOE_SK_RP][s], a[s][0], a[s][1]);
+  constexpr int SEL = SG >> 1, j = SG & 1;
+  const float d00 = g.d[0][2 * j], d10 = g.d[1][2 * j], d01 = g.d[0][2 * j + 1], d11 = g.d[1][2 * j + 1];
+  sk_mma2<SEL, 0, 0>(g, g.r[0], a[0][0], g.e[0][2 * j], g.b[0], sb);
+  sk_fma2(acc[1][1], g.du, g.r[1]);
+  sk_mma2<SEL, 0, 0>(g, g.r[1], a[1][0], g.e[1][2 * j], g.b[0], sb);
+  sk_fma2(acc[0][0], d00, g.r[0]);
+  sk_mma2<SEL, 0, 0>(g, g.r[0], a[0][0], g.e[0][2 * j], g.b[1], sb);
+  sk_fma2(acc[0][1], d00, g.r[1]);
+  sk_mma2<SEL, 0, 0>(g, g.r[1], a[1][0], g.e[1][2 * j], g.b[1], sb);
+  sk_fma2(acc[1][0], d10, g.r[0]);
+  sk_mma2<SEL, 1, 0>(g, g.r[0], a[0][1], g.e[0][2 * j + 1], g.b[0], sb);
+  sk_fma2(acc[1][1], d10, g.r[1]);
+  sk_mma2<SEL, 1, 0>(g, g.r[1], a[1][1], g.e[1][2 * j + 1], g.b[0], sb);
+  sk_fma2(acc[0][0], d01, g.r[0]);
+  sk_mma2<SEL, 1, 0>(g, g.r[0], a[0][1], g.e[0][2 * j + 1], g.b[1], sb);
+  sk_fma2(acc[0][1], d01, g.r[1]);
+  sk_mma2<SEL, 1, 0>(g, g.r[1], a[1][1], g.e[1][2 * j + 1], g.b[1], sb);
+  if constexpr ((SG & 3) == 3) {
+    // younger than the next chunk's staging: 4 pairs of two loads, and in a group's first half its exponents
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(4 * 2 + (SG == 3 ? 4 : 0)));
+    lds_barrier();
+    sdma_issue(st, lds + cur * MOE_SK_BUF_DW, 2 * G + (SG >> 2) + MOE_SK_NBUF);
+    cur ^= 1;
+    asm volatile("" ::: "memory");
+  }
+  const uint32_t *buf = lds + cur * MOE_SK_BUF_DW;
+  constexpr int nq = ((SG + 1) & 3) >> 1, nj = (SG + 1) & 1;  // the next pair's quad of its chunk
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    load_skb<64>(g.b[t], buf, lane, nq, nj, t);
+    if constexpr (nj == 0) g.d[t] = load_skd<64>(buf, lane, nq, t);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  sk_fma2(acc[1][0], d11, g.r[0]);
+  g.du = d11;
+}
+
+template <int CPOL, int SG>
+__device__ __forceinline__ void sk_group2(skring2 &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane,
+                                          int sb, int G, f32x16_t (&acc)[2][2]) {
+  if constexpr (SG < 8) {
+    sk_pair2<CPOL, SG>(g, w, st, lds, cur, lane, sb, G, acc);
+    sk_group2<CPOL, SG + 1>(g, w, st, lds, cur, lane, sb, G, acc);
+  }
+}
+
+// acc[tile][stream], block by block in order; NQ % 4 == 0.
+template <int CPOL, bool QUAD_MAJOR, class ROW>
+__device__ __forceinline__ void sk_loop2(const skw &w, const uint32_t *src, int n_src, int NQ, ROW row, uint32_t *lds,
+                                         int lane, int wave, f32x16_t (&acc)[2][2]) {
+  skring2 g;
+  uint32_t sc[2][2];
+  load_sksc(sc, w, 0);
+#pragma unroll
+  for (int i = 0; i + 1 < MOE_SK_RP; i++) load_skw<CPOL>(g.w[i], w, i);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  const sdma st = make_sdma<64>(src, n_src, NQ, QUAD_MAJOR, row(0), row(32), lane, wave);
+#pragma unroll
+  for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1));  // chunk 0 has landed, the second may be on its way
+  lds_barrier();
+  int cur = 0;
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    load_skb<64>(g.b[t], lds, lane, 0, 0, t);
+    g.d[t] = load_skd<64>(lds, lane, 0, t);
+    acc[t][0] = acc[t][1] = f32x16_t{};
+  }
+  g.r[1] = f32x16_t{};  // the first block scales a zero result: acc stays +0
+  g.du = 0.0f;
+  const int sb = (lane >> 5) ? 130 : 134;
+#pragma unroll 1
+  for (int G = 0; 4 * G < NQ; G++) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      dup_halves1(sc[s][0], g.e[s][0], g.e[s][1]);
+      dup_halves1(sc[s][1], g.e[s][2], g.e[s][3]);
+    }
+    sk_group2<CPOL, 0>(g, w, st, lds, cur, lane, sb, G, acc);
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) sc[s][j] = g.scn[s][j];
+  }
+  sk_fma2(acc[1][1], g.du, g.r[1]);
 }
 
 // The chunk buffers are free for an epilogue: the chunks issued past the end
@@ -472,7 +620,7 @@ __device__ __forceinline__ void sk_lds_free() {
 
 #define MOE_SK_YST 260  // floats from a token's row to the next in k_down_sk's LDS
 
-// gate/up -> clamp -> SwiGLU -> Q8_0(h) on items of up to 32 rows: one
+// gate/up -> clamp -> SwiGLU -> Q8_0(h) on items of up to 64 rows: one
 // workgroup of 4 waves per (quad of F, item), wave = the gate and the up tile
 // of one 32-row unit over all of K.  h quad-major in quad records.  grid (F/128,
 // item capacity), 256 threads, LDS MOE_SK_LDS_BYTES.
@@ -490,33 +638,46 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
   const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
   const int u = MOE_SK_WAVES * blockIdx.x + wave, n = lane & 31, gb = lane >> 5;
   const size_t rec = ((size_t)it.x * tiles + 2 * u) * NG * MOE_REC_BYTES;
-  const bool live = n < nt;
-  auto row = [&]() { return live ? (shared ? row0 + n - P : perm[row0 + n] / k) : -1; };
+  auto row = [&](int t0) { return t0 + n < nt ? (shared ? row0 + t0 + n - P : perm[row0 + t0 + n] / k) : -1; };
   const skw w = make_skw(w_g + rec, w_u + rec, NQ, lane);
-  f32x16_t acc[2];
+  // SwiGLU and Q8_0 of 32 tokens into the records of LDS rows t0 ..
+  auto finish = [&](const f32x16_t &g, const f32x16_t &up, int t0) {
+    float h[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) h[i] = swiglu(g[i], up[i], clamp);  // an absent token's sums are 0
+    h_quad_store(h, lds + (t0 + n) * MOE_SQ_DW, wave, lane);
+    if (htap && t0 + n < nt) {
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        htap[(size_t)(row0 + t0 + n) * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
+    }
+  };
   // an expert of one item reads its tiles once: non-temporal, as in decode;
   // the items of a larger expert share them through L2
-  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
-  else sk_loop<MOE_CPOL_NT, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
-  float h[16];
-#pragma unroll
-  for (int i = 0; i < 16; i++) h[i] = swiglu(acc[0][i], acc[1][i], clamp);  // an absent token's sums are 0
+  const bool split = (it.w & MOE_ITEM_SPLIT) != 0;
   // the 4 waves' blocks meet as whole records in LDS, and the item's records
   // of this quad leave as one run (stored from the waves in 24-byte pieces they
   // cost the weight stream 27 of 730 us at 512 tokens)
-  sk_lds_free();
-  h_quad_store(h, lds + n * MOE_SQ_DW, wave, lane);
+  if (!GROUPED && nt > MOE_SK_ROWS) {
+    f32x16_t acc[2][2];
+    if (split) sk_loop2<0, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    else sk_loop2<MOE_CPOL_NT, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    sk_lds_free();
+    finish(acc[0][0], acc[0][1], 0);
+    finish(acc[1][0], acc[1][1], 32);
+  } else {
+    f32x16_t acc[2];
+    if (split) sk_loop<0, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    else sk_loop<MOE_CPOL_NT, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    sk_lds_free();
+    finish(acc[0], acc[1], 0);
+  }
   __syncthreads();
   uint4 *dst = reinterpret_cast<uint4 *>(hs + ((size_t)blockIdx.x * (P + T) + row0) * MOE_SQ_DW);
   for (int i = threadIdx.x; i < nt * MOE_SQ_U4; i += 64 * MOE_SK_WAVES) dst[i] = reinterpret_cast<const uint4 *>(lds)[i];
-  if (htap && live) {
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-      htap[(size_t)(row0 + n) * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
-  }
 }
 
-// down x router weight on items of up to 32 rows: one workgroup of 4 waves
+// down x router weight on items of up to 64 rows: one workgroup of 4 waves
 // per (256 rows of H, item), wave = two 32-row tiles over all of F against the
 // item's h rows; y[row] = the tiles' rows x the pair's router weight (the
 // shared expert's rows unweighted).  grid (ceil(H/256), item capacity), 256
@@ -534,31 +695,45 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
   const int row0 = it.y, nt = it.z;
   const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
   const int n = lane & 31, gb = lane >> 5;
-  const bool live = n < nt;
   const int t64 = MOE_SK_WAVES * blockIdx.x + wave;  // 64 rows of H
   const bool rows = t64 < H / 64;                    // H % 256 == 128: the last workgroup's upper waves only stage
   const uint8_t *w0 = w_d + ((size_t)it.x * tiles + 4 * (rows ? t64 : 0)) * NG * MOE_REC_BYTES;
-  auto row = [&]() { return live ? row0 + n : -1; };
+  auto row = [&](int t0) { return t0 + n < nt ? row0 + t0 + n : -1; };
   const skw w = make_skw(w0, w0 + (size_t)2 * NG * MOE_REC_BYTES, NQ, lane);
-  f32x16_t acc[2];
-  if (it.w & MOE_ITEM_SPLIT) sk_loop<0, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
-  else sk_loop<MOE_CPOL_NT, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
-  // token rows of 256 columns meet in LDS and leave as runs of 1 KiB
-  sk_lds_free();
-  const float wt = live && !shared ? wts[perm[row0 + n]] : 1.0f;
-  float *red = reinterpret_cast<float *>(lds);  // [token][256 columns, 4 of padding]
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      f32x4_t v;
-#pragma unroll
-      for (int j = 0; j < 4; j++) v[j] = shared ? acc[s][4 * i + j] : __fmul_rn(acc[s][4 * i + j], wt);
-      *reinterpret_cast<f32x4_t *>(red + n * MOE_SK_YST + 64 * wave + 32 * s + 8 * i + 4 * gb) = v;
-    }
-  __syncthreads();
   const int col = 256 * blockIdx.x + 4 * lane;
-  if (col >= H) return;
-  for (int t = wave; t < nt; t += MOE_SK_WAVES)
-    *reinterpret_cast<f32x4_t *>(y + (size_t)(row0 + t) * H + col) = *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
+  // the rows of tokens t0 .. t0 + 31, 256 columns each, meet in LDS and leave as runs of 1 KiB
+  auto finish = [&](const f32x16_t &a0, const f32x16_t &a1, int t0) {
+    const bool live = t0 + n < nt;
+    const float wt = live && !shared ? wts[perm[row0 + t0 + n]] : 1.0f;
+    sk_lds_free();
+    float *red = reinterpret_cast<float *>(lds);  // [token][256 columns, 4 of padding]
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const f32x16_t &a = s ? a1 : a0;
+        f32x4_t v;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = shared ? a[4 * i + j] : __fmul_rn(a[4 * i + j], wt);
+        *reinterpret_cast<f32x4_t *>(red + n * MOE_SK_YST + 64 * wave + 32 * s + 8 * i + 4 * gb) = v;
+      }
+    __syncthreads();
+    if (col < H)
+      for (int t = wave; t < 32 && t0 + t < nt; t += MOE_SK_WAVES)
+        *reinterpret_cast<f32x4_t *>(y + (size_t)(row0 + t0 + t) * H + col) =
+            *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
+  };
+  const bool split = (it.w & MOE_ITEM_SPLIT) != 0;
+  if (!GROUPED && nt > MOE_SK_ROWS) {
+    f32x16_t acc[2][2];
+    if (split) sk_loop2<0, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    else sk_loop2<MOE_CPOL_NT, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    finish(acc[0][0], acc[0][1], 0);
+    finish(acc[1][0], acc[1][1], 32);
+  } else {
+    f32x16_t acc[2];
+    if (split) sk_loop<0, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    else sk_loop<MOE_CPOL_NT, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    finish(acc[0], acc[1], 0);
+  }
 }

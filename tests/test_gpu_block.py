@@ -811,6 +811,7 @@ def test_call_stats_count_calls_refusals_and_phases(torch_dev, oracle):
 
 @pytest.mark.parametrize("H,F,counts", [
     (2048, 1024, (1, 31, 32, 33)),    # items around 32 rows; block sums in order
+    (2048, 1024, (64, 65, 5, 128)),   # items around 64 rows: two token tiles
     (640, 384, (64, 65, 0, 15)),      # K of 5 and 3 quads: a partial last group; the last 256 rows of H half there
     (1152, 512, (8, 16, 17, 96)),     # K of 9 quads and of one whole group
     (256, 128, (40, 2, 33, 9)),       # K below one group
