@@ -48,6 +48,8 @@
 
 #include "kernels_grouped.h"
 
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
 #define MOE_SQ_DW 52    // dwords of a quad record
 #define MOE_SQ_U4 13    // its 16-byte units (odd: the operand reads of 8 tokens hit 8 bank groups)
 #define MOE_SK_ROWS 32    // tokens of an MFMA
@@ -228,7 +230,7 @@ __device__ __forceinline__ void sdma_issue(const sdma &s, uint32_t *buf, int C) 
 // ---------------------------------------------------------------------------
 // A block pair (K step) of this lane's B operands: the digits (hi or lo by lane half) of its two blocks.
 struct skb {
-  u32x4_t v[3];
+  i32x8_t x[2];  // the two blocks' MFMA operands (6 dwords of 8)
 };
 
 __device__ __forceinline__ const u32x4_t *sk_units(const uint32_t *buf, int lane) {
@@ -237,26 +239,25 @@ __device__ __forceinline__ const u32x4_t *sk_units(const uint32_t *buf, int lane
 
 // Pair j of quad q of a chunk (tile: its second 32 tokens of 64).
 template <int NT = 32>
-__device__ __forceinline__ void load_skb(skb &b, const uint32_t *buf, int lane, int q, int j, int tile = 0) {
+__device__ __forceinline__ skb load_skb(const uint32_t *buf, int lane, int q, int j, int tile = 0) {
   const u32x4_t *p = sk_units(buf, lane) + 6 * (lane >> 5) + (q * NT + 32 * tile) * MOE_SQ_U4 + 3 * j;
-#pragma unroll
-  for (int i = 0; i < 3; i++) b.v[i] = p[i];
+  const u32x2_t *t = reinterpret_cast<const u32x2_t *>(p + 1);
+  const u32x4_t w0 = p[0];
+  const u32x2_t t0 = t[0];
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");  // t0 and t1 as one load would cost the operands 4 moves a pair
+  const u32x2_t t1 = t[1];
+  const u32x4_t w1 = p[2];
+  skb b;
+  b.x[0] = i32x8_t{(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w, (int)t0.x, (int)t0.y, 0, 0};
+  b.x[1] = i32x8_t{(int)t1.x, (int)t1.y, (int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w, 0, 0};
+  return b;
 }
 
 // d of the quad's 4 blocks for this lane's token.
 template <int NT = 32>
 __device__ __forceinline__ f32x4_t load_skd(const uint32_t *buf, int lane, int q, int tile = 0) {
   return __builtin_bit_cast(f32x4_t, sk_units(buf, lane)[(q * NT + 32 * tile) * MOE_SQ_U4 + 12]);
-}
-
-// Block J of the pair as the MFMA's fp6 operand (6 dwords).
-template <int J>
-__device__ __forceinline__ i32x8_t skb_block(const skb &b) {
-  i32x8_t r;
-#pragma unroll
-  for (int i = 0; i < 6; i++) r[i] = (int)b.v[(6 * J + i) / 4][(6 * J + i) % 4];
-  r[6] = r[7] = 0;
-  return r;
 }
 
 // [x | x] and [y | y] from a register holding x in lanes 0-31, y in 32-63.
@@ -338,7 +339,7 @@ struct skring {
 template <int SEL, int J, int JD>
 __device__ __forceinline__ void sk_block(skring &g, const u32x4_t &w0, const u32x4_t &w1, const skb &b, float d, int sb,
                                          f32x16_t (&acc)[2]) {
-  const i32x8_t x = skb_block<J>(b);
+  const i32x8_t x = b.x[J];
   const i32x8_t a0 = {(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w, 0, 0, 0, 0};
   const i32x8_t a1 = {(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w, 0, 0, 0, 0};
   const f32x16_t z = {};
@@ -379,7 +380,7 @@ __device__ __forceinline__ void sk_pair(skring &g, const skw &w, const sdma &st,
     __builtin_amdgcn_sched_barrier(0);
   }
   const uint32_t *buf = lds + cur * MOE_SK_BUF_DW;
-  load_skb(g.b[(SG + 1) & 1], buf, lane, ((SG + 1) & 7) >> 1, (SG + 1) & 1);
+  g.b[(SG + 1) & 1] = load_skb(buf, lane, ((SG + 1) & 7) >> 1, (SG + 1) & 1);
   if constexpr (SG & 1) g.d[((SG >> 1) + 1) & 1] = load_skd(buf, lane, ((SG + 1) & 7) >> 1);
   u32x4_t a[2][2];
 #pragma unroll
@@ -425,7 +426,7 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1));  // chunk 0 has landed, the second may be on its way
   lds_barrier();
   int cur = 0;
-  load_skb(g.b[0], lds, lane, 0, 0);
+  g.b[0] = load_skb(lds, lane, 0, 0);
   g.d[0] = load_skd(lds, lane, 0);
 #pragma unroll
   for (int s = 0; s < 2; s++) {
@@ -435,7 +436,7 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
   g.r[1] = f32x16_t{};  // the first block scales a zero result: acc stays +0
   g.du = 0.0f;
   const int sb = (lane >> 5) ? 130 : 134;  // lo digits x 2^3 (fp6 codes are eighths), hi digits x 2^7
-  auto group = [&](int G, int quads) {
+  auto group = [&](int G, int quads) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; s++) {
       dup_halves1(sc[s][0], g.e[s][0], g.e[s][1]);
@@ -492,7 +493,7 @@ struct skring2 {
 
 template <int SEL, int J, int JD>
 __device__ __forceinline__ void sk_mma2(skring2 &g, f32x16_t &r, const u32x4_t &w, uint32_t e, const skb &b, int sb) {
-  const i32x8_t x = skb_block<J>(b);
+  const i32x8_t x = b.x[J];
   const i32x8_t a = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
   const f32x16_t z = {};
   __builtin_amdgcn_sched_barrier(0);
@@ -550,7 +551,7 @@ __device__ __forceinline__ void sk_pair2(skring2 &g, const skw &w, const sdma &s
   constexpr int nq = ((SG + 1) & 3) >> 1, nj = (SG + 1) & 1;  // the next pair's quad of its chunk
 #pragma unroll
   for (int t = 0; t < 2; t++) {
-    load_skb<64>(g.b[t], buf, lane, nq, nj, t);
+    g.b[t] = load_skb<64>(buf, lane, nq, nj, t);
     if constexpr (nj == 0) g.d[t] = load_skd<64>(buf, lane, nq, t);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -588,7 +589,7 @@ __device__ __forceinline__ void sk_loop2(const skw &w, const uint32_t *src, int 
   int cur = 0;
 #pragma unroll
   for (int t = 0; t < 2; t++) {
-    load_skb<64>(g.b[t], lds, lane, 0, 0, t);
+    g.b[t] = load_skb<64>(lds, lane, 0, 0, t);
     g.d[t] = load_skd<64>(lds, lane, 0, t);
     acc[t][0] = acc[t][1] = f32x16_t{};
   }
