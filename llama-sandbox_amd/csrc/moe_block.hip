@@ -752,8 +752,8 @@ extern "C" moe_status moe_route(moe_ctx *c, const float *logits, const float *bi
   HIPC(c, hipSetDevice(c->device));
   {
     prof_scope ps(c, K_ROUTE, (hipStream_t)stream, true);
-    hipLaunchKernelGGL(k_route, dim3(T), dim3(256), 0, (hipStream_t)stream, logits, bias, E, k, mode, norm,
-                       scale, ids, wts);
+    hipLaunchKernelGGL(E <= 64 ? k_route<1> : E <= 256 ? k_route<4> : k_route<16>, dim3(T), dim3(64), 0,
+                       (hipStream_t)stream, logits, bias, E, k, mode, norm, scale, ids, wts);
   }
   HIPC(c, hipGetLastError());
   return MOE_OK;

@@ -182,3 +182,24 @@ def test_group_drops_out_of_range_ids(blk, torch_dev, T, k, E):
     np.testing.assert_array_equal(offsets.cpu().numpy(), offsets_ref)
     np.testing.assert_array_equal(perm.cpu().numpy()[: len(perm_ref)], perm_ref)
     np.testing.assert_array_equal(inv.cpu().numpy(), inv_ref)
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 7), (64, 64), (65, 3), (256, 8), (257, 16), (1024, 64)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_route_ties_at_lane_edges(blk, torch_dev, oracle, E, k, mode):
+    """Coarse logits (many equal scores, on one lane and across lanes) at the
+    edges of the experts a lane holds: ids bit-exact, ties to the lower id."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(E + k + mode)
+    T = 5
+    lg = rng.integers(-4, 5, (T, E)).astype(np.float32) / 2
+    lg[0] = 1.0  # every score the same
+    say("route ties", E, k, mode)
+    ids = torch.empty((T, k), dtype=torch.int32, device=dev)
+    wts = torch.empty((T, k), dtype=torch.float32, device=dev)
+    blk.route(torch.from_numpy(lg).to(dev), k, mode, True, 1.0, ids, wts)
+    torch.cuda.synchronize()
+    oi, ow = oracle.route(lg, k, mode, norm=True)
+    np.testing.assert_array_equal(ids.cpu().numpy(), oi)
+    np.testing.assert_allclose(wts.cpu().numpy(), ow, rtol=1e-6)  # a few roundings of expf and the divisions
+
