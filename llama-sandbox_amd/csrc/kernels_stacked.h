@@ -35,7 +35,7 @@
 // holds.  Measured on one box against the e4m3 digits staged in pieces:
 // prefill 512 uniform 1200 -> 1153 us, Zipf 808 -> 732 us, 2048 tokens 2761 ->
 // 2368 us, the V4-Pro layer 927 -> 833 us; 300 tokens on a 5120 x 1536 layer,
-// where the 8-row octet kernels ran, 563 -> 413 us.
+// where the octet kernels ran, 571 -> 458 us (sums in f64, sk_scale).
 //
 // Operand lanes.  A lane r + 32*g holds weight row r, K [32g, 32g + 32): the
 // record layout gives lane (r, g) block 2j + g of a quad in one load, and
@@ -48,6 +48,7 @@
 
 #include "kernels_grouped.h"
 
+typedef double f64x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 #define MOE_SQ_DW 52    // dwords of a quad record
@@ -334,26 +335,36 @@ struct skring {
   float du;            // d of stream 1's pending block
 };
 
+// acc += d * r, in f64 if WIDE.
+template <bool WIDE>
+__device__ __forceinline__ void sk_scale(f32x16_t &acc, f64x16_t &wide, float d, const f32x16_t &r) {
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    if constexpr (WIDE) wide[i] = __builtin_fma((double)d, (double)r[i], wide[i]);
+    else acc[i] = __builtin_fmaf(d, r[i], acc[i]);
+  }
+  if constexpr (WIDE) asm volatile("" : "+v"(wide));
+  else asm volatile("" : "+v"(acc));
+}
+
 // One block against both streams.  Stream 0's MFMA runs while stream 1's last
 // result is scaled, and the other way round; stream 1's result stays pending.
-template <int SEL, int J, int JD>
+// WIDE: the sums in f64 (an f64 FMA issues like an f32 one; each result is
+// converted first).
+template <int SEL, int J, int JD, bool WIDE>
 __device__ __forceinline__ void sk_block(skring &g, const u32x4_t &w0, const u32x4_t &w1, const skb &b, float d, int sb,
-                                         f32x16_t (&acc)[2]) {
+                                         f32x16_t (&acc)[2], f64x16_t (&wide)[2]) {
   const i32x8_t x = b.x[J];
   const i32x8_t a0 = {(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w, 0, 0, 0, 0};
   const i32x8_t a1 = {(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w, 0, 0, 0, 0};
   const f32x16_t z = {};
   g.r[0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, x, z, 4, 2, SEL, (int)g.e[0][JD], 0, sb);
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 16; i++) acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
-  asm volatile("" : "+v"(acc[1]));
+  sk_scale<WIDE>(acc[1], wide[1], g.du, g.r[1]);
   __builtin_amdgcn_sched_barrier(0);
   g.r[1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, x, z, 4, 2, SEL, (int)g.e[1][JD], 0, sb);
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 16; i++) acc[0][i] = __builtin_fmaf(d, g.r[0][i], acc[0][i]);
-  asm volatile("" : "+v"(acc[0]));
+  sk_scale<WIDE>(acc[0], wide[0], d, g.r[0]);
   g.du = d;
   __builtin_amdgcn_sched_barrier(0);
 }
@@ -362,9 +373,9 @@ __device__ __forceinline__ void sk_block(skring &g, const u32x4_t &w0, const u32
 // before its last pair: every wave has then read its operands of that pair, so
 // the buffer is free for the chunk MOE_SK_NBUF ahead, and the next chunk,
 // loaded MOE_SK_NBUF - 1 chunks ago, is visible to all.
-template <int CPOL, int SG>
+template <int CPOL, bool WIDE, int SG>
 __device__ __forceinline__ void sk_pair(skring &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane, int sb,
-                                        int G, f32x16_t (&acc)[2]) {
+                                        int G, f32x16_t (&acc)[2], f64x16_t (&wide)[2]) {
   static_assert(MOE_SK_CH == 4 && 8 % MOE_SK_RP == 0 && MOE_SK_NBUF == 2, "a chunk is one group; two buffers");
   load_skw<CPOL>(g.w[(SG + MOE_SK_RP - 1) % MOE_SK_RP], w, G * 8 + SG + MOE_SK_RP - 1);
   if constexpr (SG == 0) load_sksc(g.scn, w, G + 1);
@@ -388,30 +399,30 @@ __device__ __forceinline__ void sk_pair(skring &g, const skw &w, const sdma &st,
   __builtin_amdgcn_sched_barrier(0);
   const f32x4_t d = g.d[(SG >> 1) & 1];
   constexpr int j = SG & 1;
-  sk_block<(SG >> 1), 0, 2 * j>(g, a[0][0], a[1][0], g.b[j], d[2 * j], sb, acc);
-  sk_block<(SG >> 1), 1, 2 * j + 1>(g, a[0][1], a[1][1], g.b[j], d[2 * j + 1], sb, acc);
+  sk_block<(SG >> 1), 0, 2 * j, WIDE>(g, a[0][0], a[1][0], g.b[j], d[2 * j], sb, acc, wide);
+  sk_block<(SG >> 1), 1, 2 * j + 1, WIDE>(g, a[0][1], a[1][1], g.b[j], d[2 * j + 1], sb, acc, wide);
 }
 
-template <int CPOL, int SG>
+template <int CPOL, bool WIDE, int SG>
 __device__ __forceinline__ void sk_group(skring &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane, int sb,
-                                         int G, int quads, f32x16_t (&acc)[2]) {
+                                         int G, int quads, f32x16_t (&acc)[2], f64x16_t (&wide)[2]) {
   if constexpr (SG < 8) {
     if (quads <= (SG >> 1)) return;  // the last group of a K that is no multiple of 512
-    sk_pair<CPOL, SG>(g, w, st, lds, cur, lane, sb, G, acc);
-    sk_group<CPOL, SG + 1>(g, w, st, lds, cur, lane, sb, G, quads, acc);
+    sk_pair<CPOL, WIDE, SG>(g, w, st, lds, cur, lane, sb, G, acc, wide);
+    sk_group<CPOL, WIDE, SG + 1>(g, w, st, lds, cur, lane, sb, G, quads, acc, wide);
   }
 }
 
 // The K loop of one wave: its two weight streams over NQ quads against the
 // staged tokens.  acc[s]: lane n + 32*g, element 4i + j = row 8i + 4g + j of
-// stream s, token n, summed block by block; GROUPED: the sums of 4-quad groups
-// added up instead.  CPOL: the weights' cache policy.
-template <int CPOL, bool GROUPED, bool QUAD_MAJOR, class ROW>
+// stream s, token n, summed block by block; WIDE: in f64,
+// rounded once.  CPOL: the weights' cache policy.
+template <int CPOL, bool WIDE, bool QUAD_MAJOR, class ROW>
 __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n_src, int NQ, ROW row, uint32_t *lds, int lane,
                                         int wave, f32x16_t (&acc)[2]) {
   skring g;
   uint32_t sc[2][2];
-  f32x16_t tot[2];
+  f64x16_t wide[2];
   // the first weights go out before the rows are known (for gate/up a load and a division away)
   load_sksc(sc, w, 0);
 #pragma unroll
@@ -431,7 +442,7 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
 #pragma unroll
   for (int s = 0; s < 2; s++) {
     acc[s] = f32x16_t{};
-    tot[s] = f32x16_t{};
+    wide[s] = f64x16_t{};
   }
   g.r[1] = f32x16_t{};  // the first block scales a zero result: acc stays +0
   g.du = 0.0f;
@@ -442,16 +453,7 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
       dup_halves1(sc[s][0], g.e[s][0], g.e[s][1]);
       dup_halves1(sc[s][1], g.e[s][2], g.e[s][3]);
     }
-    sk_group<CPOL, 0>(g, w, st, lds, cur, lane, sb, G, quads, acc);
-    if constexpr (GROUPED) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
-        tot[0][i] += acc[0][i];
-        tot[1][i] += acc[1][i];
-        acc[0][i] = acc[1][i] = g.r[1][i] = 0.0f;
-      }
-    }
+    sk_group<CPOL, WIDE, 0>(g, w, st, lds, cur, lane, sb, G, quads, acc, wide);
   };
   int G = 0;
   // whole groups in a loop of their own: with the last group's exits in it,
@@ -464,14 +466,14 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
 #pragma unroll
       for (int j = 0; j < 2; j++) sc[s][j] = g.scn[s][j];
   }
-  if constexpr (GROUPED)
+  if constexpr (WIDE)
     if (4 * G < NQ) group(G, NQ - 4 * G);
-  if constexpr (GROUPED) {
-    acc[0] = tot[0];
-    acc[1] = tot[1];
-  } else {
+  sk_scale<WIDE>(acc[1], wide[1], g.du, g.r[1]);
+  if constexpr (WIDE) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[1][i] = __builtin_fmaf(g.du, g.r[1][i], acc[1][i]);
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[s][i] = (float)wide[s][i];
   }
 }
 
@@ -625,7 +627,7 @@ __device__ __forceinline__ void sk_lds_free() {
 // workgroup of 4 waves per (quad of F, item), wave = the gate and the up tile
 // of one 32-row unit over all of K.  h quad-major in quad records.  grid (F/128,
 // item capacity), 256 threads, LDS MOE_SK_LDS_BYTES.
-template <bool GROUPED>
+template <bool WIDE>
 __global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_u, const uint32_t *__restrict__ xs,
                   const int32_t *__restrict__ items, const int32_t *__restrict__ perm, int k, int T, int F, int H,
@@ -659,7 +661,7 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
   // the 4 waves' blocks meet as whole records in LDS, and the item's records
   // of this quad leave as one run (stored from the waves in 24-byte pieces they
   // cost the weight stream 27 of 730 us at 512 tokens)
-  if (!GROUPED && nt > MOE_SK_ROWS) {
+  if (!WIDE && nt > MOE_SK_ROWS) {
     f32x16_t acc[2][2];
     if (split) sk_loop2<0, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
     else sk_loop2<MOE_CPOL_NT, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
@@ -668,8 +670,8 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
     finish(acc[1][0], acc[1][1], 32);
   } else {
     f32x16_t acc[2];
-    if (split) sk_loop<0, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
-    else sk_loop<MOE_CPOL_NT, GROUPED, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    if (split) sk_loop<0, WIDE, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    else sk_loop<MOE_CPOL_NT, WIDE, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
     sk_lds_free();
     finish(acc[0], acc[1], 0);
   }
@@ -683,7 +685,7 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
 // item's h rows; y[row] = the tiles' rows x the pair's router weight (the
 // shared expert's rows unweighted).  grid (ceil(H/256), item capacity), 256
 // threads, LDS MOE_SK_LDS_BYTES.
-template <bool GROUPED>
+template <bool WIDE>
 __global__ __launch_bounds__(64 * MOE_SK_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, int n_rows,
                const int32_t *__restrict__ items, const int32_t *__restrict__ perm, const float *__restrict__ wts, int F,
@@ -725,7 +727,7 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
             *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
   };
   const bool split = (it.w & MOE_ITEM_SPLIT) != 0;
-  if (!GROUPED && nt > MOE_SK_ROWS) {
+  if (!WIDE && nt > MOE_SK_ROWS) {
     f32x16_t acc[2][2];
     if (split) sk_loop2<0, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
     else sk_loop2<MOE_CPOL_NT, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
@@ -733,8 +735,8 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
     finish(acc[1][0], acc[1][1], 32);
   } else {
     f32x16_t acc[2];
-    if (split) sk_loop<0, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
-    else sk_loop<MOE_CPOL_NT, GROUPED, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    if (split) sk_loop<0, WIDE, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    else sk_loop<MOE_CPOL_NT, WIDE, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
     finish(acc[0], acc[1], 0);
   }
 }

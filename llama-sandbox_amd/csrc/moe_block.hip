@@ -890,14 +890,17 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
   // a few tokens (the pairs path): down per 16-row tile of H with the slot
   // combine in the same launch (k_down_few)
   const bool few = !oct && T <= MOE_DF_TMAX && k + 1 <= MOE_DF_SMAX && H % MOE_DF_ROWS == 0;
-  // the stacked kernels add their block sums one by one on the shapes that
-  // always did (results keep their bits), else in groups (a smaller error)
+  // the stacked kernels add their block sums one by one in f32 on the shapes
+  // that always did (results keep their bits).  The others' results came from
+  // the octet kernels, which err less (their separate digit planes round less
+  // often), so their sums are in f64: 300 tokens on a 5120 x 1536 layer 571 ->
+  // 458 us, rows 4.9e-8 -> 3.6e-8 from 64 bits (f32 group sums 405 us, 7.2e-8)
   const bool in_order = (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
                         (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24);
   // items of up to 64 rows from 4 pairs per expert on: the shared weights of
   // two token tiles save 7% at 64 rows per expert (2048 tokens on the V3 layer
   // 2308 -> 2134 us) and cost the fewer workgroups of a small call 6% (64
-  // tokens 241 -> 259 us); the grouped sums have no registers for two tiles
+  // tokens 241 -> 259 us); the f64 sums leave no registers for two tiles
   const int BT = sk ? (in_order && P >= 4 * E ? MOE_SK_ROWS2 : MOE_SK_ROWS) : oct ? 8 : 4;
   int32_t *counts = s.grp, *offsets = counts + E, *perm = offsets + E + 1, *inv = perm + P, *items = inv + P;
   float *htap = c->taps ? s.htap : nullptr;
