@@ -46,6 +46,7 @@
 // gate and up of the same values).
 #pragma once
 
+#include "grouped_plan.h"
 #include "kernels_grouped.h"
 
 typedef double f64x16_t __attribute__((ext_vector_type(16)));
@@ -53,8 +54,7 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 #define MOE_SQ_DW 52    // dwords of a quad record
 #define MOE_SQ_U4 13    // its 16-byte units (odd: the operand reads of 8 tokens hit 8 bank groups)
-#define MOE_SK_ROWS 32    // tokens of an MFMA
-#define MOE_SK_ROWS2 64   // rows of an item where two token tiles share the weights (sk_loop2)
+#define MOE_SK_ROWS MOE_PLAN_ROWS  // tokens of an MFMA; items of up to MOE_PLAN_ROWS2 rows take two (sk_loop2)
 #define MOE_SK_CH 4       // quads per staged chunk of 32 rows (of 64 rows: 2)
 #define MOE_SK_BUF_DW (MOE_SK_CH * MOE_SK_ROWS * MOE_SQ_DW)  // 26 KiB
 #define MOE_SK_DMA (MOE_SK_BUF_DW / 256)                     // 1 KiB loads per chunk (26)

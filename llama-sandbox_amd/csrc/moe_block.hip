@@ -9,6 +9,7 @@
 
 #include "device_common.h"
 #include "gguf_reader.h"
+#include "grouped_plan.h"
 #include "kernels_decode.h"
 #include "kernels_group.h"
 #include "kernels_grouped.h"
@@ -870,12 +871,7 @@ static moe_status forward_decode(moe_ctx *c, dev_layer &L, work_bufs &s, const f
   return MOE_OK;
 }
 
-// The grouped chain runs token pairs on the 16x16x128 MFMA for T <= 4
-// (items of at most 4 rows: NPMAX = 2 pairs), token octets on the 32x32x64
-// MFMA above that (items of at most 8 rows), and the stacked kernels on items
-// of up to 32 rows where the batch averages 2 pairs per expert or more.
-static bool use_octets(int T) { return T > 4; }
-
+// The grouped chain for T > 1, on the kernels that grouped_plan.h chooses.
 static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const float *x, const int32_t *ids,
                                   const float *wts, int T, float *out, uint32_t flags, hipStream_t st) {
   const moe_layer_desc &d = L.d;
@@ -885,23 +881,12 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
   if (P > MOE_GROUP_MAX_PAIRS || E > MOE_GROUP_MAX_E)
     return fail(c, MOE_ERR_UNSUPPORTED, "grouped: more than %d pairs or %d experts", MOE_GROUP_MAX_PAIRS,
                 MOE_GROUP_MAX_E);
-  const bool oct = use_octets(T);
-  const bool sk = oct && P >= 2 * E;
+  const grouped_plan plan = plan_grouped(T, k, E, H, F, shared != 0);
+  const bool oct = plan.octets, sk = plan.stacked, in_order = plan.in_order;
+  const int BT = plan.item_rows;
   // a few tokens (the pairs path): down per 16-row tile of H with the slot
   // combine in the same launch (k_down_few)
   const bool few = !oct && T <= MOE_DF_TMAX && k + 1 <= MOE_DF_SMAX && H % MOE_DF_ROWS == 0;
-  // the stacked kernels add their block sums one by one in f32 on the shapes
-  // that always did (results keep their bits).  The others' results came from
-  // the octet kernels, which err less (their separate digit planes round less
-  // often), so their sums are in f64: 300 tokens on a 5120 x 1536 layer 571 ->
-  // 458 us, rows 4.9e-8 -> 3.6e-8 from 64 bits (f32 group sums 405 us, 7.2e-8)
-  const bool in_order = (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
-                        (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24);
-  // items of up to 64 rows from 4 pairs per expert on: the shared weights of
-  // two token tiles save 7% at 64 rows per expert (2048 tokens on the V3 layer
-  // 2308 -> 2134 us) and cost the fewer workgroups of a small call 6% (64
-  // tokens 241 -> 259 us); the f64 sums leave no registers for two tiles
-  const int BT = sk ? (in_order && P >= 4 * E ? MOE_SK_ROWS2 : MOE_SK_ROWS) : oct ? 8 : 4;
   int32_t *counts = s.grp, *offsets = counts + E, *perm = offsets + E + 1, *inv = perm + P, *items = inv + P;
   float *htap = c->taps ? s.htap : nullptr;
   const int n_xblocks = T * (H / MOE_QK);
@@ -937,8 +922,8 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     const size_t lo = octet_lds_bytes(F / MOE_QK);
     if (sk)
       hipLaunchKernelGGL(in_order ? k_down_sk<false> : k_down_sk<true>,
-                         dim3(ceil_div(H, 64 * MOE_SK_WAVES), cap), dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st, L.m[T_DOWN].w, s.hq, P + T, items, perm, wts, F, H,
-                         s.y);
+                         dim3(ceil_div(H, 64 * MOE_SK_WAVES), cap), dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st,
+                         L.m[T_DOWN].w, s.hq, P + T, items, perm, wts, F, H, s.y);
     else if (oct && F == 128 * 16) hipLaunchKernelGGL(k_down_ol<16>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
     else if (oct && F == 128 * 6) hipLaunchKernelGGL(k_down_ol<6>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
     else if (oct && F == 128 * 8) hipLaunchKernelGGL(k_down_ol<8>, gdo, dim3(256), lo, st, MOE_DN_ARGS);

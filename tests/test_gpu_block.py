@@ -809,28 +809,34 @@ def test_call_stats_count_calls_refusals_and_phases(torch_dev, oracle):
 
 # ---- the stacked kernels at their edges ---------------------------------------------
 
-@pytest.mark.parametrize("H,F,counts", [
-    (2048, 1024, (1, 31, 32, 33)),    # items around 32 rows; block sums in order
-    (2048, 1024, (64, 65, 5, 128)),   # items around 64 rows: two token tiles
-    (640, 384, (64, 65, 0, 15)),      # K of 5 and 3 quads: a partial last group; the last 256 rows of H half there
-    (1152, 512, (8, 16, 17, 96)),     # K of 9 quads and of one whole group
-    (256, 128, (40, 2, 33, 9)),       # K below one group
-])
+# H, F, experts, rows of the first experts, rows of each other one (enough of
+# both that the call runs stacked)
+STACKED_EDGES = [
+    (2048, 1024, 32, (1, 31, 32, 33), 5),    # items around 32 rows; block sums in order
+    (2048, 1024, 128, (64, 65, 5, 128), 3),  # items around 64 rows: two token tiles
+    (640, 384, 16, (64, 65, 0, 15), 70),     # K of 5 and 3 quads: a partial last group; the last 256 rows of H half there
+    (1152, 512, 16, (8, 16, 17, 96), 40),    # K of 9 quads and of one whole group
+    (256, 128, 64, (40, 2, 33, 9), 38),      # K below one group
+]
+
+
+@pytest.mark.parametrize("H,F,E,first,rest", STACKED_EDGES)
 @pytest.mark.parametrize("per_slot", [False, True])
-def test_stacked_item_edges(blk, torch_dev, oracle, H, F, counts, per_slot):
+def test_stacked_item_edges(blk, torch_dev, oracle, H, F, E, first, rest, per_slot):
     """Items of the given sizes (one expert each, top-1) through the stacked
     gate/up and down kernels, with the shared expert's items and the clamp."""
-    shape = wl.LayerShape(hidden=H, ffn=F, n_expert=len(counts), n_used=1, has_shared=True, route_mode=1, clamp=6.0)
+    counts = first + (rest,) * (E - len(first))
+    shape = wl.LayerShape(hidden=H, ffn=F, n_expert=E, n_used=1, has_shared=True, route_mode=1, clamp=6.0)
     T = sum(counts)
     rng = np.random.default_rng(H + F)
     x = rng.standard_normal((T, H)).astype(np.float32)
-    ids = rng.permutation(np.repeat(np.arange(len(counts), dtype=np.int32), counts))[:, None].astype(np.int32)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None].astype(np.int32)
     wts = rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)
-    say("stacked edges", H, F, counts, "per_slot", per_slot)
+    say("stacked edges", H, F, E, first, rest, "per_slot", per_slot)
     blk.generate_layer(60, shape, seed=H, e_lo=116, e_span=5)
     try:
         got = run_block(blk, torch_dev, 60, x, ids, wts, mb.MOE_FWD_PER_SLOT if per_slot else 0)
         L = oracle_layer(oracle, shape, H, 60, ids, e_lo=116, e_span=5)
-        check_block(oracle, L, blk, shape, x, ids, wts, got, f"stacked {H}x{F} {counts}", per_slot=per_slot)
+        check_block(oracle, L, blk, shape, x, ids, wts, got, f"stacked {H}x{F} {first}", per_slot=per_slot)
     finally:
         blk.release_layer(60)

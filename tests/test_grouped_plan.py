@@ -1,0 +1,112 @@
+"""Which kernels a grouped call runs on (csrc/grouped_plan.h), without a GPU:
+the header is plain C++, compiled here and asked."""
+import os
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+MAIN = """
+#include <cstdio>
+#include "grouped_plan.h"
+int main() {
+  int T, k, E, H, F, s;
+  while (scanf("%d %d %d %d %d %d", &T, &k, &E, &H, &F, &s) == 6) {
+    const grouped_plan p = plan_grouped(T, k, E, H, F, s != 0);
+    printf("%s %d\\n", !p.octets ? "pairs" : !p.stacked ? "octets" : p.in_order ? "stacked_f32" : "stacked_f64", p.item_rows);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    (d / "main.cpp").write_text(MAIN)
+    exe = d / "plan"
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-I", os.path.join(REPO, "llama-sandbox_amd", "csrc"),
+                    "-o", str(exe), str(d / "main.cpp")], check=True)
+
+    def ask(calls):  # calls: (T, k, E, H, F, shared) -> (kernels, rows of an item)
+        text = "".join(" ".join(str(int(v)) for v in c) + "\n" for c in calls)
+        out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.split("\n")
+        return [(o.split()[0], int(o.split()[1])) for o in out if o]
+
+    return ask
+
+
+# Calls that the stacked kernels ran slower than the octets (us per layer with
+# cold weights, octets / stacked): too few workgroups for the chip, or too few
+# rows per expert for sums in f64.
+SLOWER_STACKED = [
+    (8, 2, 8, 5120, 1536, False),      # 33 / 57
+    (64, 2, 8, 5120, 1536, False),     # 49 / 61
+    (24, 4, 32, 5120, 1536, True),     # 90 / 111
+    (32, 8, 128, 5120, 1536, True),    # 259 / 306
+    (48, 8, 128, 6400, 2560, True),    # 556 / 604
+    (64, 8, 128, 2048, 768, True),     # 73 / 94
+    (16, 2, 8, 1152, 512, False),      # 17 / 25
+    (12, 2, 8, 7168, 1792, False),     # 44 / 75
+    (128, 2, 8, 4096, 640, False),     # 41 / 50
+    (128, 2, 8, 1024, 3072, False),    # 46 / 51
+    (16, 2, 8, 7168, 2048, False),     # 47 / 65
+    (8, 2, 8, 2048, 1024, False),      # 20 / 29
+    (32, 4, 32, 4096, 1536, True),     # 78 / 84
+    (64, 2, 8, 6144, 1024, False),     # 48 / 52
+]
+
+# and calls that gain from them: enough rows, enough workgroups (octets / stacked)
+FASTER_STACKED = [
+    (300, 6, 160, 5120, 1536, True, "stacked_f64"),
+    (128, 4, 32, 5120, 1536, True, "stacked_f64"),     # 165 / 122
+    (256, 8, 128, 6400, 2560, True, "stacked_f64"),    # 1098 / 749
+    (512, 4, 32, 1152, 512, True, "stacked_f64"),      # 70 / 47
+    (64, 8, 256, 7168, 2048, True, "stacked_f32"),
+    (128, 8, 128, 7168, 2048, True, "stacked_f32"),    # 632 / 532
+    (512, 8, 256, 7168, 2048, True, "stacked_f32"),
+    (509, 6, 384, 7168, 3072, True, "stacked_f32"),
+    (64, 2, 8, 7168, 2048, False, "stacked_f32"),      # 78 / 64
+    (512, 4, 32, 2048, 1024, True, "stacked_f32"),     # 148 / 75
+]
+
+
+def test_small_calls_run_on_octets(plan):
+    assert plan(SLOWER_STACKED) == [("octets", 8)] * len(SLOWER_STACKED)
+
+
+def test_full_calls_run_stacked(plan):
+    assert [p[0] for p in plan([c[:6] for c in FASTER_STACKED])] == [c[6] for c in FASTER_STACKED]
+
+
+def test_plan_limits(plan):
+    """Pairs up to 4 tokens; never stacked below 2 pairs per expert; the f32
+    loops only where K of both kernels is whole groups of 4 quads (they have no
+    code for a partial one)."""
+    calls = [(T, k, E, 128 * h, 128 * f, s) for T in (2, 4, 5, 9, 64, 700, 8191) for k in (1, 3, 8)
+             for E in (8, 33, 384, 1024) for h in (1, 5, 16, 31, 32, 48, 56, 80) for f in (1, 4, 6, 8, 12, 13, 16, 24, 28)
+             for s in (0, 1)]
+    seen = set()
+    for (T, k, E, H, F, _), (kind, rows) in zip(calls, plan(calls)):
+        assert (kind == "pairs") == (T <= 4)
+        if T * k < 2 * E:
+            assert not kind.startswith("stacked")
+        if kind == "stacked_f32":
+            assert H % 512 == 0 and F % 512 == 0
+        assert rows in {"pairs": (4,), "octets": (8,), "stacked_f64": (32,), "stacked_f32": (32, 64)}[kind]
+        seen.add((kind, rows))
+    assert len(seen) == 5
+
+
+def test_gpu_tests_reach_the_kernels_they_name(plan):
+    import test_gpu_block as gpu
+
+    for H, F, E, first, rest in gpu.STACKED_EDGES:
+        T = sum(first) + rest * (E - len(first))
+        kinds = plan([(T, 1, E, H, F, s) for s in (False, True)])
+        assert [k for k, _ in kinds] == ["stacked_f32" if H == 2048 else "stacked_f64"] * 2, (H, F)
+    sweep = [c for c in gpu.SWEEP if c[4] > 1]
+    kinds = [k for k, _ in plan([(T, k, E, H, F, sh) for H, F, E, k, T, sh, _, _ in sweep])]
+    assert {"pairs", "octets", "stacked_f32"} <= set(kinds)
+    octets = {c[1] // 128 for c, k in zip(sweep, kinds) if k == "octets"}  # F / 128: the down kernel's instance
+    assert {6, 8, 16, 28} <= octets and octets - {6, 8, 16, 28}  # k_down_ol<6, 8, 16, 28> and k_down_o
