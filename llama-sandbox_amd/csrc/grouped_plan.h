@@ -54,10 +54,20 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   const bool worth = p.in_order ? n8 >= 512 && (P >= 5L * E || n8 >= 1536)
                                 : n8 >= 640 && (P >= 8L * E || (P >= 4L * E && n8 >= 3000));
   p.stacked = p.octets && P >= 2L * E && worth;
-  // items of up to 64 rows from 4 pairs per expert on: the shared weights of
-  // two token tiles save 7% at 64 rows per expert (2048 tokens on the V3 layer
-  // 2308 -> 2134 us) and cost the fewer workgroups of a small call 6% (64
-  // tokens 241 -> 259 us); the f64 sums leave no registers for two tiles
-  p.item_rows = !p.octets ? 4 : !p.stacked ? 8 : p.in_order && P >= 4L * E ? MOE_PLAN_ROWS2 : MOE_PLAN_ROWS;
+  // Two token tiles per weight pair (items of up to 64 rows): a weight is read
+  // and duplicated once for both, 2048 tokens on the V3 layer 2308 -> 2134 us,
+  // but the workgroups are half as many and run twice as long.  So only where
+  // 64-row items still make two rounds of workgroups (512 a round) in the launch
+  // that has fewer, from 4 pairs per expert on (below that the shared expert's
+  // items are the only large ones: 64 tokens on the V3 layer 241 -> 259 us).  us
+  // per layer, 32-row / 64-row items, 32 and 64 rows per expert:
+  //   7168 x 2048, 8 experts 78/92  104/111; 32 experts 232/221  333/360; 128 experts 762/718  1214/1094
+  //   2048 x 1024, 8 experts 34/44  35/48; 32 experts 54/65  75/76; 128 experts 148/152  219/221
+  //   4096 x 1536, 32 experts 114/112  166/176; 128 experts 361/350  561/524
+  // The f64 sums leave no registers for two tiles.
+  const long items64 = (P / 64 > E ? P / 64 : E) + (shared ? T / 64 : 0);
+  const int gu2 = F / 128, dn2 = H / 256;  // stacked workgroups per item
+  const bool two = p.in_order && P >= 4L * E && items64 * (gu2 < dn2 ? gu2 : dn2) >= 1024;
+  p.item_rows = !p.octets ? 4 : !p.stacked ? 8 : two ? MOE_PLAN_ROWS2 : MOE_PLAN_ROWS;
   return p;
 }

@@ -79,6 +79,22 @@ def test_full_calls_run_stacked(plan):
     assert [p[0] for p in plan([c[:6] for c in FASTER_STACKED])] == [c[6] for c in FASTER_STACKED]
 
 
+def test_items_of_64_rows_only_where_the_chip_stays_full(plan):
+    """Two token tiles halve the workgroups: us per layer, 32-row / 64-row items."""
+    slower = [(128, 2, 8, 7168, 2048, False),    # 78 / 92
+              (512, 4, 32, 7168, 2048, True),    # 333 / 360
+              (256, 2, 8, 2048, 1024, False),    # 35 / 48
+              (256, 4, 32, 6144, 1024, True),    # 117 / 139
+              (64, 4, 32, 4096, 1536, True)]     # 86 / 95: the shared expert's item of 64 rows
+    faster = [(512, 8, 128, 7168, 2048, True),   # 762 / 718
+              (1024, 8, 128, 4096, 1536, True),  # 561 / 524
+              (512, 8, 256, 7168, 2048, True),   # Zipf 744 / 696
+              (509, 6, 384, 7168, 3072, True),   # Zipf 806 / 778
+              (2048, 8, 256, 7168, 2048, True)]  # 2300 / 2116
+    assert plan(slower) == [("stacked_f32", 32)] * len(slower)
+    assert plan(faster) == [("stacked_f32", 64)] * len(faster)
+
+
 def test_plan_limits(plan):
     """Pairs up to 4 tokens; never stacked below 2 pairs per expert; the f32
     loops only where K of both kernels is whole groups of 4 quads (they have no
@@ -104,7 +120,7 @@ def test_gpu_tests_reach_the_kernels_they_name(plan):
     for H, F, E, first, rest in gpu.STACKED_EDGES:
         T = sum(first) + rest * (E - len(first))
         kinds = plan([(T, 1, E, H, F, s) for s in (False, True)])
-        assert [k for k, _ in kinds] == ["stacked_f32" if H == 2048 else "stacked_f64"] * 2, (H, F)
+        assert kinds == [("stacked_f32", 64 if E == 128 else 32) if H == 2048 else ("stacked_f64", 32)] * 2, (H, F)
     sweep = [c for c in gpu.SWEEP if c[4] > 1]
     kinds = [k for k, _ in plan([(T, k, E, H, F, sh) for H, F, E, k, T, sh, _, _ in sweep])]
     assert {"pairs", "octets", "stacked_f32"} <= set(kinds)
