@@ -7,7 +7,8 @@
 // ---------------------------------------------------------------------------
 // Router, one wave per token (E <= 1024).  Scores, selection bias, top-k (ties
 // -> lower id), weights from the unbiased scores, renorm with the 2^-14 floor,
-// scale (glm_dsa/moe_block.h:48-91).
+// scale (glm_dsa/moe_block.h:48-91).  A NaN score is picked only when no number
+// is left, lowest id first, so the ids of a token are always k different experts.
 //
 // Bound by latency: a token's scores stay in its wave's registers (lane l holds
 // experts l, l + 64, ...), and a round of the top-k is one wave maximum over

@@ -203,3 +203,49 @@ def test_route_ties_at_lane_edges(blk, torch_dev, oracle, E, k, mode):
     np.testing.assert_array_equal(ids.cpu().numpy(), oi)
     np.testing.assert_allclose(wts.cpu().numpy(), ow, rtol=1e-6)  # a few roundings of expf and the divisions
 
+
+@pytest.mark.parametrize("E,k", [(63, 7), (65, 3), (257, 16), (1024, 64)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_route_bias_ties_at_lane_edges(blk, torch_dev, oracle, E, k, mode):
+    """The same with a selection bias, coarse too: picks by score + bias, ties
+    to the lower id, weights from the scores alone."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(E + k + mode)
+    lg = rng.integers(-4, 5, (5, E)).astype(np.float32) / 2
+    bias = (rng.integers(-2, 3, E) / 4).astype(np.float32)
+    say("route bias ties", E, k, mode)
+    ids = torch.empty((5, k), dtype=torch.int32, device=dev)
+    wts = torch.empty((5, k), dtype=torch.float32, device=dev)
+    blk.route(torch.from_numpy(lg).to(dev), k, mode, True, 2.5, ids, wts, bias=torch.from_numpy(bias).to(dev))
+    torch.cuda.synchronize()
+    oi, ow = oracle.route(lg, k, mode, norm=True, scale=2.5, bias=bias)
+    np.testing.assert_array_equal(ids.cpu().numpy(), oi)
+    np.testing.assert_allclose(wts.cpu().numpy(), ow, rtol=1e-6)  # as without a bias
+
+
+@pytest.mark.parametrize("E,k", [(8, 8), (64, 9), (130, 9), (600, 20)])
+def test_route_nan_and_inf_scores(blk, torch_dev, E, k):
+    """Scores that are no numbers come last, by id; infinite ones keep their
+    place; ids are distinct and in range whatever the logits are."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(E)
+    lg = rng.permutation(np.linspace(-3, 3, 6 * E).astype(np.float32)).reshape(6, E)
+    lg[0] = np.nan
+    lg[1, rng.permutation(E)[: E - k + 1]] = np.nan    # fewer numbers than picks
+    lg[2, rng.permutation(E)[: E // 2]] = np.nan
+    lg[3, rng.permutation(E)[: E // 2]] = -np.inf      # scores 0, equal: by id
+    lg[4, :2] = np.nan, -np.inf
+    lg[5, E - 1] = np.inf
+    say("route nan", E, k)
+    for mode in (1, 2, 0):
+        ids = torch.full((6, k), -7, dtype=torch.int32, device=dev)
+        wts = torch.empty((6, k), dtype=torch.float32, device=dev)
+        blk.route(torch.from_numpy(lg).to(dev), k, mode, False, 1.0, ids, wts)
+        torch.cuda.synchronize()
+        got = ids.cpu().numpy()
+        for t in range(6):
+            nan = np.isnan(lg[t])
+            if mode == 0 and (nan.any() or np.isposinf(lg[t]).any()):
+                nan[:] = True  # one of them makes the whole softmax NaN
+            want = np.lexsort((np.arange(E), np.where(nan, 0.0, -lg[t]), nan))[:k]  # the scores rise with the logits
+            np.testing.assert_array_equal(got[t], want, err_msg=f"mode {mode} row {t}")
