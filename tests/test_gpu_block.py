@@ -158,10 +158,10 @@ def test_c1_multi_token_grouped(blk, torch_dev, oracle, c1):
                 per_slot=True)
 
 
-def test_c1_grouped_two_octets_per_wave(blk, torch_dev, oracle, c1):
-    """T = 40 on C1 (160 pairs over 32 experts, >= 2 per expert on average):
-    gate/up and down run on items of up to 16 rows with one or two octets per
-    wave (k_gate_up_ol, k_down_ol2); items of both sizes occur."""
+def test_c1_grouped_several_octets_per_expert(blk, torch_dev, oracle, c1):
+    """T = 40 on C1 (160 pairs over 32 experts): gate/up and down run on octets
+    (k_gate_up_o, k_down_ol<6>), experts of one and of several octets among
+    them."""
     x, lg = wl.make_inputs(c1, 40, 23, zipf=True)
     ids, wts = oracle.route(lg, c1.n_used, c1.route_mode, norm=True)
     counts = np.bincount(ids.ravel(), minlength=c1.n_expert)
@@ -359,10 +359,8 @@ def test_prefill_bench_shapes(blk, torch_dev, oracle, which, zipf):
     configurations, at their full size, every token against the oracle:
     the reference's DeepSeek-V4-Pro layer (hip-moe/README.md:280-286:
     7168 -> 3072, 384 experts, top-6 sqrt(softplus) routing renormalised
-    and scaled by 2.5, SwiGLU clamped at 10, one shared expert;
-    k_gate_up_sk<56> over 24 slices of F, k_down_sk<24>), uniform and
-    Zipf-routed, and the V3 layer with 1536-wide experts (12 slices of F,
-    k_down_sk<12>)."""
+    and scaled by 2.5, SwiGLU clamped at 10, one shared expert), uniform and
+    Zipf-routed, and the V3 layer with 1536-wide experts; all stacked."""
     shape = wl.V4P if which == "V4P" else wl.V3F1536
     lid = 60 if which == "V4P" else 61
     T = 512
@@ -379,22 +377,41 @@ def test_prefill_bench_shapes(blk, torch_dev, oracle, which, zipf):
         blk.release_layer(lid)
 
 
+@pytest.fixture(scope="module")
+def small(blk):
+    shape = wl.LayerShape(hidden=1152, ffn=512, n_expert=16, n_used=4, has_shared=True, route_mode=wl.ROUTE_SIGMOID)
+    blk.generate_layer(3, shape, seed=303, e_lo=116, e_span=5)
+    yield shape
+    blk.release_layer(3)
+
+
+@pytest.fixture(scope="module")
+def many(blk):
+    shape = wl.LayerShape(hidden=2048, ffn=1024, n_expert=128, n_used=4, has_shared=True, route_mode=wl.ROUTE_SIGMOID)
+    blk.generate_layer(4, shape, seed=404, e_lo=116, e_span=5)
+    yield shape
+    blk.release_layer(4)
+
+
 @pytest.mark.slow
-@pytest.mark.parametrize("which, T", [("c1", 3), ("c1", 12), ("c1", 40), ("v3", 4), ("v3", 16), ("v3", 64)])
+@pytest.mark.parametrize("which, T", [("c1", 3), ("c1", 12), ("c1", 40), ("v3", 4), ("v3", 16), ("v3", 64),
+                                      ("small", 160), ("many", 192)])
 def test_out_of_range_ids_contribute_nothing(request, blk, torch_dev, oracle, which, T):
     """Pairs whose expert id is out of range (-1 or E) belong to no work item:
     their per-slot rows are exactly 0 and they add nothing to the slot sum;
     token 0 has every pair out of range (its output is exactly 0 on C1, the
     shared expert's row alone on V3).  Every down path runs: the pairs path
     with its fused slot combine (T = 3, 4), 8-row octet items (C1 T=12, V3
-    T=16), 16-row items (C1 T=40) and the stacked kernels' 32-row items (V3
-    T=64).  The yardstick is check_block on the oracle with the original
+    T=16, C1 T=40 with several per expert) and the stacked kernels' items of up
+    to 32 rows (V3 T=64, and in f64 on the small layer) and 64 rows (128
+    experts, T=192).  The yardstick is check_block on the oracle with the original
     (valid) ids and the dropped pairs' router weights set to 0, the GPU's h
     taps standing in for the kept pairs and the shared expert (the oracle's
     own h for the dropped pairs, which the GPU never computes)."""
     from parity import Taps
     shape = request.getfixturevalue(which)
-    layer, seed = (1, 101) if which == "c1" else (2, 202)
+    layer, seed = {"c1": (1, 101), "v3": (2, 202), "small": (3, 303), "many": (4, 404)}[which]
+    exps = dict(e_lo=116, e_span=5) if layer > 2 else {}  # no h beyond what Q8_0 holds: 0 x inf in the oracle's dropped rows
     E, k, F = shape.n_expert, shape.n_used, shape.ffn
     x, lg = wl.make_inputs(shape, T, 300 + T, zipf=True)
     ids, wts = oracle.route(lg, k, shape.route_mode, norm=True)
@@ -411,7 +428,7 @@ def test_out_of_range_ids_contribute_nothing(request, blk, torch_dev, oracle, wh
     order = np.nonzero(kept)[0][np.argsort(flat[kept], kind="stable")]
     row_of = np.full(T * k, -1)
     row_of[order] = np.arange(len(order))
-    L = oracle_layer(oracle, shape, seed, layer, ids)
+    L = oracle_layer(oracle, shape, seed, layer, ids, **exps)
     ref = L.forward(x, ids, wts0, n_threads=16, taps=True)
 
     def taps(with_shared):  # the last forward's h rows: grouped rows, then the shared expert's from row T*k
@@ -434,8 +451,7 @@ def test_out_of_range_ids_contribute_nothing(request, blk, torch_dev, oracle, wh
 @pytest.mark.parametrize("T", [16, 64])
 def test_graph_replay_grouped(blk, torch_dev, oracle, v3, T):
     """A grouped call captured in a graph (T=16: k_gate_up_o on the 8-row items;
-    T=64: k_gate_up_ol and k_down_ol2 on the 16-row item list): every replay equals
-    the eager call."""
+    T=64: the stacked kernels): every replay equals the eager call."""
     torch, dev = torch_dev
     say("graph capture grouped T", T)
     blk.reserve(v3, T)
@@ -485,33 +501,31 @@ def test_graph_replay_matches_eager(blk, torch_dev, oracle, v3, c1):
 # (H, F, E, k, T, shared, clamp, route): chosen so that each dispatch branch runs at
 # least once off the configs' shapes: decode k_gate_up<1> (narrow) / k_gate_up_bal2
 # (9-task workgroups) / k_gate_up_bal (other task counts); decode down (k_down_dec) at
-# several H / F; pairs (T <= 4); octets with k_gate_up_o and with k_gate_up_ol (P >= 2E,
-# H = 128 * {16, 32, 56}, F without a stacked instance); down on 16-row items with one
-# and two octets (k_down_ol2<6>), k_down_ol<8, 28> and k_down_o (F / 128 without an
-# instance); the stacked-digit kernels (P >= 2E, H = 128 * {16, 32, 48, 56}, F = 128 * {8,
-# 12, 16, 24}: k_gate_up_sk<16, 32, 48, 56>, k_down_sk<8, 12, 16, 24>, with experts of
-# more than 32 rows); shared expert and clamp on and off.
+# several H / F; pairs (T <= 4); octets (k_gate_up_o) with k_down_ol<6, 8, 16, 28> and
+# k_down_o (F / 128 without an instance), experts of one and of several octets; the
+# stacked kernels with f32 sums and experts of more than 32 rows (with f64 sums and
+# 64-row items: STACKED_EDGES); shared expert and clamp on and off.
 SWEEP = [
     (3072, 768, 32, 4, 1, False, 0.0, wl.ROUTE_SOFTMAX),      # decode, narrow: k_gate_up<1>
     (2048, 2048, 64, 8, 1, True, 0.0, wl.ROUTE_SIGMOID),      # decode, 256 workgroups: bal2
     (1024, 2048, 16, 5, 1, False, 4.0, wl.ROUTE_SIGMOID),     # decode, 1280 tasks: k_gate_up_bal
     (1024, 3584, 8, 2, 3, False, 0.0, wl.ROUTE_SOFTMAX),      # pairs, F = 3584
-    (4096, 1024, 64, 6, 32, True, 0.0, wl.ROUTE_SIGMOID),     # stacked: k_gate_up_sk<32>, k_down_sk<8>
-    (2048, 1536, 16, 2, 20, False, 6.0, wl.ROUTE_SOFTMAX),    # stacked: k_gate_up_sk<16>, k_down_sk<12>, 2-3 rows
+    (4096, 1024, 64, 6, 32, True, 0.0, wl.ROUTE_SIGMOID),     # octets, 3 rows per expert, k_down_ol<8>
+    (2048, 1536, 16, 2, 20, False, 6.0, wl.ROUTE_SOFTMAX),    # octets, k_down_o, 2-3 rows
     (1024, 1024, 256, 8, 7, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_gate_up_o, k_down_ol<8>
-    (7168, 768, 16, 4, 9, False, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # ol<56>, 16-row items, k_down_ol2<6>
-    (2048, 3584, 8, 2, 33, True, 8.0, wl.ROUTE_SIGMOID),      # ol<16>, k_down_ol<28>, clamp
+    (7168, 768, 16, 4, 9, False, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets, k_down_ol<6>
+    (2048, 3584, 8, 2, 33, True, 8.0, wl.ROUTE_SIGMOID),      # octets, k_down_ol<28>, clamp
     (5120, 2048, 32, 6, 1, True, 0.0, wl.ROUTE_SIGMOID),      # decode, H = 5120
     (6144, 1024, 16, 4, 1, False, 3.0, wl.ROUTE_SOFTMAX),     # decode, H = 6144, clamp
     (4096, 1024, 16, 4, 64, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 16 rows per expert, shared rows
-    (7168, 768, 8, 4, 40, False, 5.0, wl.ROUTE_SOFTMAX),      # k_down_ol2<6>, 16 + 4-row items, clamp
-    (2048, 2048, 16, 4, 24, True, 0.0, wl.ROUTE_SIGMOID),     # stacked: k_gate_up_sk<16>, k_down_sk<16>
+    (7168, 768, 8, 4, 40, False, 5.0, wl.ROUTE_SOFTMAX),      # octets, k_down_ol<6>, several per expert, clamp
+    (2048, 2048, 16, 4, 24, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_ol<16>
     (2048, 1024, 8, 4, 80, False, 3.0, wl.ROUTE_SOFTMAX),     # stacked, experts of 32 + n rows, clamp
-    (4096, 1280, 16, 4, 32, True, 0.0, wl.ROUTE_SIGMOID),     # ol<32> (F without a stacked instance), k_down_o
-    (7168, 3072, 16, 6, 8, True, 6.0, wl.ROUTE_SQRT_SOFTPLUS),  # stacked: k_down_sk<24> (V4-Pro F), clamp
-    (7168, 3072, 8, 6, 64, True, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # k_down_sk<24>, experts of 48 rows
-    (7168, 1536, 16, 8, 8, True, 0.0, wl.ROUTE_SIGMOID),      # stacked: k_down_sk<12>
-    (6144, 2048, 16, 8, 40, False, 0.0, wl.ROUTE_SIGMOID),    # stacked: k_gate_up_sk<48> (glm-dsa H), 20 rows
+    (4096, 1280, 16, 4, 32, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_o, H = 4096
+    (7168, 3072, 16, 6, 8, True, 6.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets, k_down_o (V4-Pro F), clamp
+    (7168, 3072, 8, 6, 64, True, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # stacked, experts of 48 rows
+    (7168, 1536, 16, 8, 8, True, 0.0, wl.ROUTE_SIGMOID),      # octets, k_down_o, F = 1536
+    (6144, 2048, 16, 8, 40, False, 0.0, wl.ROUTE_SIGMOID),    # stacked (glm-dsa H), 20 rows
 ]
 
 

@@ -121,6 +121,11 @@ def test_gpu_tests_reach_the_kernels_they_name(plan):
         T = sum(first) + rest * (E - len(first))
         kinds = plan([(T, 1, E, H, F, s) for s in (False, True)])
         assert kinds == [("stacked_f32", 64 if E == 128 else 32) if H == 2048 else ("stacked_f64", 32)] * 2, (H, F)
+    # the layers of test_out_of_range_ids_contribute_nothing
+    dropped = plan([(12, 4, 32, 2048, 768, False), (16, 8, 256, 7168, 2048, True), (64, 8, 256, 7168, 2048, True),
+                    (160, 4, 16, 1152, 512, True), (160, 4, 16, 1152, 512, False), (192, 4, 128, 2048, 1024, True)])
+    assert dropped == [("octets", 8), ("octets", 8), ("stacked_f32", 32), ("stacked_f64", 32), ("stacked_f64", 32),
+                       ("stacked_f32", 64)]
     sweep = [c for c in gpu.SWEEP if c[4] > 1]
     kinds = [k for k, _ in plan([(T, k, E, H, F, sh) for H, F, E, k, T, sh, _, _ in sweep])]
     assert {"pairs", "octets", "stacked_f32"} <= set(kinds)
