@@ -22,38 +22,31 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   grouped_plan p;
   const long P = (long)T * k;
   p.octets = T > MOE_PLAN_PAIR_TOKENS;
-  // the stacked kernels add their block sums one by one in f32 on the shapes
-  // that always did (results keep their bits).  The others' results came from
-  // the octet kernels, which err less (their separate digit planes round less
-  // often), so their sums are in f64: 300 tokens on a 5120 x 1536 layer 571 ->
-  // 458 us, rows 4.9e-8 -> 3.6e-8 from 64 bits (f32 group sums 405 us, 7.2e-8)
+  // Order of the stacked kernels' block sums: one by one in f32 on the shapes
+  // that they first ran on (results keep their bits), in f64 on all others,
+  // which came from the octet kernels.  Those err less than f32 in order (their
+  // separate digit planes round less often), so f32 would lose precision there:
+  // rms of output rows from 64 bits, f32 / octets / f64, 0.9-1.3e-7 / 4.1-5.8e-8
+  // / 3.6e-8.  And f64 everywhere costs the first shapes more than the stacked
+  // kernels gained them: V3 layer, 64 and 512 tokens Zipf, 512 and 2048 uniform
+  // 227 -> 301, 680 -> 948, 1136 -> 1342, 2148 -> 3144 us.
   p.in_order = (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
                (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24);
   // A stacked workgroup reads an expert's weights once for up to 32 rows, but
-  // it has twice the rows of weights of an octet workgroup, all of K instead
-  // of half of it, and the same work however few rows its item holds.  So it
-  // wants at least a round of octet workgroups to replace (two per CU, 512;
-  // below that the chip is not full and the shorter workgroup wins), and rows:
-  // 8 per expert with f64 sums (two vector instructions per MFMA value), 5 with
-  // f32 sums (one).  us per layer, cold weights, uniform routing, octets /
-  // stacked:
-  //   5120 x 1536, 8 experts, 2, 8, 16, 32 rows each   33/57  44/58  49/61  70/65
-  //   2048 x 768, 32 experts, 2, 8, 16, 32 rows        28/35  39/43  49/44  70/58
-  //   6400 x 2560, 128 experts, 2, 4, 8, 16 rows       512/575  572/646  734/696  1098/749
-  //   7168 x 2048 (f32), 8 experts, 2, 8, 16 rows      43/64  63/65  78/64
-  //   7168 x 2048 (f32), 128 experts, 2, 4, 8 rows     415/427  496/487  632/532
-  // Large calls run stacked at fewer rows too, since skewed routing, which the
-  // host does not see, gains more there than even routing loses: f32 from 1536
-  // workgroups on (2048 x 3072, 233 experts, 4.5 rows, Zipf 249/141; 2048 x
-  // 2048, 229 experts, 2.6 rows, uniform 235/258), f64 from 3000 and 4 rows on
-  // (random shapes at 4-6 rows: Zipf 22-24% faster, uniform 7-12% slower; at
-  // 2-4 rows, or with 1536-3000 workgroups, the two sides cancel or lose).  The
-  // workgroups are counted for uniform routing, in the launch with fewer.
+  // it has twice the rows of weights of an octet workgroup and all of K instead
+  // of half of it.  Where the octets do not fill the chip (two workgroups per
+  // CU are 512), the shorter workgroup wins, whatever the rows.  The octets'
+  // workgroups are counted for uniform routing, in the launch that has fewer.
+  // us per layer, cold weights, uniform, octets / stacked, and their count:
+  //   5120 x 1536, 8 experts, 2, 16, 32 rows each   33/46  49/61  70/65 (144, 480, 864)
+  //   5120 x 1536, 32 experts, 2, 4, 8 rows         81/88  96/99  116/109 (624, 864, 1344)
+  //   6400 x 2560, 128 experts, 2, 4, 8 rows        512/493  572/539  734/601
+  // With f32 sums the line lies lower (calls keep the bits that they had):
+  //   7168 x 2048, 8 experts, 2, 8, 16 rows         42/65  62/59  78/64 (192, 384, 640)
+  //   2048 x 1024, 8 experts, 8, 16, 32 rows        22/30  28/32  36/34 (192, 320, 576)
   const int gu = F / 64, dn = H / 128;  // octet workgroups per item: k_gate_up_o, k_down_o
   const long n8 = (P / 8 + E / 2 + (shared ? T / 8 : 0)) * (gu < dn ? gu : dn);
-  const bool worth = p.in_order ? n8 >= 512 && (P >= 5L * E || n8 >= 1536)
-                                : n8 >= 640 && (P >= 8L * E || (P >= 4L * E && n8 >= 3000));
-  p.stacked = p.octets && P >= 2L * E && worth;
+  p.stacked = p.octets && P >= 2L * E && n8 >= (p.in_order ? 300 : 512);
   // Two token tiles per weight pair (items of up to 64 rows): a weight is read
   // and duplicated once for both, 2048 tokens on the V3 layer 2308 -> 2134 us,
   // but the workgroups are half as many and run twice as long.  So only where

@@ -28,6 +28,11 @@
 // (a build that staged 96 bytes per block that way: gate/up of 2048 tokens on
 // the V3 layer 2003 us, 1353 us with the same bytes contiguous).
 //
+// Items of up to 16 rows, of which small batches and the remainders of long
+// chunks are made, run the MFMA with its operands swapped (skf_loop): tokens on
+// D's elements, and only the elements of tokens that the item holds are scaled.
+// Items of 33-64 rows share each weight pair between two token tiles (sk_loop2).
+//
 // What bounds them (V3 layer): at 512 tokens, uniform, the weight stream
 // (gate/up 740 us, 712 us with the staging and the scaling left out; the bare
 // stream of the same bytes 560 us); at 2048 tokens the vector issue, 26
@@ -46,10 +51,14 @@
 // gate and up of the same values).
 #pragma once
 
+#include <type_traits>
+
 #include "grouped_plan.h"
 #include "kernels_grouped.h"
 
 typedef double f64x16_t __attribute__((ext_vector_type(16)));
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 #define MOE_SQ_DW 52    // dwords of a quad record
@@ -614,6 +623,175 @@ __device__ __forceinline__ void sk_loop2(const skw &w, const uint32_t *src, int 
   sk_fma2(acc[1][1], g.du, g.r[1]);
 }
 
+// ---------------------------------------------------------------------------
+// The same for items of at most 8 * NG rows, with the MFMA's operands swapped
+// (their lane layouts are alike): tokens are the A rows and weight rows the B
+// columns, so D lane n + 32*g holds weight row n, tokens 8i + 4g + j at element
+// 4i + j, and only the 4 * NG elements of tokens that the item can hold are
+// scaled, each by its own token's d (broadcast reads from LDS, a pair ahead):
+// 4 or 8 scaling FMAs per MFMA instead of 16, in f64 10 or 20 instructions
+// instead of 32.  The block sums and their order are those of sk_loop: the same
+// bits.  us per layer, cold weights, 2, 4, 8 rows per expert: 5120 x 1536 (f64),
+// 128 experts, 292 -> 251, 315 -> 283, 348 -> 313; 7168 x 2048, 32 experts, 137
+// -> 132, 168 -> 160, 172 -> 163.  NG = 3 does not fit the registers of two
+// waves per SIMD (spills; 2-14% slower than scaling all 16 elements).
+template <int NG>
+struct skringf {
+  u32x4_t w[MOE_SK_RP][2];
+  uint32_t e[2][4];
+  uint32_t scn[2][2];
+  skb b[2];
+  f32x2_t d[2][4 * NG];  // d of this pair's two blocks and of the next pair's
+  f32x16_t r[2];
+  float du[4 * NG];      // d of stream 1's pending block
+};
+
+template <int NG>
+__device__ __forceinline__ void load_skfd(f32x2_t (&d)[4 * NG], const uint32_t *buf, int lane, int q, int j) {
+  const uint32_t *p = buf + (4 * (lane >> 5) + q * MOE_SK_ROWS) * MOE_SQ_DW + 48 + 2 * j;
+#pragma unroll
+  for (int i = 0; i < 4 * NG; i++)
+    d[i] = *reinterpret_cast<const f32x2_t *>(p + (8 * (i >> 2) + (i & 3)) * MOE_SQ_DW);
+}
+
+template <bool WIDE, int NG>
+__device__ __forceinline__ void skf_scale(f32x4_t (&acc)[NG], f64x4_t (&wide)[NG], const float (&d)[4 * NG],
+                                          const f32x16_t &r) {
+#pragma unroll
+  for (int i = 0; i < 4 * NG; i++) {
+    if constexpr (WIDE) wide[i >> 2][i & 3] = __builtin_fma((double)d[i], (double)r[i], wide[i >> 2][i & 3]);
+    else acc[i >> 2][i & 3] = __builtin_fmaf(d[i], r[i], acc[i >> 2][i & 3]);
+  }
+#pragma unroll
+  for (int i = 0; i < NG; i++) {
+    if constexpr (WIDE) asm volatile("" : "+v"(wide[i]));
+    else asm volatile("" : "+v"(acc[i]));
+  }
+}
+
+template <int SEL, int J, int JD, bool WIDE, int NG>
+__device__ __forceinline__ void skf_block(skringf<NG> &g, const u32x4_t &w0, const u32x4_t &w1, const skb &b,
+                                          const f32x2_t (&dp)[4 * NG], int sb, f32x4_t (&acc)[2][NG],
+                                          f64x4_t (&wide)[2][NG]) {
+  const i32x8_t x = b.x[J];
+  const i32x8_t a0 = {(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w, 0, 0, 0, 0};
+  const i32x8_t a1 = {(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w, 0, 0, 0, 0};
+  const f32x16_t z = {};
+  float d[4 * NG];
+#pragma unroll
+  for (int i = 0; i < 4 * NG; i++) d[i] = dp[i][J];
+  g.r[0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, a0, z, 2, 4, 0, sb, SEL, (int)g.e[0][JD]);
+  __builtin_amdgcn_sched_barrier(0);
+  skf_scale<WIDE, NG>(acc[1], wide[1], g.du, g.r[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  g.r[1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, a1, z, 2, 4, 0, sb, SEL, (int)g.e[1][JD]);
+  __builtin_amdgcn_sched_barrier(0);
+  skf_scale<WIDE, NG>(acc[0], wide[0], d, g.r[0]);
+#pragma unroll
+  for (int i = 0; i < 4 * NG; i++) g.du[i] = d[i];
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Pair SG of group G: waits and barrier as in sk_pair.
+template <int CPOL, bool WIDE, int NG, int SG>
+__device__ __forceinline__ void skf_pair(skringf<NG> &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane,
+                                         int sb, int G, f32x4_t (&acc)[2][NG], f64x4_t (&wide)[2][NG]) {
+  load_skw<CPOL>(g.w[(SG + MOE_SK_RP - 1) % MOE_SK_RP], w, G * 8 + SG + MOE_SK_RP - 1);
+  if constexpr (SG == 0) load_sksc(g.scn, w, G + 1);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (SG == 7) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(8 * 2 + 4));
+    lds_barrier();
+    sdma_issue(st, lds + cur * MOE_SK_BUF_DW, G + MOE_SK_NBUF);
+    cur ^= 1;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const uint32_t *buf = lds + cur * MOE_SK_BUF_DW;
+  constexpr int nq = ((SG + 1) & 7) >> 1, nj = (SG + 1) & 1;  // the next pair's quad of its chunk
+  g.b[nj] = load_skb(buf, lane, nq, nj);
+  load_skfd<NG>(g.d[nj], buf, lane, nq, nj);
+  u32x4_t a[2][2];
+#pragma unroll
+  for (int s = 0; s < 2; s++) dup_halves(g.w[SG % MOE_SK_RP][s], a[s][0], a[s][1]);
+  __builtin_amdgcn_sched_barrier(0);
+  constexpr int j = SG & 1;
+  skf_block<(SG >> 1), 0, 2 * j, WIDE, NG>(g, a[0][0], a[1][0], g.b[j], g.d[j], sb, acc, wide);
+  skf_block<(SG >> 1), 1, 2 * j + 1, WIDE, NG>(g, a[0][1], a[1][1], g.b[j], g.d[j], sb, acc, wide);
+}
+
+template <int CPOL, bool WIDE, int NG, int SG>
+__device__ __forceinline__ void skf_group(skringf<NG> &g, const skw &w, const sdma &st, uint32_t *lds, int &cur, int lane,
+                                          int sb, int G, int quads, f32x4_t (&acc)[2][NG], f64x4_t (&wide)[2][NG]) {
+  if constexpr (SG < 8) {
+    if (quads <= (SG >> 1)) return;
+    skf_pair<CPOL, WIDE, NG, SG>(g, w, st, lds, cur, lane, sb, G, acc, wide);
+    skf_group<CPOL, WIDE, NG, SG + 1>(g, w, st, lds, cur, lane, sb, G, quads, acc, wide);
+  }
+}
+
+// acc[s][i]: lane n + 32*g, element j = row n of stream s, token 8i + 4g + j.
+template <int CPOL, bool WIDE, int NG, bool QUAD_MAJOR, class ROW>
+__device__ __forceinline__ void skf_loop(const skw &w, const uint32_t *src, int n_src, int NQ, ROW row, uint32_t *lds,
+                                         int lane, int wave, f32x4_t (&acc)[2][NG]) {
+  skringf<NG> g;
+  uint32_t sc[2][2];
+  f64x4_t wide[2][NG];
+  load_sksc(sc, w, 0);
+#pragma unroll
+  for (int i = 0; i + 1 < MOE_SK_RP; i++) load_skw<CPOL>(g.w[i], w, i);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  const sdma st = make_sdma<32>(src, n_src, NQ, QUAD_MAJOR, row(0), 0, lane, wave);
+#pragma unroll
+  for (int c = 0; c < MOE_SK_NBUF; c++) sdma_issue(st, lds + c * MOE_SK_BUF_DW, c);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(MOE_SK_WDMA - 1));  // chunk 0 has landed, the second may be on its way
+  lds_barrier();
+  int cur = 0;
+  g.b[0] = load_skb(lds, lane, 0, 0);
+  load_skfd<NG>(g.d[0], lds, lane, 0, 0);
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int i = 0; i < NG; i++) {
+      acc[s][i] = f32x4_t{};
+      wide[s][i] = f64x4_t{};
+    }
+  g.r[1] = f32x16_t{};  // the first block scales a zero result: acc stays +0
+#pragma unroll
+  for (int i = 0; i < 4 * NG; i++) g.du[i] = 0.0f;
+  const int sb = (lane >> 5) ? 130 : 134;
+  auto group = [&](int G, int quads) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      dup_halves1(sc[s][0], g.e[s][0], g.e[s][1]);
+      dup_halves1(sc[s][1], g.e[s][2], g.e[s][3]);
+    }
+    skf_group<CPOL, WIDE, NG, 0>(g, w, st, lds, cur, lane, sb, G, quads, acc, wide);
+  };
+  int G = 0;
+#pragma unroll 1
+  for (; 4 * G + 4 <= NQ; G++) {
+    group(G, 4);
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) sc[s][j] = g.scn[s][j];
+  }
+  if constexpr (WIDE)
+    if (4 * G < NQ) group(G, NQ - 4 * G);
+  skf_scale<WIDE, NG>(acc[1], wide[1], g.du, g.r[1]);
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int i = 0; i < 4 * NG; i++) acc[s][i >> 2][i & 3] = (float)wide[s][i >> 2][i & 3];
+  }
+}
+
 // The chunk buffers are free for an epilogue: the chunks issued past the end
 // (zeros) have landed, and every wave has read its last operands.
 __device__ __forceinline__ void sk_lds_free() {
@@ -638,7 +816,7 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
   const int NQ = H / 128, NG = moe_nq4(NQ), tiles = F / MOE_TILE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int P = T * k, row0 = it.y, nt = it.z;
-  const bool shared = (it.w & MOE_ITEM_SHARED) != 0;
+  const bool shared = (it.w & MOE_ITEM_SHARED) != 0, split = (it.w & MOE_ITEM_SPLIT) != 0;
   const int u = MOE_SK_WAVES * blockIdx.x + wave, n = lane & 31, gb = lane >> 5;
   const size_t rec = ((size_t)it.x * tiles + 2 * u) * NG * MOE_REC_BYTES;
   auto row = [&](int t0) { return t0 + n < nt ? (shared ? row0 + t0 + n - P : perm[row0 + t0 + n] / k) : -1; };
@@ -655,9 +833,31 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
         htap[(size_t)(row0 + t0 + n) * F + (size_t)u * MOE_UNIT + 8 * (i >> 2) + 4 * gb + (i & 3)] = h[i];
     }
   };
+  // the same after skf_loop, lanes = rows of F: h by token in LDS, quantized
+  // from there
+  auto finish_few = [&](auto &acc, auto ng) {
+    constexpr int NG_ = decltype(ng)::value;
+    float *hb = reinterpret_cast<float *>(lds + MOE_SK_ROWS * MOE_SQ_DW);  // [token][128], behind the records
+#pragma unroll
+    for (int i = 0; i < 4 * NG_; i++) {
+      const int t = 8 * (i >> 2) + 4 * gb + (i & 3);
+      const float h = swiglu(acc[0][i >> 2][i & 3], acc[1][i >> 2][i & 3], clamp);
+      hb[t * 128 + MOE_UNIT * wave + n] = h;
+      if (htap && t < nt) htap[(size_t)(row0 + t) * F + (size_t)u * MOE_UNIT + n] = h;
+    }
+    __syncthreads();
+    stage_quant_quads(hb, 4 * nt, lds, threadIdx.x, 64 * MOE_SK_WAVES);
+  };
+  auto few = [&](auto ng) {
+    constexpr int NG_ = decltype(ng)::value;
+    f32x4_t acc[2][NG_];
+    if (split) skf_loop<0, WIDE, NG_, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    else skf_loop<MOE_CPOL_NT, WIDE, NG_, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
+    sk_lds_free();
+    finish_few(acc, ng);
+  };
   // an expert of one item reads its tiles once: non-temporal, as in decode;
   // the items of a larger expert share them through L2
-  const bool split = (it.w & MOE_ITEM_SPLIT) != 0;
   // the 4 waves' blocks meet as whole records in LDS, and the item's records
   // of this quad leave as one run (stored from the waves in 24-byte pieces they
   // cost the weight stream 27 of 730 us at 512 tokens)
@@ -668,6 +868,10 @@ void k_gate_up_sk(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w
     sk_lds_free();
     finish(acc[0][0], acc[0][1], 0);
     finish(acc[1][0], acc[1][1], 32);
+  } else if (nt <= 8) {
+    few(std::integral_constant<int, 1>{});
+  } else if (nt <= 16) {
+    few(std::integral_constant<int, 2>{});
   } else {
     f32x16_t acc[2];
     if (split) sk_loop<0, WIDE, false>(w, xs, T, NQ, row, lds, lane, wave, acc);
@@ -705,6 +909,14 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
   const skw w = make_skw(w0, w0 + (size_t)2 * NG * MOE_REC_BYTES, NQ, lane);
   const int col = 256 * blockIdx.x + 4 * lane;
   // the rows of tokens t0 .. t0 + 31, 256 columns each, meet in LDS and leave as runs of 1 KiB
+  auto store_rows = [&](int t0) {
+    __syncthreads();
+    const float *red = reinterpret_cast<const float *>(lds);
+    if (col < H)
+      for (int t = wave; t < 32 && t0 + t < nt; t += MOE_SK_WAVES)
+        *reinterpret_cast<f32x4_t *>(y + (size_t)(row0 + t0 + t) * H + col) =
+            *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
+  };
   auto finish = [&](const f32x16_t &a0, const f32x16_t &a1, int t0) {
     const bool live = t0 + n < nt;
     const float wt = live && !shared ? wts[perm[row0 + t0 + n]] : 1.0f;
@@ -720,19 +932,42 @@ void k_down_sk(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
         for (int j = 0; j < 4; j++) v[j] = shared ? a[4 * i + j] : __fmul_rn(a[4 * i + j], wt);
         *reinterpret_cast<f32x4_t *>(red + n * MOE_SK_YST + 64 * wave + 32 * s + 8 * i + 4 * gb) = v;
       }
-    __syncthreads();
-    if (col < H)
-      for (int t = wave; t < 32 && t0 + t < nt; t += MOE_SK_WAVES)
-        *reinterpret_cast<f32x4_t *>(y + (size_t)(row0 + t0 + t) * H + col) =
-            *reinterpret_cast<const f32x4_t *>(red + t * MOE_SK_YST + 4 * lane);
+    store_rows(t0);
   };
   const bool split = (it.w & MOE_ITEM_SPLIT) != 0;
+  // items of up to 16 tokens, lanes = rows of H
+  auto few = [&](auto ng) {
+    constexpr int NG_ = decltype(ng)::value;
+    f32x4_t acc[2][NG_];
+    if (split) skf_loop<0, WIDE, NG_, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    else skf_loop<MOE_CPOL_NT, WIDE, NG_, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
+    float wt[4 * NG_];
+#pragma unroll
+    for (int i = 0; i < 4 * NG_; i++) {
+      const int t = 8 * (i >> 2) + 4 * gb + (i & 3);
+      wt[i] = t < nt && !shared ? wts[perm[row0 + t]] : 1.0f;
+    }
+    sk_lds_free();
+    float *red = reinterpret_cast<float *>(lds);
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int i = 0; i < 4 * NG_; i++) {
+        const float a = acc[s][i >> 2][i & 3];
+        red[(8 * (i >> 2) + 4 * gb + (i & 3)) * MOE_SK_YST + 64 * wave + 32 * s + n] = shared ? a : __fmul_rn(a, wt[i]);
+      }
+    store_rows(0);
+  };
   if (!WIDE && nt > MOE_SK_ROWS) {
     f32x16_t acc[2][2];
     if (split) sk_loop2<0, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
     else sk_loop2<MOE_CPOL_NT, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);
     finish(acc[0][0], acc[0][1], 0);
     finish(acc[1][0], acc[1][1], 32);
+  } else if (nt <= 8) {
+    few(std::integral_constant<int, 1>{});
+  } else if (nt <= 16) {
+    few(std::integral_constant<int, 2>{});
   } else {
     f32x16_t acc[2];
     if (split) sk_loop<0, WIDE, true>(w, hs, n_rows, NQ, row, lds, lane, wave, acc);

@@ -503,14 +503,14 @@ def test_graph_replay_matches_eager(blk, torch_dev, oracle, v3, c1):
 # (9-task workgroups) / k_gate_up_bal (other task counts); decode down (k_down_dec) at
 # several H / F; pairs (T <= 4); octets (k_gate_up_o) with k_down_ol<6, 8, 16, 28> and
 # k_down_o (F / 128 without an instance), experts of one and of several octets; the
-# stacked kernels with f32 sums and experts of more than 32 rows (with f64 sums and
-# 64-row items: STACKED_EDGES); shared expert and clamp on and off.
+# stacked kernels with f32 and f64 sums, experts of a few and of more than 32 rows
+# (64-row items: STACKED_EDGES); shared expert and clamp on and off.
 SWEEP = [
     (3072, 768, 32, 4, 1, False, 0.0, wl.ROUTE_SOFTMAX),      # decode, narrow: k_gate_up<1>
     (2048, 2048, 64, 8, 1, True, 0.0, wl.ROUTE_SIGMOID),      # decode, 256 workgroups: bal2
     (1024, 2048, 16, 5, 1, False, 4.0, wl.ROUTE_SIGMOID),     # decode, 1280 tasks: k_gate_up_bal
     (1024, 3584, 8, 2, 3, False, 0.0, wl.ROUTE_SOFTMAX),      # pairs, F = 3584
-    (4096, 1024, 64, 6, 32, True, 0.0, wl.ROUTE_SIGMOID),     # octets, 3 rows per expert, k_down_ol<8>
+    (4096, 1024, 64, 6, 32, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 3 rows per expert
     (2048, 1536, 16, 2, 20, False, 6.0, wl.ROUTE_SOFTMAX),    # octets, k_down_o, 2-3 rows
     (1024, 1024, 256, 8, 7, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_gate_up_o, k_down_ol<8>
     (7168, 768, 16, 4, 9, False, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets, k_down_ol<6>
@@ -519,13 +519,14 @@ SWEEP = [
     (6144, 1024, 16, 4, 1, False, 3.0, wl.ROUTE_SOFTMAX),     # decode, H = 6144, clamp
     (4096, 1024, 16, 4, 64, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 16 rows per expert, shared rows
     (7168, 768, 8, 4, 40, False, 5.0, wl.ROUTE_SOFTMAX),      # octets, k_down_ol<6>, several per expert, clamp
-    (2048, 2048, 16, 4, 24, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_ol<16>
+    (2048, 2048, 16, 4, 24, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 6 rows per expert
     (2048, 1024, 8, 4, 80, False, 3.0, wl.ROUTE_SOFTMAX),     # stacked, experts of 32 + n rows, clamp
-    (4096, 1280, 16, 4, 32, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_o, H = 4096
-    (7168, 3072, 16, 6, 8, True, 6.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets, k_down_o (V4-Pro F), clamp
+    (4096, 1280, 16, 4, 32, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, sums in f64, 8 rows per expert
+    (7168, 3072, 16, 6, 8, True, 6.0, wl.ROUTE_SQRT_SOFTPLUS),  # stacked (V4-Pro F), 3 rows per expert, clamp
     (7168, 3072, 8, 6, 64, True, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # stacked, experts of 48 rows
-    (7168, 1536, 16, 8, 8, True, 0.0, wl.ROUTE_SIGMOID),      # octets, k_down_o, F = 1536
+    (7168, 1536, 16, 8, 8, True, 0.0, wl.ROUTE_SIGMOID),      # stacked, 4 rows per expert
     (6144, 2048, 16, 8, 40, False, 0.0, wl.ROUTE_SIGMOID),    # stacked (glm-dsa H), 20 rows
+    (2048, 2048, 16, 4, 10, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_ol<16>
 ]
 
 
@@ -831,6 +832,8 @@ STACKED_EDGES = [
     (640, 384, 16, (64, 65, 0, 15), 70),     # K of 5 and 3 quads: a partial last group; the last 256 rows of H half there
     (1152, 512, 16, (8, 16, 17, 96), 40),    # K of 9 quads and of one whole group
     (256, 128, 64, (40, 2, 33, 9), 38),      # K below one group
+    (2048, 1024, 128, (7, 8, 9, 15, 16, 17, 24, 25), 4),  # items around 8 and 16 rows: operands swapped
+    (640, 384, 64, (1, 7, 8, 9, 15, 16, 17, 24), 13),     # the same with sums in f64
 ]
 
 
