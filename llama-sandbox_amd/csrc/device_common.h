@@ -58,6 +58,14 @@ __device__ __forceinline__ float dpp_f(float v) {
       0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // Sum over 16-lane rows, every lane of a row gets its row's sum.
 __device__ __forceinline__ float row16_sum(float v) {
   v += dpp_f<0xB1>(v);  // quad_perm [1,0,3,2]

@@ -15,6 +15,7 @@ struct grouped_plan {
   bool octets;    // T > 4
   bool stacked;   // octets, but on the stacked kernels
   bool in_order;  // stacked: sums block by block in f32 (else in f64)
+  bool octet_f64; // octets with sums in f64 (else in f32)
   int item_rows;
 };
 
@@ -47,6 +48,11 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   const int gu = F / 64, dn = H / 128;  // octet workgroups per item: k_gate_up_o, k_down_o
   const long n8 = (P / 8 + E / 2 + (shared ? T / 8 : 0)) * (gu < dn ? gu : dn);
   p.stacked = p.octets && P >= 2L * E && n8 >= (p.in_order ? 300 : 512);
+  // Shapes that sum in f64 do so on octets too, from 2 pairs per expert on: the
+  // same rows, bit for bit, as in a larger call.  It costs 3-6% (8 tokens on 5120
+  // x 1536, 8 experts 33.2 -> 34.7 us; 32 tokens on 32 experts 95.6 -> 97.9 us;
+  // 2048 x 768, 8-12%).
+  p.octet_f64 = p.octets && !p.stacked && !p.in_order && P >= 2L * E;
   // Two token tiles per weight pair (items of up to 64 rows): a weight is read
   // and duplicated once for both, 2048 tokens on the V3 layer 2308 -> 2134 us,
   // but the workgroups are half as many and run twice as long.  So only where

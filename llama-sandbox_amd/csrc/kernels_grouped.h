@@ -488,6 +488,19 @@ __global__ __launch_bounds__(64 * MOE_DF_WAVES) void k_down_few(
 // dword.
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef double f64x16_t __attribute__((ext_vector_type(16)));
+
+// Accumulator of an octet kernel.
+template <bool WIDE>
+struct octet_acc {
+  typedef f32x16_t vec;
+  typedef float val;
+};
+template <>
+struct octet_acc<true> {
+  typedef f64x16_t vec;
+  typedef double val;
+};
 
 // A 32-row tile: 16-row tiles tile16 and tile16 + 1 of the tensor.
 __device__ __forceinline__ wstream make_wstream32(const uint8_t *w, size_t tile16, int NG) {
@@ -565,9 +578,16 @@ __device__ __forceinline__ void load_bq32(bq32<NO> &b, const gsrc &src, const gs
     }
 }
 
-template <int SEL, int NW, int NO>
+// acc += d * r: AV f32x16_t, or f64x16_t for sums in f64.
+__device__ __forceinline__ void octet_scale(f32x16_t &acc, float d, const f32x16_t &r) { acc = acc + d * r; }
+__device__ __forceinline__ void octet_scale(f64x16_t &acc, float d, const f32x16_t &r) {
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = __builtin_fma((double)d, (double)r[e], acc[e]);
+}
+
+template <int SEL, int NW, int NO, class AV>
 __device__ __forceinline__ void quad_mma32(const wq32<NW> &w, const uint32_t (&sc)[NW][2], const bq32<NO> &b,
-                                           bool upper, int sb, f32x16_t (&acc)[NO][NW]) {
+                                           bool upper, int sb, AV (&acc)[NO][NW]) {
 #pragma unroll
   for (int o = 0; o < NO; o++)
 #pragma unroll
@@ -584,7 +604,7 @@ __device__ __forceinline__ void quad_mma32(const wq32<NW> &w, const uint32_t (&s
 #pragma unroll
         for (int e = 0; e < 16; e++) z[e] = 0.0f;
         const f32x16_t r = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, bv, z, 4, 0, SEL, (int)sc[i][j], 0, sb);
-        acc[o][i] = acc[o][i] + b.d[o][j] * r;
+        octet_scale(acc[o][i], b.d[o][j], r);
       }
     }
 #pragma unroll
@@ -610,10 +630,10 @@ struct oring {
 // One quad of the loop: issue B for quad qB into slot SLOT+2 and weights
 // for quad qW into slot SLOT+3 (if wanted), then multiply slot SLOT with
 // exponent group G (op_sel SEL = quad % 4).
-template <int SEL, int SLOT, int G, bool WB, bool WW, int NW, int NO, int NG, int CPOL>
+template <int SEL, int SLOT, int G, bool WB, bool WW, int NW, int NO, int NG, int CPOL, class AV>
 __device__ __forceinline__ void ostep(oring<NW, NO, NG> &r, const wstream (&ws)[NW], const aoff32 &ao,
                                       const gsrc &src, const gsel (&gs)[NO], int qB, int qW, bool upper, int sb,
-                                      f32x16_t (&acc)[NO][NW]) {
+                                      AV (&acc)[NO][NW]) {
   if constexpr (WB) load_bq32<NO>(r.b[(SLOT + 2) & 3], src, gs, qB);
   if constexpr (WW) load_wq32<NW, CPOL>(r.w[(SLOT + 3) & 3], ws, ao, qW);
   asm volatile("" ::: "memory");
@@ -622,10 +642,10 @@ __device__ __forceinline__ void ostep(oring<NW, NO, NG> &r, const wstream (&ws)[
 }
 
 // Quads QL .. NQW-1 of a fully unrolled loop from q0 (q0 % 4 == 0).
-template <int QL, int NQW, int NW, int NO, int NG, int CPOL>
+template <int QL, int NQW, int NW, int NO, int NG, int CPOL, class AV>
 __device__ __forceinline__ void ofixed_from(oring<NW, NO, NG> &r, const wstream (&ws)[NW], const aoff32 &ao,
                                             int q0, const gsrc &src, const gsel (&gs)[NO], bool upper, int sb,
-                                            f32x16_t (&acc)[NO][NW]) {
+                                            AV (&acc)[NO][NW]) {
   if constexpr (QL < NQW) {
     if constexpr ((QL & 3) == 0 && (QL >> 2) + 1 < NG) load_sc32<NW>(r.sc[(QL >> 2) + 1], ws, ao, (q0 >> 2) + (QL >> 2) + 1);
     ostep<QL & 3, QL & 3, QL / 4, (QL + 2 < NQW), (QL + 3 < NQW), NW, NO, NG, CPOL>(
@@ -636,15 +656,15 @@ __device__ __forceinline__ void ofixed_from(oring<NW, NO, NG> &r, const wstream 
 
 // K loop over NQW quads from q0 (q0 % 4 == 0), fully unrolled; the rings
 // as in gloop_fixed (B 2 quads ahead, weights 3 quads ahead).
-template <int NW, int NO, int CPOL, int NQW>
+template <int NW, int NO, int CPOL, int NQW, class AV>
 __device__ __forceinline__ void oloop_fixed(const wstream (&ws)[NW], const aoff32 &ao, int q0, const gsrc &src,
-                                            const gsel (&gs)[NO], int lane, f32x16_t (&acc)[NO][NW]) {
+                                            const gsel (&gs)[NO], int lane, AV (&acc)[NO][NW]) {
 #pragma unroll
   for (int o = 0; o < NO; o++)
 #pragma unroll
     for (int i = 0; i < NW; i++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[o][i][e] = 0.0f;
+      for (int e = 0; e < 16; e++) acc[o][i][e] = 0;
   constexpr int NG = (NQW + 3) / 4;
   const bool upper = lane_upper32(lane);
   const int sb = lane_bscale32(lane);
@@ -662,16 +682,16 @@ __device__ __forceinline__ void oloop_fixed(const wstream (&ws)[NW], const aoff3
 
 // Run-time number of quads [q0, q1): windows of 4 quads, loads past the
 // end re-read the last quad, guarded tail.
-template <int NW, int NO, int CPOL>
+template <int NW, int NO, int CPOL, class AV>
 __device__ __forceinline__ void oloop_rolled(const wstream (&ws)[NW], const aoff32 &ao, int q0, int q1,
                                              const gsrc &src, const gsel (&gs)[NO], int lane,
-                                             f32x16_t (&acc)[NO][NW]) {
+                                             AV (&acc)[NO][NW]) {
 #pragma unroll
   for (int o = 0; o < NO; o++)
 #pragma unroll
     for (int i = 0; i < NW; i++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[o][i][e] = 0.0f;
+      for (int e = 0; e < 16; e++) acc[o][i][e] = 0;
   if (q1 <= q0) return;
   const bool upper = lane_upper32(lane);
   const int sb = lane_bscale32(lane);
@@ -703,10 +723,10 @@ __device__ __forceinline__ void oloop_rolled(const wstream (&ws)[NW], const aoff
   if (qb + 2 < q1) ostep<2, 2, 0, true, true, NW, NO, 1, CPOL>(r, ws, ao, src, gs, qc(qb + 4), qc(qb + 5), upper, sb, acc);
 }
 
-template <int NW, int NO, int CPOL>
+template <int NW, int NO, int CPOL, class AV>
 __device__ __forceinline__ void oloop_any(const wstream (&ws)[NW], const aoff32 &ao, int q0, int q1,
                                           const gsrc &src, const gsel (&gs)[NO], int lane,
-                                          f32x16_t (&acc)[NO][NW]) {
+                                          AV (&acc)[NO][NW]) {
   switch (q1 - q0) {
     case 28: oloop_fixed<NW, NO, CPOL, 28>(ws, ao, q0, src, gs, lane, acc); break;
     case 16: oloop_fixed<NW, NO, CPOL, 16>(ws, ao, q0, src, gs, lane, acc); break;
@@ -723,18 +743,27 @@ __device__ __forceinline__ float col4_sum(float v) {
   v += dpp_f<0x4E>(v);  // lane ^ 2
   return v;
 }
+__device__ __forceinline__ double col4_sum(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  return v;
+}
 
 // Grouped gate/up on octets: one workgroup of 4 waves per (2 units of F,
 // item of <= 8 rows): wave w streams unit 2*blockIdx.x + w%2 (gate and up,
 // 32 rows each) over K-half w/2; the K-halves meet in LDS; then each
 // 32-lane half of a wave takes one (unit, token), applies clamp + SwiGLU and
 // writes the unit's Q8_0 h block of that token.  grid (F/64, item capacity).
+// WIDE: sums in f64, rounded once.
+template <bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_gate_up_o(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_u, const uint32_t *__restrict__ xq,
                  const float *__restrict__ xd, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
                  int k, int T, int F, int H, float clamp, uint32_t *__restrict__ hs, float *__restrict__ hd,
                  float *__restrict__ htap) {
-  __shared__ __align__(16) float red[4][2][8][MOE_UNIT];  // [wave][gate/up][token][row]
+  typedef typename octet_acc<WIDE>::vec AV;
+  typedef typename octet_acc<WIDE>::val val;
+  __shared__ __align__(16) val red[4][2][8][MOE_UNIT];  // [wave][gate/up][token][row]
   if ((int)blockIdx.y >= items[0]) return;
   const int4 it = item_of(items, blockIdx.y);
   const int NQ = H / 128, NQ4 = moe_nq4(NQ), U = F / MOE_UNIT, tiles = F / MOE_TILE, KB = H / MOE_QK;
@@ -756,7 +785,7 @@ void k_gate_up_o(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_
     if (i < nt) xr = shared ? row0 + i - P : perm[row0 + i] / k;
     gs[0] = make_gsel32(lane, xr, KB);
   }
-  f32x16_t acc[1][2];
+  AV acc[1][2];
   // non-temporal weights where no other item of the expert reads them
   if (it.w & MOE_ITEM_SPLIT) oloop_any<2, 1, 0>(ws, ao, q0, q1, src, gs, lane, acc);
   else oloop_any<2, 1, MOE_CPOL_NT>(ws, ao, q0, q1, src, gs, lane, acc);
@@ -765,7 +794,7 @@ void k_gate_up_o(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int e = 0; e < 16; e++) {
-      const float v = col4_sum(acc[0][i][e]);
+      const val v = col4_sum(acc[0][i][e]);
       if ((n & 3) == 0) red[wave][i][n >> 2][8 * (e >> 2) + 4 * gb + (e & 3)] = v;
     }
   __syncthreads();
@@ -776,8 +805,8 @@ void k_gate_up_o(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_
     const int ul2 = c >> 3, t = c & 7, j = lane & 31;
     const bool live = t < nt;
     // waves ul2 (K-half 0) and ul2 + 2 (K-half 1) hold this unit
-    const float gsum = red[ul2][0][t][j] + red[ul2 + 2][0][t][j];
-    const float usum = red[ul2][1][t][j] + red[ul2 + 2][1][t][j];
+    const float gsum = (float)(red[ul2][0][t][j] + red[ul2 + 2][0][t][j]);
+    const float usum = (float)(red[ul2][1][t][j] + red[ul2 + 2][1][t][j]);
     const float h = live ? swiglu(gsum, usum, clamp) : 0.0f;
     const int hrow = row0 + (live ? t : 0), uu = 2 * blockIdx.x + ul2;
     h_unit_store(h, live, hs + ((size_t)hrow * U + uu) * MOE_XSW, hd + (size_t)hrow * U + uu, lane);
@@ -788,7 +817,8 @@ void k_gate_up_o(const uint8_t *__restrict__ w_g, const uint8_t *__restrict__ w_
 // Grouped down on octets: each wave streams one 32-row tile of H of the
 // item's down matrix over all of F against the item's (<= 8) h rows;
 // y[r][H] = (row . h[r]) * wts[perm[r]] (routed) or * 1 (shared).
-// grid (H/128, item capacity), 4 waves.
+// grid (H/128, item capacity), 4 waves.  WIDE as in k_gate_up_o.
+template <bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_down_o(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, const float *__restrict__ hd,
               int n_rows, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
@@ -805,7 +835,7 @@ void k_down_o(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, 
   const gsrc src = make_gsrc(hs, hd, n_rows, KB);
   const int n = lane & 31, gb = lane >> 5, t = n >> 2;
   gsel gs[1] = {make_gsel32(lane, t < nt ? row0 + t : -1, KB)};
-  f32x16_t acc[1][1];
+  typename octet_acc<WIDE>::vec acc[1][1];
   oloop_any<1, 1, 0>(ws, ao, 0, NQ, src, gs, lane, acc);
   const bool live = t < nt;
   const int r = row0 + (live ? t : 0);
@@ -813,7 +843,7 @@ void k_down_o(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, 
   float v[16];
 #pragma unroll
   for (int e = 0; e < 16; e++) {
-    v[e] = col4_sum(acc[0][0][e]);
+    v[e] = (float)col4_sum(acc[0][0][e]);
     if (!shared) v[e] = __fmul_rn(v[e], wt);
   }
   if ((n & 3) == 0 && live) {
@@ -890,10 +920,10 @@ __device__ __forceinline__ void oprime_l(oring_l<NW, NO, NG> &r, const wstream (
   if (NQW > 2) load_wq32<NW, CPOL>(r.w[2], ws, ao, 2);
 }
 
-template <int QL, int NQW, int NW, int NO, int NG, int CPOL, int OB, int OD>
+template <int QL, int NQW, int NW, int NO, int NG, int CPOL, int OB, int OD, class AV>
 __device__ __forceinline__ void olfixed_from(oring_l<NW, NO, NG> &r, const wstream (&ws)[NW], const aoff32 &ao,
                                              const u32x4_t *bl, const float *dl, int lane, int dlo, bool upper,
-                                             int sb, f32x16_t (&acc)[NO][NW]) {
+                                             int sb, AV (&acc)[NO][NW]) {
   if constexpr (QL < NQW) {
     if constexpr ((QL & 3) == 0 && (QL >> 2) + 1 < NG) load_sc32<NW>(r.sc[(QL >> 2) + 1], ws, ao, (QL >> 2) + 1);
     if constexpr (QL + 1 < NQW) load_bq32_lds<NO, OB, OD>(r.b[(QL + 1) & 1], bl, dl, lane, dlo, QL + 1);
@@ -908,8 +938,8 @@ __device__ __forceinline__ void olfixed_from(oring_l<NW, NO, NG> &r, const wstre
 // Grouped down on octets with B in LDS: k_down_o's work split (each wave one
 // 32-row tile of H over all of F, y = (row . h) * router weight), NQ = F/128
 // in {6, 8, 16, 28}.  grid (H/128, item capacity), 4 waves, LDS
-// octet_lds_bytes(F/32).
-template <int NQ>
+// octet_lds_bytes(F/32).  WIDE as in k_gate_up_o.
+template <int NQ, bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_down_ol(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs, const float *__restrict__ hd,
                int n_rows, const int32_t *__restrict__ items, const int32_t *__restrict__ perm,
@@ -935,9 +965,9 @@ void k_down_ol(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
   __syncthreads();
   const int n = lane & 31, gb = lane >> 5, t = n >> 2;
   const int dlo = t * 2 + (n & 1);
-  f32x16_t acc[1][1];
+  typename octet_acc<WIDE>::vec acc[1][1];
 #pragma unroll
-  for (int e = 0; e < 16; e++) acc[0][0][e] = 0.0f;
+  for (int e = 0; e < 16; e++) acc[0][0][e] = 0;
   load_bq32_lds<1, 0, 0>(r.b[0], bl, dl, lane, dlo, 0);
   if (split)
     olfixed_from<0, NQ, 1, 1, NG, 0, 0, 0>(r, ws, ao, bl, dl, lane, dlo, lane_upper32(lane), lane_bscale32(lane), acc);
@@ -950,7 +980,7 @@ void k_down_ol(const uint8_t *__restrict__ w_d, const uint32_t *__restrict__ hs,
   float v[16];
 #pragma unroll
   for (int e = 0; e < 16; e++) {
-    v[e] = col4_sum(acc[0][0][e]);
+    v[e] = (float)col4_sum(acc[0][0][e]);
     if (!shared) v[e] = __fmul_rn(v[e], wt);
   }
   if ((n & 3) == 0 && live) {

@@ -56,7 +56,6 @@
 #include "grouped_plan.h"
 #include "kernels_grouped.h"
 
-typedef double f64x16_t __attribute__((ext_vector_type(16)));
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));

@@ -882,7 +882,7 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
     return fail(c, MOE_ERR_UNSUPPORTED, "grouped: more than %d pairs or %d experts", MOE_GROUP_MAX_PAIRS,
                 MOE_GROUP_MAX_E);
   const grouped_plan plan = plan_grouped(T, k, E, H, F, shared != 0);
-  const bool oct = plan.octets, sk = plan.stacked, in_order = plan.in_order;
+  const bool oct = plan.octets, sk = plan.stacked, in_order = plan.in_order, wide = plan.octet_f64;
   const int BT = plan.item_rows;
   // a few tokens (the pairs path): down per 16-row tile of H with the slot
   // combine in the same launch (k_down_few)
@@ -909,7 +909,9 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
       hipLaunchKernelGGL(in_order ? k_gate_up_sk<false> : k_gate_up_sk<true>, dim3(F / 128, cap),
                          dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st, L.m[T_GATE].w, L.m[T_UP].w, s.xq, items, perm, k,
                          T, F, H, d.clamp, s.hq, htap);
-    else if (oct) hipLaunchKernelGGL(k_gate_up_o, dim3(F / (2 * MOE_UNIT), cap), dim3(256), 0, st, MOE_GU_ARGS);
+    else if (oct)
+      hipLaunchKernelGGL(wide ? k_gate_up_o<true> : k_gate_up_o<false>, dim3(F / (2 * MOE_UNIT), cap), dim3(256), 0, st,
+                         MOE_GU_ARGS);
     else hipLaunchKernelGGL(k_gate_up_g<2>, dim3(F / MOE_UNIT, cap), dim3(256), 0, st, MOE_GU_ARGS);
 #undef MOE_GU_ARGS
   }
@@ -920,20 +922,23 @@ static moe_status forward_grouped(moe_ctx *c, dev_layer &L, work_bufs &s, const 
 #define MOE_DN_ARGS L.m[T_DOWN].w, s.hq, s.hd, P + T, items, perm, wts, F, H, s.y
     const dim3 gdo(H / 128, cap);
     const size_t lo = octet_lds_bytes(F / MOE_QK);
+#define MOE_DOWN_OL(NQ) \
+  hipLaunchKernelGGL((wide ? k_down_ol<NQ, true> : k_down_ol<NQ, false>), gdo, dim3(256), lo, st, MOE_DN_ARGS)
     if (sk)
       hipLaunchKernelGGL(in_order ? k_down_sk<false> : k_down_sk<true>,
                          dim3(ceil_div(H, 64 * MOE_SK_WAVES), cap), dim3(64 * MOE_SK_WAVES), MOE_SK_LDS_BYTES, st,
                          L.m[T_DOWN].w, s.hq, P + T, items, perm, wts, F, H, s.y);
-    else if (oct && F == 128 * 16) hipLaunchKernelGGL(k_down_ol<16>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
-    else if (oct && F == 128 * 6) hipLaunchKernelGGL(k_down_ol<6>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
-    else if (oct && F == 128 * 8) hipLaunchKernelGGL(k_down_ol<8>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
-    else if (oct && F == 128 * 28) hipLaunchKernelGGL(k_down_ol<28>, gdo, dim3(256), lo, st, MOE_DN_ARGS);
-    else if (oct) hipLaunchKernelGGL(k_down_o, gdo, dim3(256), 0, st, MOE_DN_ARGS);
+    else if (oct && F == 128 * 16) MOE_DOWN_OL(16);
+    else if (oct && F == 128 * 6) MOE_DOWN_OL(6);
+    else if (oct && F == 128 * 8) MOE_DOWN_OL(8);
+    else if (oct && F == 128 * 28) MOE_DOWN_OL(28);
+    else if (oct) hipLaunchKernelGGL(wide ? k_down_o<true> : k_down_o<false>, gdo, dim3(256), 0, st, MOE_DN_ARGS);
     else if (few)
       hipLaunchKernelGGL(k_down_few<2>, dim3(H / MOE_DF_ROWS), dim3(64 * MOE_DF_WAVES), 0, st, L.m[T_DOWN].w, s.hq,
                          s.hd, P + T, items, perm, wts, T, k, F, H, shared, per_slot ? 1 : 0, out);
     else hipLaunchKernelGGL(k_down_g<2>, dim3(ceil_div(H / (2 * MOE_TILE), MOE_DG_WAVES), cap),
                             dim3(64 * MOE_DG_WAVES), 0, st, MOE_DN_ARGS);
+#undef MOE_DOWN_OL
 #undef MOE_DN_ARGS
   }
   if (few) {  // k_down_few wrote out

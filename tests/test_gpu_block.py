@@ -513,12 +513,12 @@ SWEEP = [
     (4096, 1024, 64, 6, 32, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 3 rows per expert
     (2048, 1536, 16, 2, 20, False, 6.0, wl.ROUTE_SOFTMAX),    # octets, k_down_o, 2-3 rows
     (1024, 1024, 256, 8, 7, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_gate_up_o, k_down_ol<8>
-    (7168, 768, 16, 4, 9, False, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets, k_down_ol<6>
-    (2048, 3584, 8, 2, 33, True, 8.0, wl.ROUTE_SIGMOID),      # octets, k_down_ol<28>, clamp
+    (7168, 768, 16, 4, 9, False, 0.0, wl.ROUTE_SQRT_SOFTPLUS),  # octets in f64, k_down_ol<6>
+    (2048, 3584, 8, 2, 33, True, 8.0, wl.ROUTE_SIGMOID),      # octets in f64, k_down_ol<28>, clamp
     (5120, 2048, 32, 6, 1, True, 0.0, wl.ROUTE_SIGMOID),      # decode, H = 5120
     (6144, 1024, 16, 4, 1, False, 3.0, wl.ROUTE_SOFTMAX),     # decode, H = 6144, clamp
     (4096, 1024, 16, 4, 64, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 16 rows per expert, shared rows
-    (7168, 768, 8, 4, 40, False, 5.0, wl.ROUTE_SOFTMAX),      # octets, k_down_ol<6>, several per expert, clamp
+    (7168, 768, 8, 4, 40, False, 5.0, wl.ROUTE_SOFTMAX),      # octets in f64, several per expert, clamp
     (2048, 2048, 16, 4, 24, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, 6 rows per expert
     (2048, 1024, 8, 4, 80, False, 3.0, wl.ROUTE_SOFTMAX),     # stacked, experts of 32 + n rows, clamp
     (4096, 1280, 16, 4, 32, True, 0.0, wl.ROUTE_SIGMOID),     # stacked, sums in f64, 8 rows per expert
@@ -527,6 +527,8 @@ SWEEP = [
     (7168, 1536, 16, 8, 8, True, 0.0, wl.ROUTE_SIGMOID),      # stacked, 4 rows per expert
     (6144, 2048, 16, 8, 40, False, 0.0, wl.ROUTE_SIGMOID),    # stacked (glm-dsa H), 20 rows
     (2048, 2048, 16, 4, 10, True, 0.0, wl.ROUTE_SIGMOID),     # octets, k_down_ol<16>
+    (2048, 3584, 32, 2, 9, True, 8.0, wl.ROUTE_SIGMOID),      # octets below 2 rows per expert, k_down_ol<28>, clamp
+    (1024, 768, 32, 4, 9, False, 0.0, wl.ROUTE_SOFTMAX),      # the same, k_down_ol<6>
 ]
 
 
@@ -857,3 +859,34 @@ def test_stacked_item_edges(blk, torch_dev, oracle, H, F, E, first, rest, per_sl
         check_block(oracle, L, blk, shape, x, ids, wts, got, f"stacked {H}x{F} {first}", per_slot=per_slot)
     finally:
         blk.release_layer(60)
+
+
+# H, F, experts, tokens of a stacked call and of an octet call, top-1: K of 9 and 5
+# quads in gate/up; down on k_down_ol<6, 8, 16, 28> and k_down_o
+F64_LAYERS = [(1152, 768, 16, 420, 40), (1152, 1024, 16, 420, 33), (1152, 2048, 16, 420, 64), (1152, 3584, 16, 420, 47),
+              (640, 384, 16, 800, 35)]
+
+
+@pytest.mark.parametrize("H,F,E,T,few", F64_LAYERS)
+def test_octets_in_f64_equal_the_stacked_rows(blk, torch_dev, oracle, H, F, E, T, few):
+    """The first tokens of a call that runs stacked with sums in f64, called
+    alone on octets with sums in f64: the same rows.  Both sums are exact to
+    about 1e-15 and rounded to f32 once, so a row could differ only where a sum
+    lies that close to a rounding boundary (1 value in 10^7 or so; these inputs
+    are fixed and have none)."""
+    shape = wl.LayerShape(hidden=H, ffn=F, n_expert=E, n_used=1, has_shared=False, route_mode=1, clamp=6.0)
+    rng = np.random.default_rng(F)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    ids = rng.integers(0, E, (T, 1)).astype(np.int32)
+    wts = rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)
+    say("f64 octets", H, F, E, T, few)
+    blk.generate_layer(62, shape, seed=F, e_lo=116, e_span=5)
+    try:
+        all_rows = run_block(blk, torch_dev, 62, x, ids, wts)
+        h_all = blk.debug_last_h(T * F).reshape(T, F)[oracle.group(ids, E)["inv"]]
+        got = run_block(blk, torch_dev, 62, x[:few], ids[:few], wts[:few])
+        h_few = blk.debug_last_h(few * F).reshape(few, F)[oracle.group(ids[:few], E)["inv"]]
+        np.testing.assert_array_equal(h_few, h_all[:few])
+        np.testing.assert_array_equal(got, all_rows[:few])
+    finally:
+        blk.release_layer(62)

@@ -14,7 +14,7 @@ int main() {
   int T, k, E, H, F, s;
   while (scanf("%d %d %d %d %d %d", &T, &k, &E, &H, &F, &s) == 6) {
     const grouped_plan p = plan_grouped(T, k, E, H, F, s != 0);
-    printf("%s %d\\n", !p.octets ? "pairs" : !p.stacked ? "octets" : p.in_order ? "stacked_f32" : "stacked_f64", p.item_rows);
+    printf("%s %d\\n", !p.octets ? "pairs" : !p.stacked ? (p.octet_f64 ? "octets_f64" : "octets") : p.in_order ? "stacked_f32" : "stacked_f64", p.item_rows);
   }
 }
 """
@@ -68,7 +68,8 @@ FASTER_STACKED = [
 
 
 def test_small_calls_run_on_octets(plan):
-    assert plan(SLOWER_STACKED) == [("octets", 8)] * len(SLOWER_STACKED)
+    f32 = [(7168, 2048), (2048, 1024)]
+    assert plan(SLOWER_STACKED) == [("octets" if c[3:5] in f32 else "octets_f64", 8) for c in SLOWER_STACKED]
 
 
 def test_full_calls_run_stacked(plan):
@@ -102,12 +103,12 @@ def test_plan_limits(plan):
     for (T, k, E, H, F, _), (kind, rows) in zip(calls, plan(calls)):
         assert (kind == "pairs") == (T <= 4)
         if T * k < 2 * E:
-            assert not kind.startswith("stacked")
+            assert kind in ("pairs", "octets")
         if kind == "stacked_f32":
             assert H % 512 == 0 and F % 512 == 0
-        assert rows in {"pairs": (4,), "octets": (8,), "stacked_f64": (32,), "stacked_f32": (32, 64)}[kind]
+        assert rows in {"pairs": (4,), "octets": (8,), "octets_f64": (8,), "stacked_f64": (32,), "stacked_f32": (32, 64)}[kind]
         seen.add((kind, rows))
-    assert len(seen) == 5
+    assert len(seen) == 6
 
 
 def test_gpu_tests_reach_the_kernels_they_name(plan):
@@ -120,10 +121,13 @@ def test_gpu_tests_reach_the_kernels_they_name(plan):
     # the layers of test_out_of_range_ids_contribute_nothing
     dropped = plan([(12, 4, 32, 2048, 768, False), (16, 8, 256, 7168, 2048, True), (64, 8, 256, 7168, 2048, True),
                     (160, 4, 16, 1152, 512, True), (160, 4, 16, 1152, 512, False), (192, 4, 128, 2048, 1024, True)])
-    assert dropped == [("octets", 8), ("octets", 8), ("stacked_f32", 32), ("stacked_f64", 32), ("stacked_f64", 32),
+    assert dropped[:2] == [("octets", 8), ("octets", 8)]
+    assert dropped[2:] == [("stacked_f32", 32), ("stacked_f64", 32), ("stacked_f64", 32),
                        ("stacked_f32", 64)]
+    for H, F, E, T, few in gpu.F64_LAYERS:
+        assert plan([(T, 1, E, H, F, False), (few, 1, E, H, F, False)]) == [("stacked_f64", 32), ("octets_f64", 8)]
     sweep = [c for c in gpu.SWEEP if c[4] > 1]
     kinds = [k for k, _ in plan([(T, k, E, H, F, sh) for H, F, E, k, T, sh, _, _ in sweep])]
-    assert {"pairs", "octets", "stacked_f32"} <= set(kinds)
+    assert {"pairs", "octets", "octets_f64", "stacked_f32", "stacked_f64"} <= set(kinds)
     octets = {c[1] // 128 for c, k in zip(sweep, kinds) if k == "octets"}  # F / 128: the down kernel's instance
     assert {6, 8, 16, 28} <= octets and octets - {6, 8, 16, 28}  # k_down_ol<6, 8, 16, 28> and k_down_o
