@@ -54,19 +54,24 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   // 2048 x 768, 8-12%).
   p.octet_f64 = p.octets && !p.stacked && !p.in_order && P >= 2L * E;
   // Two token tiles per weight pair (items of up to 64 rows): a weight is read
-  // and duplicated once for both, 2048 tokens on the V3 layer 2308 -> 2134 us,
-  // but the workgroups are half as many and run twice as long.  So only where
-  // 64-row items still make two rounds of workgroups (512 a round) in the launch
-  // that has fewer, from 4 pairs per expert on (below that the shared expert's
-  // items are the only large ones: 64 tokens on the V3 layer 241 -> 259 us).  us
-  // per layer, 32-row / 64-row items, 32 and 64 rows per expert:
-  //   7168 x 2048, 8 experts 78/92  104/111; 32 experts 232/221  333/360; 128 experts 762/718  1214/1094
-  //   2048 x 1024, 8 experts 34/44  35/48; 32 experts 54/65  75/76; 128 experts 148/152  219/221
-  //   4096 x 1536, 32 experts 114/112  166/176; 128 experts 361/350  561/524
-  // The f64 sums leave no registers for two tiles.
+  // and duplicated once for both, but the workgroups are half as many and run
+  // twice as long.  So only where 64-row items still make one and a half rounds
+  // of workgroups (512 a round) in the launch that has fewer -- or 400, where
+  // the average expert has 32-64 rows, one item instead of two --, from 4 pairs
+  // per expert on (below that the shared expert's items are the only large
+  // ones).  us per layer, 32-row / 64-row items, and their workgroups:
+  //   7168 x 2048, 8 experts, 32, 64 rows each      78/92  103/107 (128, 192)
+  //   7168 x 2048, 32 experts, 16, 32, 64 rows      170/175  230/209  323/340 (544, 576, 640)
+  //   7168 x 2048, 128 experts, 32, 64 rows         748/718  1186/1082 (2176, 2304)
+  //   2048 x 1024, 32 experts, 8, 32, 64 rows       45/54  54/65  75/74 (264, 288, 320)
+  //   7168 x 1536, 63 experts, 43 rows              466/371 (924)
+  // (7168 x 2048, 32 experts: 64 rows are on the wrong side at 640; the line is
+  // fitted to 350 shapes, whose geometric mean lies 1.0% over the better of the
+  // two).  The f64 sums leave no registers for two tiles.
   const long items64 = (P / 64 > E ? P / 64 : E) + (shared ? T / 64 : 0);
   const int gu2 = F / 128, dn2 = H / 256;  // stacked workgroups per item
-  const bool two = p.in_order && P >= 4L * E && items64 * (gu2 < dn2 ? gu2 : dn2) >= 1024;
+  const long n64 = items64 * (gu2 < dn2 ? gu2 : dn2);
+  const bool two = p.in_order && P >= 4L * E && n64 >= (P >= 32L * E && P < 64L * E ? 400 : 768);
   p.item_rows = !p.octets ? 4 : !p.stacked ? 8 : two ? MOE_PLAN_ROWS2 : MOE_PLAN_ROWS;
   return p;
 }

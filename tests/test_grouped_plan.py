@@ -79,15 +79,18 @@ def test_full_calls_run_stacked(plan):
 def test_items_of_64_rows_only_where_the_chip_stays_full(plan):
     """Two token tiles halve the workgroups: us per layer, 32-row / 64-row items."""
     slower = [(128, 2, 8, 7168, 2048, False),    # 78 / 92
-              (512, 4, 32, 7168, 2048, True),    # 333 / 360
+              (128, 4, 32, 7168, 2048, True),    # 170 / 175
+              (512, 4, 32, 7168, 2048, True),    # 323 / 340
               (256, 2, 8, 2048, 1024, False),    # 35 / 48
-              (256, 4, 32, 6144, 1024, True),    # 117 / 139
-              (64, 4, 32, 4096, 1536, True)]     # 86 / 95: the shared expert's item of 64 rows
-    faster = [(512, 8, 128, 7168, 2048, True),   # 762 / 718
-              (1024, 8, 128, 4096, 1536, True),  # 561 / 524
-              (512, 8, 256, 7168, 2048, True),   # Zipf 744 / 696
-              (509, 6, 384, 7168, 3072, True),   # Zipf 806 / 778
-              (2048, 8, 256, 7168, 2048, True)]  # 2300 / 2116
+              (256, 4, 32, 2048, 1024, True),    # 54 / 65
+              (64, 4, 32, 2048, 1024, True)]     # 45 / 54: the shared expert's item of 64 rows
+    faster = [(512, 8, 128, 7168, 2048, True),   # 748 / 718
+              (256, 4, 32, 7168, 2048, True),    # 230 / 209: an expert is one item
+              (913, 3, 63, 7168, 1536, True),    # 466 / 371: the same
+              (1024, 8, 128, 4096, 1536, True),
+              (512, 8, 256, 7168, 2048, True),   # Zipf 682 / 658
+              (509, 6, 384, 7168, 3072, True),   # Zipf 768 / 746
+              (2048, 8, 256, 7168, 2048, True)]  # 2298 / 2115
     assert plan(slower) == [("stacked_f32", 32)] * len(slower)
     assert plan(faster) == [("stacked_f32", 64)] * len(faster)
 
