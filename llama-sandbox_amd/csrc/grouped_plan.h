@@ -28,9 +28,10 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   // which came from the octet kernels.  Those err less than f32 in order (their
   // separate digit planes round less often), so f32 would lose precision there:
   // rms of output rows from 64 bits, f32 / octets / f64, 0.9-1.3e-7 / 4.1-5.8e-8
-  // / 3.6e-8.  And f64 everywhere costs the first shapes more than the stacked
-  // kernels gained them: V3 layer, 64 and 512 tokens Zipf, 512 and 2048 uniform
-  // 227 -> 301, 680 -> 948, 1136 -> 1342, 2148 -> 3144 us.
+  // / 3.6e-8.  And f64 everywhere costs the first shapes more than these kernels
+  // gained them over their e4m3 form: V3 layer, 64 and 512 tokens Zipf, 512 and
+  // 2048 uniform, e4m3 / f32 / f64: 241/227/253, 835/689/907, 1214/1143/1308,
+  // 2868/2196/3174 us.
   p.in_order = (H == 128 * 56 || H == 128 * 48 || H == 128 * 32 || H == 128 * 16) &&
                (F == 128 * 8 || F == 128 * 12 || F == 128 * 16 || F == 128 * 24);
   // A stacked workgroup reads an expert's weights once for up to 32 rows, but

@@ -12,9 +12,11 @@
 //
 // Bound by latency: a token's scores stay in its wave's registers (lane l holds
 // experts l, l + 64, ...), and a round of the top-k is one wave maximum over
-// DPP and one ballot, with no LDS and no barrier.  Between events: 256 experts,
-// top-8, T = 512 19.3 -> 8.5 us; 32 experts, top-4, T = 1 7.9 -> 5.8 us (against
-// a 256-thread workgroup per token, scores in LDS, shuffles in every round).
+// DPP and one ballot, with no LDS and no barrier.  Kernel trace, median of 200
+// in a row: 256 experts, top-8, T = 512 13.9 -> 5.8 us, T = 1 12.3 -> 4.5; 32
+// experts, top-4, T = 1 6.0 -> 2.3; 1024 experts, T = 512 25.3 -> 13.3 (against a
+// 256-thread workgroup per token, scores in LDS, shuffles in every round).  The
+// first launch of a process takes about 20 us.
 #define MOE_ROUTE_MAX_E 1024
 
 // Score of one logit for the element-wise score functions (mode 1: sigmoid,

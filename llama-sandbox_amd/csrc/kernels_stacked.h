@@ -12,9 +12,8 @@
 //
 // The digits (hi in [-8, 7], lo in [0, 15]) are e2m3 codes (fp6: digit / 8,
 // the code of a magnitude is the magnitude itself, the sign bit 32), not e4m3:
-// with fp6 an MFMA takes 45-54 cycles instead of 77 (random operands, the
-// clock that the chip holds under them), and a token's block 48 bytes instead
-// of 64.
+// with fp6 an MFMA keeps the matrix core busy for 32 cycles instead of 64
+// (counters), and a token's block takes 48 bytes instead of 64.
 //
 // Staged activations ("quad records"): per row and quad of 4 blocks 208 bytes
 //   [0, 96)    hi digits of blocks 0..3, 24 bytes each (6 bits per K offset)
@@ -24,23 +23,23 @@
 // quad (an item's rows of a quad are one run).  The direct global-to-LDS loads
 // of a chunk (1 KiB each) read such runs in order, about 10 cache lines per
 // load; with one 16-byte piece per (token, block) and load, 64 lines, the load
-// path bounds the kernel
-// (a build that staged 96 bytes per block that way: gate/up of 2048 tokens on
-// the V3 layer 2003 us, 1353 us with the same bytes contiguous).
+// path bounds the kernel (a build that staged 96 bytes per block that way:
+// gate/up of 2048 tokens on the V3 layer 2003 us, 1353 us with the same bytes
+// contiguous).
 //
 // Items of up to 16 rows, of which small batches and the remainders of long
 // chunks are made, run the MFMA with its operands swapped (skf_loop): tokens on
 // D's elements, and only the elements of tokens that the item holds are scaled.
 // Items of 33-64 rows share each weight pair between two token tiles (sk_loop2).
 //
-// What bounds them (V3 layer): at 512 tokens, uniform, the weight stream
-// (gate/up 740 us, 712 us with the staging and the scaling left out; the bare
-// stream of the same bytes 560 us); at 2048 tokens the vector issue, 26
-// instructions per MFMA in 88% of the cycles at the 1.5 GHz that the chip
-// holds.  Measured on one box against the e4m3 digits staged in pieces:
-// prefill 512 uniform 1200 -> 1153 us, Zipf 808 -> 732 us, 2048 tokens 2761 ->
-// 2368 us, the V4-Pro layer 927 -> 833 us; 300 tokens on a 5120 x 1536 layer,
-// where the octet kernels ran, 571 -> 458 us (sums in f64, sk_scale).
+// What bounds them (V3 layer, profiles/prefill_stacked_counters.md): at 512
+// tokens, uniform, the weight stream (vector issue 43% of the cycles, matrix
+// cores 17%; the bare stream of gate/up's bytes takes 560 us); at 2048 tokens
+// the vector issue, 19 instructions per MFMA in 66% of the cycles at the 1.7 GHz
+// that the chip holds.  Timed on one box against the kernels before them (e4m3
+// digits staged in pieces): 512 tokens uniform 1171 -> 1101 us, Zipf 829 -> 686,
+// 2048 tokens 2831 -> 2140, the V4-Pro layer 933 -> 764; 300 tokens on a 5120 x
+// 1536 layer, octets before, 553 -> 421 (sums in f64, sk_scale).
 //
 // Operand lanes.  A lane r + 32*g holds weight row r, K [32g, 32g + 32): the
 // record layout gives lane (r, g) block 2j + g of a quad in one load, and
@@ -488,9 +487,9 @@ __device__ __forceinline__ void sk_loop(const skw &w, const uint32_t *src, int n
 // ---------------------------------------------------------------------------
 // The same for items of 33-64 rows: two token tiles share each weight pair, so
 // the weights of a large expert are read (mostly from L2) and duplicated
-// across the lane halves half as often: 21 vector instructions per MFMA
-// instead of 26.  A chunk is 2 quads of 64 rows.  V3 layer: 512 tokens Zipf
-// 744 -> 696 us, 2048 tokens 2300 -> 2116 us; V4-Pro layer 806 -> 778 us.
+// across the lane halves half as often.  A chunk is 2 quads of 64 rows.  V3
+// layer: 512 tokens Zipf 682 -> 658 us, 2048 tokens 2298 -> 2115 us; V4-Pro
+// layer 768 -> 746 us.
 struct skring2 {
   u32x4_t w[MOE_SK_RP][2];
   uint32_t e[2][4];
