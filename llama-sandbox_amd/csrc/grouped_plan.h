@@ -3,8 +3,7 @@
 //
 // Token pairs (16x16x128 MFMA, items of up to 4 rows) for T <= 4, token octets
 // (32x32x64 MFMA, items of up to 8 rows) above that, and the stacked kernels
-// (items of up to 32 or 64 rows) where an expert's rows fill several octets or
-// the chip has octets to spare.
+// (items of up to 32 or 64 rows) for calls that fill the chip.
 #pragma once
 
 #define MOE_PLAN_PAIR_TOKENS 4
@@ -15,7 +14,7 @@ struct grouped_plan {
   bool octets;    // T > 4
   bool stacked;   // octets, but on the stacked kernels
   bool in_order;  // stacked: sums block by block in f32 (else in f64)
-  bool octet_f64; // octets with sums in f64 (else in f32)
+  bool octet_f64;  // octets with sums in f64 (else in f32)
   int item_rows;
 };
 
@@ -66,9 +65,8 @@ static inline grouped_plan plan_grouped(int T, int k, int E, int H, int F, bool 
   //   7168 x 2048, 128 experts, 32, 64 rows         748/718  1186/1082 (2176, 2304)
   //   2048 x 1024, 32 experts, 8, 32, 64 rows       45/54  54/65  75/74 (264, 288, 320)
   //   7168 x 1536, 63 experts, 43 rows              466/371 (924)
-  // (7168 x 2048, 32 experts: 64 rows are on the wrong side at 640; the line is
-  // fitted to 350 shapes, whose geometric mean lies 1.0% over the better of the
-  // two).  The f64 sums leave no registers for two tiles.
+  // (fitted to 350 random shapes: in the mean 1.0% over the better of the two).
+  // The f64 sums leave no registers for two tiles.
   const long items64 = (P / 64 > E ? P / 64 : E) + (shared ? T / 64 : 0);
   const int gu2 = F / 128, dn2 = H / 256;  // stacked workgroups per item
   const long n64 = items64 * (gu2 < dn2 ? gu2 : dn2);
